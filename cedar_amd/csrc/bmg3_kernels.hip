@@ -14,6 +14,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 namespace cdr {
 namespace k3 {
 
@@ -753,19 +755,19 @@ __global__ __launch_bounds__(256) void oi_cube_k(const double *__restrict__ so, 
 // BMG3_SymStd_SETUP_ITLI27_ex.f90).  P is the prolongation applied by interp_add: fine offset
 // d from coarse point C has weight CI(C + max(d, 0), plane(d)), weight 1 at d = 0.  A is the fine
 // operator, A(f, f + o) = -so(f + s(o), plane(o)) with (s, plane) from the neighbour list.
-// Fine points outside the interior carry no unknown and are skipped.  One thread per coarse
-// point computes its 14 entries; loop order fixes the rounding.
+// Fine points outside the interior carry no unknown and are skipped; loop order fixes the
+// rounding.
 // ------------------------------------------------------------------------------------------
 // tables indexed by (dz+1)*9 + (dy+1)*3 + (dx+1)
-__constant__ int PW3_PLANE[27] = {
+__constant__ constexpr int PW3_PLANE[27] = {
     ltne, lyznw, ltnw, lxzne, lxza, lxznw, ltse, lyzne, ltsw,
     lxyne, lxya, lxynw, lxyr, 0, lxyl, lxyse, lxyb, lxysw,
     lbne, lyzsw, lbnw, lxzse, lxzb, lxzsw, lbse, lyzse, lbsw};
 // stored position s and plane of A(f, f + o)
-__constant__ signed char A_SI[27] = {0, 0, 1, 0, 0, 1, 0, 0, 1,  0, 0, 1, 0, 0, 1, 0, 0, 1,  0, 0, 1, 0, 0, 1, 0, 0, 1};
-__constant__ signed char A_SJ[27] = {0, 0, 0, 0, 0, 0, 1, 1, 1,  0, 0, 0, 0, 0, 0, 1, 1, 1,  0, 0, 0, 0, 0, 0, 1, 1, 1};
-__constant__ signed char A_SK[27] = {0, 0, 0, 0, 0, 0, 0, 0, 0,  0, 0, 0, 0, 0, 0, 0, 0, 0,  1, 1, 1, 1, 1, 1, 1, 1, 1};
-__constant__ signed char A_PL[27] = {
+__constant__ constexpr signed char A_SI[27] = {0, 0, 1, 0, 0, 1, 0, 0, 1,  0, 0, 1, 0, 0, 1, 0, 0, 1,  0, 0, 1, 0, 0, 1, 0, 0, 1};
+__constant__ constexpr signed char A_SJ[27] = {0, 0, 0, 0, 0, 0, 1, 1, 1,  0, 0, 0, 0, 0, 0, 1, 1, 1,  0, 0, 0, 0, 0, 0, 1, 1, 1};
+__constant__ constexpr signed char A_SK[27] = {0, 0, 0, 0, 0, 0, 0, 0, 0,  0, 0, 0, 0, 0, 0, 0, 0, 0,  1, 1, 1, 1, 1, 1, 1, 1, 1};
+__constant__ constexpr signed char A_PL[27] = {
     kbsw, kbs, kbse, kbw, kb, kbe, kbnw, kbn, kbne,
     kpsw, kps, kpnw, kpw, kp, kpw, kpnw, kps, kpsw,
     kbne, kbn, kbnw, kbe, kb, kbw, kbse, kbs, kbsw};
@@ -785,53 +787,90 @@ __device__ inline double aentry3(const double *__restrict__ so, std::size_t P, i
     return -S3(i + A_SI[t], j + A_SJ[t], k + A_SK[t], A_PL[t]);
 }
 
-template <bool NINE>
-__device__ double kpair3(const double *__restrict__ so, const double *__restrict__ ci, int iif, int jjf,
-                         int kkf, int iic, int jjc, int kkc, int icx, int jcx, int kcx, int DX, int DY,
-                         int DZ) {
-    const int ii = iif, jj = jjf;
-    const std::size_t P = (std::size_t)iif * jjf * kkf, Pc = (std::size_t)iic * jjc * kkc;
-    const int X0 = 2 * (icx - 1), Y0 = 2 * (jcx - 1), Z0 = 2 * (kcx - 1);
-    double sum = 0.0;
-#pragma unroll 1
-    for (int fz = -1; fz <= 1; ++fz)
-#pragma unroll 1
-        for (int fy = -1; fy <= 1; ++fy)
-#pragma unroll 1
-            for (int fx = -1; fx <= 1; ++fx) {
-                const int x = X0 + fx, y = Y0 + fy, z = Z0 + fz;
-                if (x < 2 || x > iif - 1 || y < 2 || y > jjf - 1 || z < 2 || z > kkf - 1) continue;
-                double inner = 0.0;
-                bool any = false;
-#pragma unroll 1
-                for (int oz = -1; oz <= 1; ++oz)
-#pragma unroll 1
-                    for (int oy = -1; oy <= 1; ++oy)
-#pragma unroll 1
-                        for (int ox = -1; ox <= 1; ++ox) {
-                            const int gx = fx + ox - 2 * DX, gy = fy + oy - 2 * DY, gz = fz + oz - 2 * DZ;
-                            if (gx < -1 || gx > 1 || gy < -1 || gy > 1 || gz < -1 || gz > 1) continue;
-                            const int xg = x + ox, yg = y + oy, zg = z + oz;
-                            if (xg < 2 || xg > iif - 1 || yg < 2 || yg > jjf - 1 || zg < 2 || zg > kkf - 1)
-                                continue;
-                            if (!NINE && (ox != 0) + (oy != 0) + (oz != 0) > 1) continue;
-                            inner += aentry3<NINE>(so, P, ii, jj, x, y, z, ox, oy, oz) *
-                                     pweight3(ci, Pc, iic, jjc, icx + DX, jcx + DY, kcx + DZ, gx, gy, gz);
-                            any = true;
-                        }
-                if (any) sum += pweight3(ci, Pc, iic, jjc, icx, jcx, kcx, fx, fy, fz) * inner;
-            }
-    return sum;
-}
-
 // coarse plane d at g couples g + a with g + b
-__constant__ signed char CP_D[13] = {kpw, kps, kb, kpsw, kpnw, kbw, kbnw, kbn, kbne, kbe, kbse, kbs, kbsw};
-__constant__ signed char CP_A[13][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, -1, 0}, {0, 0, 0}, {0, -1, 0},
+__constant__ constexpr signed char CP_D[13] = {kpw, kps, kb, kpsw, kpnw, kbw, kbnw, kbn, kbne, kbe, kbse, kbs, kbsw};
+__constant__ constexpr signed char CP_A[13][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, -1, 0}, {0, 0, 0}, {0, -1, 0},
                                         {0, -1, 0}, {-1, -1, 0}, {-1, 0, 0}, {-1, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-__constant__ signed char CP_B[13][3] = {{-1, 0, 0}, {0, -1, 0}, {0, 0, -1}, {-1, -1, 0}, {-1, 0, 0}, {-1, 0, -1},
+__constant__ constexpr signed char CP_B[13][3] = {{-1, 0, 0}, {0, -1, 0}, {0, 0, -1}, {-1, -1, 0}, {-1, 0, 0}, {-1, 0, -1},
                                         {-1, 0, -1}, {0, 0, -1}, {0, 0, -1}, {0, 0, -1}, {0, -1, -1}, {0, -1, -1},
                                         {-1, -1, -1}};
 
+// The 14 entries of one row of P^T A P at once: couplings of the coarse point C to C + D, with D
+// = b - a of the 13 stored planes and D = 0 (index 13).  Every sum runs over the fine points f =
+// C - 1 .. C + 1 and, inside, over the neighbours f + o that interpolate from C + D, both in
+// increasing (z, y, x) order, as one pass over f and o in which each entry A(f, f + o) is read
+// once and feeds every D it reaches; which terms exist is known at compile time (about 1300 for
+// 27 points).
+template <int T>
+struct row_dir {
+    static constexpr int x = T < 13 ? CP_B[T % 13][0] - CP_A[T % 13][0] : 0;
+    static constexpr int y = T < 13 ? CP_B[T % 13][1] - CP_A[T % 13][1] : 0;
+    static constexpr int z = T < 13 ? CP_B[T % 13][2] - CP_A[T % 13][2] : 0;
+};
+
+struct row_ctx {
+    const double *__restrict__ so, *__restrict__ ci;
+    std::size_t P, Pc;
+    // element offsets of the fine positions -1 .. 2 and of the coarse positions -1 .. 1 around C,
+    // kept inside the arrays; whether the fine positions -2 .. 2 lie in the interior
+    unsigned xf[4], yf[4], zf[4], xc[3], yc[3], zc[3];
+    bool vx[5], vy[5], vz[5];
+};
+
+template <int DX, int DY, int DZ, int GX, int GY, int GZ>
+__device__ inline double row_weight(const row_ctx &c) {
+    constexpr int g = (GZ + 1) * 9 + (GY + 1) * 3 + (GX + 1);
+    if constexpr (g == 13) {
+        return 1.0;
+    } else {
+        return c.ci[(std::size_t)(PW3_PLANE[g] - 1) * c.Pc +
+                    (c.zc[DZ + (GZ > 0) + 1] + c.yc[DY + (GY > 0) + 1] + c.xc[DX + (GX > 0) + 1])];
+    }
+}
+
+template <bool NINE, int F, int O, int... T>
+__device__ inline void row_neighbour(const row_ctx &c, double (&inner)[14],
+                                     std::integer_sequence<int, T...>) {
+    constexpr int fx = F % 3 - 1, fy = F / 3 % 3 - 1, fz = F / 9 - 1;
+    constexpr int ox = O % 3 - 1, oy = O / 3 % 3 - 1, oz = O / 9 - 1;
+    if constexpr (NINE || (ox != 0) + (oy != 0) + (oz != 0) <= 1) {
+        const bool ok = c.vx[fx + ox + 2] && c.vy[fy + oy + 2] && c.vz[fz + oz + 2];
+        double a = c.so[(std::size_t)(A_PL[O] - 1) * c.P +
+                        (c.zf[fz + A_SK[O] + 1] + c.yf[fy + A_SJ[O] + 1] + c.xf[fx + A_SI[O] + 1])];
+        if constexpr (O != 13) a = -a;
+        (
+            [&] {
+                using D = row_dir<T>;
+                constexpr int gx = fx + ox - 2 * D::x, gy = fy + oy - 2 * D::y, gz = fz + oz - 2 * D::z;
+                if constexpr (gx >= -1 && gx <= 1 && gy >= -1 && gy <= 1 && gz >= -1 && gz <= 1) {
+                    const double t = a * row_weight<D::x, D::y, D::z, gx, gy, gz>(c);
+                    inner[T] += ok ? t : 0.0;  // a point outside carries no unknown
+                }
+            }(),
+            ...);
+    }
+}
+
+template <bool NINE, int F, int... O>
+__device__ inline void row_fine_point(const row_ctx &c, double (&sum)[14],
+                                      std::integer_sequence<int, O...>) {
+    constexpr int fx = F % 3 - 1, fy = F / 3 % 3 - 1, fz = F / 9 - 1;
+    if (!(c.vx[fx + 2] && c.vy[fy + 2] && c.vz[fz + 2])) return;
+    double inner[14] = {0.0};
+    (row_neighbour<NINE, F, O>(c, inner, std::make_integer_sequence<int, 14>{}), ...);
+    const double w = row_weight<0, 0, 0, fx, fy, fz>(c);
+#pragma unroll
+    for (int t = 0; t < 14; ++t) sum[t] += w * inner[t];  // a direction out of reach adds zero
+}
+
+template <bool NINE, int... F>
+__device__ inline void row_sums(const row_ctx &c, double (&sum)[14],
+                                std::integer_sequence<int, F...>) {
+    (row_fine_point<NINE, F>(c, sum, std::make_integer_sequence<int, 27>{}), ...);
+}
+
+// One thread per coarse point C: its row, each entry stored at the point g = C - a where the
+// plane keeps it (zero where g couples a point outside the grid).
 template <bool NINE>
 __global__ __launch_bounds__(256) void galerkin3_k(const double *__restrict__ so,
                                                    const double *__restrict__ ci,
@@ -841,16 +880,40 @@ __global__ __launch_bounds__(256) void galerkin3_k(const double *__restrict__ so
     const int jc = blockIdx.y * 4 + (threadIdx.x / 64) + 2;
     const int kc = blockIdx.z + 2;
     if (ic > iic - 1 || jc > jjc - 1) return;
-    const std::size_t Pc = (std::size_t)iic * jjc * kkc, pc = ix3(ic, jc, kc, iic, jjc);
-    soc[pc] = kpair3<NINE>(so, ci, iif, jjf, kkf, iic, jjc, kkc, ic, jc, kc, 0, 0, 0);
-#pragma unroll 1
+    row_ctx c{so, ci, (std::size_t)iif * jjf * kkf, (std::size_t)iic * jjc * kkc};
+    const int X0 = 2 * (ic - 1), Y0 = 2 * (jc - 1), Z0 = 2 * (kc - 1);
+#pragma unroll
+    for (int p = -1; p <= 2; ++p) {
+        c.xf[p + 1] = (unsigned)(min(X0 + p, iif) - 1);
+        c.yf[p + 1] = (unsigned)(min(Y0 + p, jjf) - 1) * (unsigned)iif;
+        c.zf[p + 1] = (unsigned)(min(Z0 + p, kkf) - 1) * (unsigned)(iif * jjf);
+    }
+#pragma unroll
+    for (int p = -1; p <= 1; ++p) {
+        c.xc[p + 1] = (unsigned)(ic + p - 1);
+        c.yc[p + 1] = (unsigned)(jc + p - 1) * (unsigned)iic;
+        c.zc[p + 1] = (unsigned)(kc + p - 1) * (unsigned)(iic * jjc);
+    }
+#pragma unroll
+    for (int p = -2; p <= 2; ++p) {
+        c.vx[p + 2] = X0 + p >= 2 && X0 + p <= iif - 1;
+        c.vy[p + 2] = Y0 + p >= 2 && Y0 + p <= jjf - 1;
+        c.vz[p + 2] = Z0 + p >= 2 && Z0 + p <= kkf - 1;
+    }
+    double sum[14] = {0.0};
+    row_sums<NINE>(c, sum, std::make_integer_sequence<int, 27>{});
+    const std::size_t Pc = c.Pc, pc = ix3(ic, jc, kc, iic, jjc);
+    soc[pc] = sum[13];
+#pragma unroll
     for (int t = 0; t < 13; ++t) {
-        const int xa = ic + CP_A[t][0], ya = jc + CP_A[t][1], za = kc + CP_A[t][2];
-        const int xb = ic + CP_B[t][0], yb = jc + CP_B[t][1], zb = kc + CP_B[t][2];
-        double v = 0.0;
-        if (xa >= 2 && ya >= 2 && za >= 2 && xb >= 2 && yb >= 2 && zb >= 2)
-            v = -kpair3<NINE>(so, ci, iif, jjf, kkf, iic, jjc, kkc, xa, ya, za, xb - xa, yb - ya, zb - za);
-        soc[(std::size_t)(CP_D[t] - 1) * Pc + pc] = v;
+        const int ax = CP_A[t][0], ay = CP_A[t][1], az = CP_A[t][2];
+        const int gx = ic - ax, gy = jc - ay, gz = kc - az;  // where the coupling is kept
+        double *d = soc + (std::size_t)(CP_D[t] - 1) * Pc;
+        if (gx <= iic - 1 && gy <= jjc - 1 && gz <= kkc - 1)
+            d[ix3(gx, gy, gz, iic, jjc)] =
+                (gx + CP_B[t][0] >= 2 && gy + CP_B[t][1] >= 2 && gz + CP_B[t][2] >= 2) ? -sum[t] : 0.0;
+        // no row reaches the points on the low side of a coupling whose a lies outside
+        if (ic + ax < 2 || jc + ay < 2 || kc + az < 2) d[pc] = 0.0;
     }
 }
 
@@ -1031,7 +1094,7 @@ __global__ __launch_bounds__(256) void ci_copy_k(double *__restrict__ ci, int ii
 // product are taken in the unwrapped geometry between X and Y, so each stored coupling is the
 // one across its own side, as the reference's hand-expanded products form it; only the array
 // reads wrap (coarse indices into 2..n+1, fine points into the interior).  Summation order as
-// in kpair3.
+// in galerkin3_k.
 __device__ inline int wrap_in(int n, int m) { return ((n - 2) % m + m) % m + 2; }
 
 template <bool NINE>
