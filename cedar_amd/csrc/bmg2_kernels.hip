@@ -16,6 +16,7 @@
 #include "../../include/cedar_hip.h"
 #include "band_chol.hpp"
 #include "bmg2_launch.hpp"
+#include "tile_order.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -81,36 +82,8 @@ __device__ inline void block_sum_store(double v, double *dst) {
 // Batched problems: every kernel below takes the problem index from the last grid dimension
 // (blockIdx.z for tiled kernels, blockIdx.y for line kernels, blockIdx.x for one-workgroup
 // kernels); the problems of a batch are stored back to back, each with the layout above.
-//
-// Problems that share an operator come in groups of rep right-hand sides (problem b uses
-// operator b / rep).  Such launches renumber their workgroups so that the rep workgroups of one
-// tile of one operator run one after another on one XCD (workgroups are dealt round-robin over
-// the 8 XCDs in launch order): the operator's tile comes from HBM once and from that XCD's L2
-// for the other right-hand sides.  t (the workgroup's tile, tiles per problem) and b (its
-// problem) are replaced by the logical pair; the map is a permutation of the launch, so every
-// tile of every problem is still done once.  Launches whose tiles per problem are not a
-// multiple of 8 keep the launch order.  Measured on 29 operators of 2049^2 with 4 right-hand
-// sides each (mixed V(1,1) line-xy solve): 688 against 720 ms.
-__device__ inline void shared_op_order(int tiles, int rep, int &t, int &b) {
-    if (rep <= 1 || tiles % 8 != 0) return;
-    const int op = b / rep;
-    const int off = (b - op * rep) * tiles + t;  // position in the operator's range, which
-    const int k = off / 8;                       // starts on an XCD-0 workgroup
-    t = (k / rep) * 8 + off % 8;
-    b = op * rep + k % rep;
-}
-
-// logical tile (x, y) and problem z of a tiled launch (problem index in blockIdx.z)
-struct wg_pos {
-    int x, y;
-    std::size_t z;
-};
-__device__ inline wg_pos tiled_wg(int rep) {
-    if (rep <= 1) return {(int)blockIdx.x, (int)blockIdx.y, (std::size_t)blockIdx.z};
-    int t = (int)(blockIdx.y * gridDim.x + blockIdx.x), b = (int)blockIdx.z;
-    shared_op_order((int)(gridDim.x * gridDim.y), rep, t, b);
-    return {t % (int)gridDim.x, t / (int)gridDim.x, (std::size_t)b};
-}
+//  Shared
+// operators: tile_order.hpp.
 
 // one block of 1024 threads: sum of n partials in a fixed order -> *out.  Thread t adds
 // partials t, t+1024, t+2048, ... in that order; loads are batched so they overlap.
@@ -1664,6 +1637,7 @@ template <typename T>
 void relax_gs(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj,
               int updown, hipStream_t s, int nb, int rep) {
     if (nstncl == 5) {
+        if (relax_gs9_rows<T>(so, qf, q, sor, ii, jj, updown, s, nb, rep)) return;
         // DOWN: (i odd, j odd), (even, odd), (odd, even), (even, even); UP: reverse
         static const int order[4][2] = {{1, 1}, {0, 1}, {1, 0}, {0, 0}};
         const dim3 g = gridb(ii / 2 + 1, jj / 2 + 1, nb);

@@ -68,6 +68,12 @@ template <typename T>
 void relax_gs(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj,
               int updown, hipStream_t s, int nb = 1, int rep = 1);
 
+// The nine-point relax_gs with both colours of a row in one launch; false (nothing launched) for
+// rows of more than 4096 points.
+template <typename T>
+bool relax_gs9_rows(const T *so, const T *qf, T *q, const T *sor, int ii, int jj, int updown,
+                    hipStream_t s, int nb, int rep);
+
 // LDL^T factors of every line (x: rows, y: columns, stored transposed); info (zero on entry)
 // is raised to the largest failing pivot index (1-based, line-local); it stays 0 when every
 // line is SPD.

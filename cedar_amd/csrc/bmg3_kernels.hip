@@ -11,6 +11,7 @@
 #include "band_chol.hpp"
 #include "bmg2_launch.hpp"
 #include "bmg3_launch.hpp"
+#include "bmg3_stencil.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -23,8 +24,6 @@ namespace {
 
 constexpr int WAVE = 64;
 
-// stencil planes, 1-based (src/3d/ftn/BMG_stencils_f90.h:46-48)
-enum { kp = 1, kpw, kps, kb, kpsw, kpnw, kbw, kbnw, kbn, kbne, kbe, kbse, kbs, kbsw };
 // prolongation planes, 1-based (src/3d/ftn/BMG_stencils_f90.h:59-65)
 enum {
     lxyl = 1, lxyr, lxya, lxyb, lxza, lxzb, lxyne, lxyse, lxysw, lxynw, lxzsw, lxznw, lxzne,
@@ -56,26 +55,6 @@ __device__ inline double lump3(double a, double b, double c, double p, double ep
 __device__ inline double lumpd(double dp, double s, double ep) {
     return dp + (s - dp) * dmax2(s - (1.0 + ep) * dp, 0.0) / (fabs(s - (1.0 + ep) * dp) + EMACH);
 }
-
-// ------------------------------------------------------------------------------------------
-// The 26 neighbour terms of the 27-point operator in the reference's order
-// (src/3d/ftn/BMG3_SymStd_residual.f90:71-97): X(si, sj, sk, plane, oi, oj, ok) = coefficient
-// at (i,j,k) + s times q at (i,j,k) + o.  The 7-point operator is the sub-list below
-// (src/3d/ftn/BMG3_SymStd_residual.f90:106-112).
-// ------------------------------------------------------------------------------------------
-#define NB27_LIST(X)                                                                              \
-    X(0, 0, 0, kpw, -1, 0, 0) X(0, 1, 0, kpnw, -1, 1, 0) X(0, 1, 0, kps, 0, 1, 0)                 \
-    X(1, 1, 0, kpsw, 1, 1, 0) X(1, 0, 0, kpw, 1, 0, 0) X(1, 0, 0, kpnw, 1, -1, 0)                 \
-    X(0, 0, 0, kps, 0, -1, 0) X(0, 0, 0, kpsw, -1, -1, 0) X(0, 0, 0, kb, 0, 0, -1)                \
-    X(0, 0, 0, kbw, -1, 0, -1) X(0, 1, 0, kbnw, -1, 1, -1) X(0, 1, 0, kbn, 0, 1, -1)              \
-    X(1, 1, 0, kbne, 1, 1, -1) X(1, 0, 0, kbe, 1, 0, -1) X(1, 0, 0, kbse, 1, -1, -1)              \
-    X(0, 0, 0, kbs, 0, -1, -1) X(0, 0, 0, kbsw, -1, -1, -1) X(0, 0, 1, kb, 0, 0, 1)               \
-    X(0, 0, 1, kbe, -1, 0, 1) X(0, 1, 1, kbse, -1, 1, 1) X(0, 1, 1, kbs, 0, 1, 1)                 \
-    X(1, 1, 1, kbsw, 1, 1, 1) X(1, 0, 1, kbw, 1, 0, 1) X(1, 0, 1, kbnw, 1, -1, 1)                 \
-    X(0, 0, 1, kbn, 0, -1, 1) X(0, 0, 1, kbne, -1, -1, 1)
-#define NB7_LIST(X)                                                                               \
-    X(0, 0, 0, kpw, -1, 0, 0) X(0, 1, 0, kps, 0, 1, 0) X(1, 0, 0, kpw, 1, 0, 0)                   \
-    X(0, 0, 0, kps, 0, -1, 0) X(0, 0, 0, kb, 0, 0, -1) X(0, 0, 1, kb, 0, 0, 1)
 
 #define CDR3_ADD(si, sj, sk, d, oi, oj, ok)                                                       \
     v = v + S3(i + (si), j + (sj), k + (sk), d) * Q3(q, i + (oi), j + (oj), k + (ok));
@@ -1523,6 +1502,7 @@ template <typename T>
 void relax_gs(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj, int kk,
               int updown, hipStream_t s) {
     if (nstncl == 14) {
+        if (relax_gs27_rows<T>(so, qf, q, sor, ii, jj, kk, updown, s)) return;
         // DOWN: colours pts = 8 .. 1, UP: 1 .. 8; colour pts starts at
         // (2 + mod(pts-1, 2), 2 + mod((pts-1)/2, 2), 2 + mod((pts-1)/4, 2))
         for (int t = 0; t < 8; ++t) {

@@ -38,6 +38,12 @@ template <typename T>
 void relax_gs(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj, int kk,
               int updown, hipStream_t s);
 
+// The 27-point relax_gs with both colours of a row in one launch; false (nothing launched) for rows
+// of more than 512 points.
+template <typename T>
+bool relax_gs27_rows(const T *so, const T *qf, T *q, const T *sor, int ii, int jj, int kk,
+                     int updown, hipStream_t s);
+
 template <typename T>
 void restrict_(const T *ci, const T *q, T *qc, int iif, int jjf, int kkf, int iic, int jjc,
                int kkc, hipStream_t s);

@@ -58,3 +58,77 @@ def test_galerkin3(dims, ns):
     inner = (slice(None),) + (slice(1, -1),) * 3
     assert np.array_equal(host(soc)[inner], ref[inner])
     assert (host(soc)[:, 0] == 7.0).all() and (host(soc)[:, :, :, -1] == 7.0).all()  # ghosts untouched
+
+
+def _so2(rng, nx, ny, ns):
+    """Random couplings inside the grid, diagonally dominant, zero across the boundary."""
+    so = np.zeros((ns, ny + 2, nx + 2))
+    so[1, 1:-1, 2:-1] = rng.uniform(0.1, 1.0, (ny, nx - 1))
+    so[2, 2:-1, 1:-1] = rng.uniform(0.1, 1.0, (ny - 1, nx))
+    if ns == 5:
+        so[3, 2:-1, 2:-1] = rng.uniform(0.1, 1.0, (ny - 1, nx - 1))
+        so[4, 2:-1, 2:-1] = rng.uniform(0.1, 1.0, (ny - 1, nx - 1))
+    so[0, 1:-1, 1:-1] = 9.0
+    return so
+
+
+# rows of 64, 128, ... points, one less and one more (thread classes), odd and even, up to the
+# longest row of the fused kernel and beyond; boundary values that are not zero.  Extents of at
+# least 2: with one the oracle's loops over the second colour run into the ghost layer.
+@pytest.mark.parametrize("nx,ny", [(2, 2), (2, 3), (3, 2), (63, 9), (64, 8), (65, 17), (128, 5),
+                                   (129, 4), (257, 6), (512, 3), (513, 3), (1025, 3), (2047, 4),
+                                   (2049, 3), (4096, 2), (4097, 3)])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_gs9_rows(nx, ny, dtype):
+    import cedar_amd as C
+    print(f"\ngs9 {nx}x{ny} {dtype}", flush=True)
+    rng = np.random.default_rng(nx + ny)
+    dt = torch.float64 if dtype == "f64" else torch.float32
+    q, qf = rng.standard_normal((ny + 2, nx + 2)), rng.standard_normal((ny + 2, nx + 2))
+    so = _so2(rng, nx, ny, 5)
+    sor = O.setup_recip(so)
+    for ud in (O.DOWN, O.UP):
+        ref = O.relax_gs(so, qf, q, sor, ud)
+        g = host(C.relax_gs(dev(so, dt), dev(qf, dt), dev(q, dt), dev(sor, dt), ud))
+        if dtype == "f64":
+            assert np.array_equal(g, ref), ud
+        else:  # 9 products and sums of values of order 1 a point, two colours deep
+            assert np.abs(g - ref).max() <= 20 * 2.0 ** -24 * np.abs(ref).max(), ud
+
+
+def test_gs9_rows_batch_of_shared_operators():
+    """Several right-hand sides per operator: each problem as if relaxed alone."""
+    import cedar_amd as C
+    rng = np.random.default_rng(3)
+    nops, nrhs, nx, ny = 3, 4, 130, 70
+    ops = np.stack([_so2(rng, nx, ny, 5) for _ in range(nops)])
+    b = rng.standard_normal((nops * nrhs, ny + 2, nx + 2))
+    kw = dict(relaxation="point", maxiter=3, tol=1e-30)
+    x, _ = C.Solver(dev(ops), nrhs=nrhs, **kw).solve(dev(b))
+    for k in range(nops * nrhs):
+        one, _ = C.Solver(dev(ops[k // nrhs]), **kw).solve(dev(b[k]))
+        assert torch.equal(x[k], one), k
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (2, 3, 3), (15, 4, 5), (16, 5, 4), (17, 9, 3),
+                                  (33, 6, 7), (64, 3, 4), (65, 7, 2), (129, 3, 3), (257, 3, 2),
+                                  (512, 2, 3), (513, 3, 2)])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_gs27_rows(dims, dtype):
+    import cedar_amd as C
+    print(f"\ngs27 {dims} {dtype}", flush=True)
+    nx, ny, nz = dims
+    rng = np.random.default_rng(sum(dims))
+    dt = torch.float64 if dtype == "f64" else torch.float32
+    so = rand_so3(rng, nx, ny, nz, 14)
+    shp = (nz + 2, ny + 2, nx + 2)
+    q, qf = rng.standard_normal(shp), rng.standard_normal(shp)
+    sor = O3.setup_recip(so)
+    K = C.cdr3
+    for ud in (K.DOWN, K.UP):
+        ref = O3.relax_gs(so, qf, q, sor, ud)
+        g = host(K.relax_gs(dev(so, dt), dev(qf, dt), dev(q, dt), dev(sor, dt), ud))
+        if dtype == "f64":
+            assert np.array_equal(g, ref), ud
+        else:  # 27 products and sums a point, eight colours deep
+            assert np.abs(g - ref).max() <= 100 * 2.0 ** -24 * np.abs(ref).max(), ud
