@@ -15,6 +15,7 @@
 // accesses along i, 64-wide wavefronts, deterministic fixed-order reductions.
 #include "../../include/cedar_hip.h"
 #include "band_chol.hpp"
+#include "bmg2_device.hpp"
 #include "bmg2_launch.hpp"
 #include "tile_order.hpp"
 
@@ -35,48 +36,8 @@ namespace k2 {
 
 namespace {
 
-constexpr int WAVE = 64;
-
-__host__ __device__ inline std::size_t pidx(int i, int j, int ii) {
-    return (std::size_t)j * (std::size_t)ii + (std::size_t)i;
-}
-
 inline dim3 grid2(int nx, int ny, int bx, int by) {
     return dim3((unsigned)((nx + bx - 1) / bx), (unsigned)((ny + by - 1) / by), 1);
-}
-
-// ------------------------------------------------------------------------------------------
-// deterministic block reduction of one double per thread (256 threads = 4 waves)
-// ------------------------------------------------------------------------------------------
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    return v;
-}
-
-// barrier that orders LDS only: prefetched global loads stay in flight across it
-__device__ inline void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// LDS_ONLY: the barrier orders LDS alone (global loads issued before it stay in flight)
-template <int NWAVES = 4, bool LDS_ONLY = false>
-__device__ inline void block_sum_store(double v, double *dst) {
-    __shared__ double part[NWAVES];
-    v = wave_sum(v);
-    int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    if (lane == 0) part[wid] = v;
-    if (LDS_ONLY)
-        lds_barrier();
-    else
-        __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = part[0];
-        for (int w = 1; w < NWAVES; ++w) t += part[w];
-        *dst = t;
-    }
 }
 
 // Batched problems: every kernel below takes the problem index from the last grid dimension
@@ -109,22 +70,6 @@ __global__ __launch_bounds__(1024) void finalize_sum_k(const double *__restrict_
 // residual  r = f + sum(couplings * q) - c q   (src/2d/ftn/BMG2_SymStd_residual.f90:85-119)
 // block: 64 (i) x 4 (j)
 // ------------------------------------------------------------------------------------------
-template <typename T, bool NINE>
-__device__ inline T apply_offdiag(const T *__restrict__ so, std::size_t P, const T *__restrict__ q,
-                                  std::size_t p, int ii, T acc) {
-    acc = acc + so[P * KW + p] * q[p - 1];
-    acc = acc + so[P * KW + p + 1] * q[p + 1];
-    acc = acc + so[P * KS + p] * q[p - ii];
-    acc = acc + so[P * KS + p + ii] * q[p + ii];
-    if (NINE) {
-        acc = acc + so[P * KSW + p] * q[p - ii - 1];
-        acc = acc + so[P * KNW + p + 1] * q[p - ii + 1];
-        acc = acc + so[P * KNW + p + ii] * q[p + ii - 1];
-        acc = acc + so[P * KSW + p + ii + 1] * q[p + ii + 1];
-    }
-    return acc;
-}
-
 template <typename T, bool NINE, bool NORM>
 __global__ __launch_bounds__(256) void residual_k(const T *__restrict__ so, const T *__restrict__ qf,
                                                   const T *__restrict__ q, T *__restrict__ res,
@@ -384,649 +329,10 @@ __global__ void setup_lines_y_k(const double *__restrict__ so, double *__restric
     if (!(D[n - 1] > 0.0)) atomicMax(info, n);
 }
 
-// Inclusive scans of affine maps y -> a*y + b across the 64 lanes of a wavefront.
-// up:   lane l gets F_l o F_{l-1} o ... o F_0        (forward substitution)
-// down: lane l gets G_l o G_{l+1} o ... o G_63       (backward substitution)
-template <typename T>
-__device__ inline void scan_affine_up(T &a, T &b, int lane) {
-#pragma unroll
-    for (int d = 1; d < WAVE; d <<= 1) {
-        const T ap = __shfl_up(a, d, WAVE);
-        const T bp = __shfl_up(b, d, WAVE);
-        if (lane >= d) {
-            b = a * bp + b;
-            a = a * ap;
-        }
-    }
-}
-
-template <typename T>
-__device__ inline void scan_affine_down(T &a, T &b, int lane) {
-#pragma unroll
-    for (int d = 1; d < WAVE; d <<= 1) {
-        const T an = __shfl_down(a, d, WAVE);
-        const T bn = __shfl_down(b, d, WAVE);
-        if (lane + d < WAVE) {
-            b = a * bn + b;
-            a = a * an;
-        }
-    }
-}
-
-// Same inclusive scan with DPP lane moves (row_shr 1/2/4/8 inside 16-lane rows, then
-// row_bcast 15 and 31 across rows) instead of LDS permutes: a few cycles per step, which keeps
-// the carry chain of a line short.  Lanes whose source is out of range keep the identity (1, 0).
-template <int CTRL, int RMASK>
-__device__ inline float dpp_move(float v, float ident) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, ident),
-                                                                 __builtin_bit_cast(int, v), CTRL,
-                                                                 RMASK, 0xF, false));
-}
-
-template <int CTRL, int RMASK>
-__device__ inline double dpp_move(double v, double ident) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned long long o = __builtin_bit_cast(unsigned long long, ident);
-    const int lo = __builtin_amdgcn_update_dpp((int)(unsigned)o, (int)(unsigned)u, CTRL, RMASK, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(unsigned)(o >> 32), (int)(unsigned)(u >> 32), CTRL,
-                                               RMASK, 0xF, false);
-    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-
-// The affine step a * c + b of the line recurrences: a fused multiply-add in FP32 (the
-// preconditioning V-cycle of the mixed solver), separate rounding in FP64.  Every line kernel
-// evaluates its recurrences through this one function, so all of them (every launch shape, the
-// direct and the transposed y sweeps, the fused coarse cycle) still round identically.
-__device__ inline float affine(float a, float c, float b) { return __builtin_fmaf(a, c, b); }
-__device__ inline double affine(double a, double c, double b) { return a * c + b; }
-// y / d for a line pivot d: FP32 multiplies by the hardware reciprocal (about 1 ulp), FP64
-// divides (correctly rounded, as the sequential substitution does).
-__device__ inline float div_pivot(float y, float d) { return y * __builtin_amdgcn_rcpf(d); }
-__device__ inline double div_pivot(double y, double d) { return y / d; }
-
-// the source lane's value, 0 where the source lane is out of range or the row is masked off
-template <int CTRL, int RMASK>
-__device__ inline float dpp_zero(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                                 CTRL, RMASK, 0xF, true));
-}
-template <int CTRL, int RMASK>
-__device__ inline double dpp_zero(double v) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, RMASK, 0xF, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, RMASK, 0xF, true);
-    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-
-// lanes that receive a value in each step of the scan (row_shr:1/2/4/8 within 16-lane rows,
-// row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3); the others keep (a, b)
-__device__ inline int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
-template <int STEP>
-__device__ inline bool dpp_valid(int lane) {
-    return STEP == 0 ? (lane & 15) >= 1 : STEP == 1 ? (lane & 15) >= 2 : STEP == 2 ? (lane & 15) >= 4
-         : STEP == 3 ? (lane & 15) >= 8 : STEP == 4 ? ((lane >> 4) & 1) != 0 : lane >= 32;
-}
-
-// One step: (a, b) <- (a * a', a * b' + b) with (a', b') from the source lane.  Where no value
-// arrives, b' reads 0 (a * 0 + b = b exactly) and a is kept: the identity map.  The product
-// a * b' is rounded on its own in both precisions (a multiply that takes its lane move for free
-// is cheaper here than a fused multiply-add, which cannot).
-// The broadcast steps move data into every row (row 0 reads 0); the lanes outside the rows the
-// step feeds are then restored by the select, as the row_shr steps restore a.
-template <int CTRL, int STEP, typename T>
-__device__ inline void dpp_scan_step(T &a, T &b, int lane) {
-    const T ap = dpp_zero<CTRL, 0xF>(a);
-    const T bp = dpp_zero<CTRL, 0xF>(b);
-    const bool v = dpp_valid<STEP>(lane);
-    const T bn = a * bp + b;
-    b = (STEP < 4 || v) ? bn : b;
-    a = v ? a * ap : a;
-}
-
-template <typename T>
-__device__ inline void scan_affine_dpp(T &a, T &b) {
-    const int lane = lane_id();
-    dpp_scan_step<0x111, 0>(a, b, lane);  // row_shr:1
-    dpp_scan_step<0x112, 1>(a, b, lane);  // row_shr:2
-    dpp_scan_step<0x114, 2>(a, b, lane);  // row_shr:4
-    dpp_scan_step<0x118, 3>(a, b, lane);  // row_shr:8
-    dpp_scan_step<0x142, 4>(a, b, lane);  // row_bcast:15, kept in rows 1 and 3
-    dpp_scan_step<0x143, 5>(a, b, lane);  // row_bcast:31, kept in rows 2 and 3
-}
-
-// the multiplier part of scan_affine_dpp alone (the same products in the same order)
-template <int CTRL, int STEP, typename T>
-__device__ inline void dpp_prod_step(T &a, int lane) {
-    const T ap = dpp_zero<CTRL, 0xF>(a);
-    a = dpp_valid<STEP>(lane) ? a * ap : a;
-}
-
-template <typename T>
-__device__ inline void scan_prod_dpp(T &a) {
-    const int lane = lane_id();
-    dpp_prod_step<0x111, 0>(a, lane);
-    dpp_prod_step<0x112, 1>(a, lane);
-    dpp_prod_step<0x114, 2>(a, lane);
-    dpp_prod_step<0x118, 3>(a, lane);
-    dpp_prod_step<0x142, 4>(a, lane);
-    dpp_prod_step<0x143, 5>(a, lane);
-}
-
-// value of lane 63, broadcast (v_readlane: no LDS round trip)
-__device__ inline float last_lane(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), WAVE - 1));
-}
-__device__ inline double last_lane(double v) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, WAVE - 1);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), WAVE - 1);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// One wavefront solves one line: L D L^T x = rhs with the stored factors.  Forward pass in
-// 64-element chunks: y_k = rhs_k - E_{k-1} y_{k-1}, stores c_k = y_k / D_k in place of q;
-// backward pass: x_k = c_k - E_k x_{k+1}.  A line of one colour only reads lines of the other
-// colour, so the in-place staging is race free.
-//
-// DIR 0: x-lines (row j = first + 2*line, elements along i, unit stride)
-// DIR 1: y-lines (column i = first + 2*line, elements along j, stride ii; factors transposed)
-template <typename T, bool NINE, int DIR>
-__global__ __launch_bounds__(256) void relax_lines_k(const T *__restrict__ so, const T *__restrict__ qf,
-                                                     T *__restrict__ q, const T *__restrict__ sor,
-                                                     int ii, int jj, int first, int nlines, int rep) {
-    const int lane = threadIdx.x % WAVE;
-    int bx = (int)blockIdx.x, prob = (int)blockIdx.y;
-    shared_op_order((int)gridDim.x, rep, bx, prob);
-    const int line = bx * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-    if (line >= nlines) return;  // whole wavefront leaves together; no block barrier below
-    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = bz / rep;
-    so += bo * (NINE ? 5 : 3) * P;
-    qf += bz * P;
-    q += bz * P;
-    sor += bo * 2 * P;
-    const int fixed = first + 2 * line;
-    const int n = (DIR == 0) ? ii - 2 : jj - 2;
-    const std::size_t stride = (DIR == 0) ? 1 : (std::size_t)ii;
-    const std::size_t base = (DIR == 0) ? pidx(1, fixed, ii) : pidx(fixed, 1, ii);  // element 0
-    const T *D = (DIR == 0) ? sor + pidx(1, fixed, ii) : sor + (std::size_t)fixed * jj + 1;
-    const T *E = (DIR == 0) ? sor + P + pidx(2, fixed, ii) : sor + P + (std::size_t)fixed * jj + 2;
-    const int nch = (n + WAVE - 1) / WAVE;
-
-    T carry = T(0);
-    for (int c = 0; c < nch; ++c) {
-        const int k = c * WAVE + lane;
-        const bool act = k < n;
-        T a = T(0), b = T(0);
-        if (act) {
-            const std::size_t p = base + (std::size_t)k * stride;
-            T rhs = qf[p];
-            if (DIR == 0) {
-                rhs = rhs + so[P * KS + p] * q[p - ii];
-                rhs = rhs + so[P * KS + p + ii] * q[p + ii];
-            } else {
-                rhs = rhs + so[P * KW + p] * q[p - 1];
-                rhs = rhs + so[P * KW + p + 1] * q[p + 1];
-            }
-            if (NINE) {
-                rhs = rhs + so[P * KSW + p] * q[p - ii - 1];
-                rhs = rhs + so[P * KNW + p + 1] * q[p - ii + 1];
-                rhs = rhs + so[P * KNW + p + ii] * q[p + ii - 1];
-                rhs = rhs + so[P * KSW + p + ii + 1] * q[p + ii + 1];
-            }
-            b = rhs;
-            a = (k > 0) ? -E[k - 1] : T(0);
-        }
-        scan_affine_up(a, b, lane);
-        const T y = affine(a, carry, b);
-        carry = __shfl(y, WAVE - 1, WAVE);
-        if (act) q[base + (std::size_t)k * stride] = div_pivot(y, D[k]);
-    }
-    carry = T(0);
-    for (int c = nch - 1; c >= 0; --c) {
-        const int k = c * WAVE + lane;
-        const bool act = k < n;
-        T a = T(1), b = T(0);
-        if (act) {
-            b = q[base + (std::size_t)k * stride];
-            a = (k < n - 1) ? -E[k] : T(0);
-        }
-        scan_affine_down(a, b, lane);
-        const T x = affine(a, carry, b);
-        carry = __shfl(x, 0, WAVE);
-        if (act) q[base + (std::size_t)k * stride] = x;
-    }
-}
-
-// Workgroup index remapped so that consecutive logical tiles run on the same XCD (workgroups
-// are dealt round-robin over the 8 XCDs): neighbouring lines share rows of q and of the
-// operator, which then stay in one XCD's L2.  Launch 8 * ceil(ntiles / 8) workgroups.
-// rev: each XCD walks its range of tiles from the end, so that a launch starts on the lines the
-// previous launch touched last (still in the memory-side cache); the work is unchanged.
-__device__ inline int xcd_tile(int bx, int ntiles, int rev = 0) {
-    const int per = (ntiles + 7) / 8;
-    const int k = bx / 8;
-    return (bx % 8) * per + (rev ? per - 1 - k : k);
-}
-
-// raw operands of the right-hand side of one point of a line
-template <typename T>
-struct line_raw {
-    T qf, s0, q0, s1, q1, sw0, q0m, nw0, q0p, nw1, q1m, sw1, q1p;
-};
-
-// Right-hand side of one point in the reference's order.  X-lines: s0/q0 = coupling to the row
-// below, s1/q1 = to the row above; y-lines: the column to the left / right.
-// SWAP adds the two NW terms in the opposite order: an x-line of the transposed grid then sums
-// its terms in exactly the order of the corresponding y-line of the original grid.
-template <typename T, bool NINE, bool SWAP = false>
-__device__ inline T line_rhs(const line_raw<T> &r) {
-    T rhs = r.qf;
-    rhs = affine(r.s0, r.q0, rhs);
-    rhs = affine(r.s1, r.q1, rhs);
-    if (NINE) {
-        rhs = affine(r.sw0, r.q0m, rhs);
-        if (SWAP) {
-            rhs = affine(r.nw1, r.q1m, rhs);
-            rhs = affine(r.nw0, r.q0p, rhs);
-        } else {
-            rhs = affine(r.nw0, r.q0p, rhs);
-            rhs = affine(r.nw1, r.q1m, rhs);
-        }
-        rhs = affine(r.sw1, r.q1p, rhs);
-    }
-    return rhs;
-}
-
-// loads the operands of point p (array index) of an x-line (DIR 0) or y-line (DIR 1)
-template <typename T, bool NINE, int DIR>
-__device__ inline void line_load(line_raw<T> &r, const T *__restrict__ so, const T *__restrict__ qf,
-                                 const T *__restrict__ q, std::size_t P, int ii, std::size_t p,
-                                 bool zq = false) {
-    r.qf = qf[p];
-    if (DIR == 0) {
-        r.s0 = so[P * KS + p];
-        r.q0 = zq ? T(0) : q[p - ii];
-        r.s1 = so[P * KS + p + ii];
-        r.q1 = zq ? T(0) : q[p + ii];
-    } else {
-        r.s0 = so[P * KW + p];
-        r.q0 = zq ? T(0) : q[p - 1];
-        r.s1 = so[P * KW + p + 1];
-        r.q1 = zq ? T(0) : q[p + 1];
-    }
-    if (NINE) {
-        r.sw0 = so[P * KSW + p];
-        r.q0m = zq ? T(0) : q[p - ii - 1];
-        r.nw0 = so[P * KNW + p + 1];
-        r.q0p = zq ? T(0) : q[p - ii + 1];
-        r.nw1 = so[P * KNW + p + ii];
-        r.q1m = zq ? T(0) : q[p + ii - 1];
-        r.sw1 = so[P * KSW + p + ii + 1];
-        r.q1p = zq ? T(0) : q[p + ii + 1];
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// Segmented line solves.  W wavefronts share a line: wavefront w owns the CPW chunks
-// [w*CPW, (w+1)*CPW) of 64 elements.  Every operand of a wavefront's chunks is loaded before the
-// first scan, so no load latency sits inside the carry chain, and at most CPW chunks live in
-// registers; W wavefronts per line put W times as many wavefronts in flight as there are lines.
-//
-// The carries between chunks are evaluated in exactly the single-wavefront order: chunk m's
-// scanned map (a_m, b_m) at its last element goes to LDS, and the carry into chunk m is
-// c_m = a_{m-1} c_{m-1} + b_{m-1} from c_0 = 0, the same operations the one-wavefront loop
-// performs.  Results are therefore bitwise identical for every (CPW, W) and workgroup shape, so
-// the shape can be picked by timing alone.
-// ------------------------------------------------------------------------------------------
-template <typename T>
-struct seg_map {
-    T a, b;  // carry_out = a * carry_in + b
-};
-
-// Forward recurrence y_k = a_k y_{k-1} + b_k over the wavefront's chunks.  On entry b[u] holds
-// chunk u's right-hand sides; afun(u) returns its multipliers a_k (reloaded when needed, so that
-// only b stays in registers) and dval(u) its pivots.  On exit b[u] = y_k / d_k.  xch: this
-// line's LDS slots, one per chunk of the line.
-template <typename T, int CPW, int W, typename AF, typename DF>
-__device__ inline void seg_forward(T (&b)[CPW], AF afun, DF dval, seg_map<T> *xch, int w) {
-    if (W > 1) {
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) {
-            T a = afun(u);
-            scan_affine_dpp(a, b[u]);
-            const seg_map<T> m{last_lane(a), last_lane(b[u])};
-            if (w < W - 1 && threadIdx.x % WAVE == 0) xch[w * CPW + u] = m;
-        }
-        lds_barrier();
-        // the multipliers are reloaded below rather than kept live across the exchange
-        asm volatile("" ::: "memory");
-    }
-    T carry = T(0);
-    for (int m = 0; m < w * CPW; ++m) carry = affine(xch[m].a, carry, xch[m].b);
-#pragma unroll
-    for (int u = 0; u < CPW; ++u) {
-        T a = afun(u);
-        if (W > 1)
-            scan_prod_dpp(a);
-        else
-            scan_affine_dpp(a, b[u]);
-        const T y = affine(a, carry, b[u]);
-        carry = last_lane(y);
-        b[u] = div_pivot(y, dval(u));
-    }
-}
-
-// Backward recurrence x_k = a_k x_{k+1} + b_k, lanes in reversed element order (lane l of chunk
-// c holds element 64c + 63 - l); the carry runs from the line's last chunk to its first.
-// coef(u, a, b[u]) turns b[u] (the forward results) into the chunk's coefficients and returns
-// the multipliers in a; afun(u) returns the multipliers alone.  On exit b[u] = x.
-template <typename T, int CPW, int W, typename CF, typename AF>
-__device__ inline void seg_backward(T (&b)[CPW], CF coef, AF afun, seg_map<T> *xch, int w) {
-    if (W > 1) {
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) {
-            T a;
-            coef(u, a, b[u]);
-            scan_affine_dpp(a, b[u]);
-            const seg_map<T> m{last_lane(a), last_lane(b[u])};
-            if (w > 0 && threadIdx.x % WAVE == 0) xch[w * CPW + u] = m;
-        }
-        lds_barrier();
-        // the multipliers are reloaded below rather than kept live across the exchange
-        asm volatile("" ::: "memory");
-    }
-    T carry = T(0);
-    for (int m = W * CPW - 1; m >= (w + 1) * CPW; --m) carry = affine(xch[m].a, carry, xch[m].b);
-#pragma unroll
-    for (int u = CPW - 1; u >= 0; --u) {
-        T a;
-        if (W > 1) {
-            a = afun(u);
-            scan_prod_dpp(a);
-        } else {
-            coef(u, a, b[u]);
-            scan_affine_dpp(a, b[u]);
-        }
-        const T x = affine(a, carry, b[u]);
-        carry = last_lane(x);
-        b[u] = x;
-    }
-}
-
-// Register-rich forms of the two recurrences (scanned multipliers kept in a[]), used by the
-// x-line kernel: forward recurrence y_k = a_k y_{k-1} + b_k over the wavefront's chunks; on exit
-// b[u] = y_k / D(u) with D(u) the pivots of chunk u (a functor, loaded after the scans).
-// xch: this line's LDS slots, one per chunk of the line.
-template <typename T, int CPW, int W, typename DF>
-__device__ inline void seg_forward_ab(T (&a)[CPW], T (&b)[CPW], DF dval, seg_map<T> *xch, int w) {
-#pragma unroll
-    for (int u = 0; u < CPW; ++u) scan_affine_dpp(a[u], b[u]);
-    T carry = T(0);
-    if (W > 1) {
-        if (w < W - 1) {  // chunk-end maps of all but the last segment
-#pragma unroll
-            for (int u = 0; u < CPW; ++u) {
-                const seg_map<T> m{last_lane(a[u]), last_lane(b[u])};
-                if (threadIdx.x % WAVE == 0) xch[w * CPW + u] = m;
-            }
-        }
-        lds_barrier();
-        for (int m = 0; m < w * CPW; ++m) carry = affine(xch[m].a, carry, xch[m].b);
-    }
-#pragma unroll
-    for (int u = 0; u < CPW; ++u) {
-        const T y = affine(a[u], carry, b[u]);
-        carry = last_lane(y);
-        b[u] = div_pivot(y, dval(u));
-    }
-}
-
-// Backward recurrence x_k = a_k x_{k+1} + b_k, lanes in reversed element order (lane l of chunk
-// c holds element 64c + 63 - l); the carry runs from the line's last chunk to its first.  On
-// exit b[u] = x.
-template <typename T, int CPW, int W>
-__device__ inline void seg_backward_ab(T (&a)[CPW], T (&b)[CPW], seg_map<T> *xch, int w) {
-#pragma unroll
-    for (int u = 0; u < CPW; ++u) scan_affine_dpp(a[u], b[u]);
-    T carry = T(0);
-    if (W > 1) {
-        if (w > 0) {
-#pragma unroll
-            for (int u = 0; u < CPW; ++u) {
-                const seg_map<T> m{last_lane(a[u]), last_lane(b[u])};
-                if (threadIdx.x % WAVE == 0) xch[w * CPW + u] = m;
-            }
-        }
-        lds_barrier();
-        for (int m = W * CPW - 1; m >= (w + 1) * CPW; --m) carry = affine(xch[m].a, carry, xch[m].b);
-    }
-#pragma unroll
-    for (int u = CPW - 1; u >= 0; --u) {
-        const T x = affine(a[u], carry, b[u]);
-        carry = last_lane(x);
-        b[u] = x;
-    }
-}
-
-// x-lines of one colour, in place: L lines per workgroup, W wavefronts per line.  TR: the grid
-// is the transpose of a y-line problem (right-hand side terms in the y-line order).
-// rev: the tile walk of xcd_tile.  ZQ (zero start): q holds zeros outside the lines of this
-// colour (a sweep that starts from a zero iterate), so the neighbour rows are not read and
-// literal zeros enter the same arithmetic (a compile-time switch: a run-time select in front of
-// the loads slowed the kernel by a quarter).
-template <typename T, bool NINE, int CPW, int W, int L, bool TR = false, bool ZQ = false>
-__global__ __launch_bounds__(L *W * 64) void relax_xlines_seg_k(const T *__restrict__ so,
-                                                               const T *__restrict__ qf,
-                                                               T *__restrict__ q,
-                                                               const T *__restrict__ sor, int ii,
-                                                               int jj, int first, int nlines,
-                                                               int ntiles, int rev, int rep) {
-    __shared__ seg_map<T> xch[2][L][W > 1 ? W * CPW : 1];
-    int bx = (int)blockIdx.x, prob = (int)blockIdx.y;
-    shared_op_order((int)gridDim.x, rep, bx, prob);  // gridDim.x is a multiple of 8
-    const int tile = xcd_tile(bx, ntiles, rev);
-    if (tile >= ntiles) return;  // uniform over the workgroup
-    const int wl = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const int slot = wl / W, w = wl % W;
-    const int line = tile * L + slot;
-    const bool valid = line < nlines;  // invalid wavefronts solve a copy of the last line
-    const int j = first + 2 * min(line, nlines - 1);
-    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = bz / rep;
-    so += bo * (NINE ? 5 : 3) * P;
-    qf += bz * P;
-    q += bz * P;
-    sor += bo * 2 * P;
-    const int n = ii - 2;
-    const std::size_t row = (std::size_t)j * ii;
-    const T *D = sor + row + 1;      // D[k]
-    const T *E = sor + P + row + 2;  // E[k], k < n-1
-    const int rl = WAVE - 1 - lane;
-    auto bwd_coef = [&](int u, T &au, T &bu) {  // chunk u of the backward pass, reversed lanes
-        const int k = (w * CPW + u) * WAVE + rl;
-        const T c = __shfl(bu, rl, WAVE);
-        const T e = E[min(k, max(n - 2, 0))];
-        au = (k < n - 1) ? -e : T(0);
-        au = (k < n) ? au : T(1);
-        bu = (k < n) ? c : T(0);
-    };
-    T b[CPW];
-    if constexpr (W == 1) {
-        // one wavefront per line: scan and carry chunk by chunk, only the results kept
-        T carry = T(0);
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) {
-            const int k = u * WAVE + lane;
-            const int kc = min(k, n - 1);
-            line_raw<T> r;
-            line_load<T, NINE, 0>(r, so, qf, q, P, ii, row + kc + 1, ZQ);
-            T bu = line_rhs<T, NINE, TR>(r);
-            T au = (k > 0) ? -E[max(kc - 1, 0)] : T(0);
-            scan_affine_dpp(au, bu);
-            const T y = affine(au, carry, bu);
-            carry = last_lane(y);
-            b[u] = div_pivot(y, D[kc]);
-        }
-        carry = T(0);
-#pragma unroll
-        for (int u = CPW - 1; u >= 0; --u) {
-            T au;
-            bwd_coef(u, au, b[u]);
-            scan_affine_dpp(au, b[u]);
-            const T x = affine(au, carry, b[u]);
-            carry = last_lane(x);
-            b[u] = x;
-        }
-    } else {
-        T a[CPW];
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) {
-            const int k = (w * CPW + u) * WAVE + lane;
-            const int kc = min(k, n - 1);
-            line_raw<T> r;
-            line_load<T, NINE, 0>(r, so, qf, q, P, ii, row + kc + 1, ZQ);
-            b[u] = line_rhs<T, NINE, TR>(r);
-            a[u] = (k > 0) ? -E[max(kc - 1, 0)] : T(0);
-        }
-        seg_forward_ab<T, CPW, W>(
-            a, b, [&](int u) { return D[min((w * CPW + u) * WAVE + lane, n - 1)]; },
-            xch[0][slot], w);
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) bwd_coef(u, a[u], b[u]);
-        seg_backward_ab<T, CPW, W>(a, b, xch[1][slot], w);
-    }
-    if (valid) {
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) {
-            const int k = (w * CPW + u) * WAVE + rl;
-            if (k < n) q[row + k + 1] = b[u];
-        }
-    }
-}
-
-// y-lines of one colour, in place: NC columns per workgroup, W wavefronts per column.  The
-// right-hand sides of G chunk rows at a time are formed by the whole workgroup with
-// row-contiguous loads (thread t: column t % NC, row t / NC of the W*64 rows) and handed to the
-// column owners through LDS; results return through LDS for row-contiguous stores.
-template <typename T, bool NINE, int CPW, int W, int NC, int G>
-__global__ __launch_bounds__(NC *W * 64) void relax_ylines_seg_k(const T *__restrict__ so,
-                                                                const T *__restrict__ qf,
-                                                                T *__restrict__ q,
-                                                                const T *__restrict__ sor,
-                                                                int ii, int jj, int first,
-                                                                int ncols, int ntiles, int rev,
-                                                                int rep) {
-    static_assert(CPW % G == 0, "G must divide CPW");
-    __shared__ T tile_s[G][W][NC][WAVE + 1];
-    __shared__ seg_map<T> xch[2][NC][W > 1 ? W * CPW : 1];
-    int bx = (int)blockIdx.x, prob = (int)blockIdx.y;
-    shared_op_order((int)gridDim.x, rep, bx, prob);  // gridDim.x is a multiple of 8
-    const int tile = xcd_tile(bx, ntiles, rev);
-    if (tile >= ntiles) return;  // uniform over the workgroup
-    const int wl = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const int cs = wl / W, w = wl % W;
-    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = bz / rep;
-    so += bo * (NINE ? 5 : 3) * P;
-    qf += bz * P;
-    q += bz * P;
-    sor += bo * 2 * P;
-    const int n = jj - 2;
-    const int col0 = tile * NC;
-    const int nc = min(NC, ncols - col0);
-    const int cb = first + 2 * col0;
-    // the wavefront's own column (factors contiguous in j)
-    const int ime = cb + 2 * min(cs, nc - 1);
-    const T *D = sor + (std::size_t)ime * jj + 1;
-    const T *E = sor + P + (std::size_t)ime * jj + 2;
-    // this thread's tile position for the right-hand sides and the stores
-    const int tc = threadIdx.x % NC, tr = threadIdx.x / NC;
-    const int tseg = tr / WAVE, trow = tr % WAVE;
-    const bool tok = tc < nc;
-    const int ti = cb + 2 * min(tc, nc - 1);
-    const int rl = WAVE - 1 - lane;
-    auto fwd_a = [&](int u) {  // forward coefficient of chunk u
-        const int k = (w * CPW + u) * WAVE + lane;
-        return (k > 0) ? -E[max(min(k, n - 1) - 1, 0)] : T(0);
-    };
-    // Right-hand sides of chunk rows g .. g+G-1 go through the tile.  The raw operands of the
-    // next group are loaded before the current group's barrier (software pipelining), so one
-    // group of loads is always in flight across the LDS exchange.
-    line_raw<T> raw[G];
-    auto load_group = [&](int g) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int k = min((tseg * CPW + g + u) * WAVE + trow, n - 1);
-            line_load<T, NINE, 1>(raw[u], so, qf, q, P, ii, pidx(ti, k + 1, ii));
-        }
-    };
-    auto form_tile = [&](int g) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) tile_s[u][tseg][tc][trow] = line_rhs<T, NINE>(raw[u]);
-        if (g + G < CPW) load_group(g + G);
-    };
-    load_group(0);
-    auto bwd_a = [&](int u) {  // backward multipliers of chunk u, reversed lanes
-        const int k = (w * CPW + u) * WAVE + rl;
-        const T e = E[min(k, max(n - 2, 0))];
-        const T a = (k < n - 1) ? -e : T(0);
-        return (k < n) ? a : T(1);
-    };
-    auto bwd_coef = [&](int u, T &au, T &bu) {
-        const int k = (w * CPW + u) * WAVE + rl;
-        const T c = __shfl(bu, rl, WAVE);
-        au = bwd_a(u);
-        bu = (k < n) ? c : T(0);
-    };
-    // all right-hand sides first (memory streaming only), then the scans
-    T b[CPW];
-#pragma unroll
-    for (int g = 0; g < CPW; g += G) {
-        form_tile(g);
-        lds_barrier();
-#pragma unroll
-        for (int u = 0; u < G; ++u) b[g + u] = tile_s[u][w][cs][lane];
-        lds_barrier();
-    }
-    seg_forward<T, CPW, W>(
-        b, fwd_a, [&](int u) { return D[min((w * CPW + u) * WAVE + lane, n - 1)]; }, xch[0][cs],
-        w);
-    seg_backward<T, CPW, W>(b, bwd_coef, bwd_a, xch[1][cs], w);
-#pragma unroll
-    for (int g = 0; g < CPW; g += G) {
-#pragma unroll
-        for (int u = 0; u < G; ++u) tile_s[u][w][cs][rl] = b[g + u];
-        lds_barrier();
-#pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int k = (tseg * CPW + g + u) * WAVE + trow;
-            if (tok && k < n) q[pidx(ti, k + 1, ii)] = tile_s[u][tseg][tc][trow];
-        }
-        lds_barrier();
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // restriction qc = P^T q (src/2d/ftn/BMG2_SymStd_restrict.f90:76-92); coarse (ic, jc) sits on
 // fine (2ic-1, 2jc-1)
 // ------------------------------------------------------------------------------------------
-// coarse point (ic, jc) of qc = P^T q (the reference's operation order); ci, q, qc of one problem
-template <typename T>
-__device__ inline T restrict_point(const T *__restrict__ ci, const T *__restrict__ q, int iif,
-                                   int iic, std::size_t Pc, int ic, int jc) {
-    const int i = 2 * ic - 1, j = 2 * jc - 1;
-    auto CI = [&](int a, int b, int k) { return ci[Pc * k + pidx(a, b, iic)]; };
-    auto Q = [&](int a, int b) { return q[pidx(a, b, iif)]; };
-    T v = CI(ic, jc, LNE) * Q(i - 1, j - 1);
-    v = v + CI(ic, jc, LA) * Q(i, j - 1);
-    v = v + CI(ic + 1, jc, LNW) * Q(i + 1, j - 1);
-    v = v + CI(ic, jc, LR) * Q(i - 1, j);
-    v = v + Q(i, j);
-    v = v + CI(ic + 1, jc, LL) * Q(i + 1, j);
-    v = v + CI(ic, jc + 1, LSE) * Q(i - 1, j + 1);
-    v = v + CI(ic, jc + 1, LB) * Q(i, j + 1);
-    v = v + CI(ic + 1, jc + 1, LSW) * Q(i + 1, j + 1);
-    return v;
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void restrict_k(const T *__restrict__ ci, const T *__restrict__ q,
                                                   T *__restrict__ qc, int iif, int jjf, int iic,
@@ -1102,110 +408,6 @@ __global__ __launch_bounds__(64 * rc_rows<T>) void restrict_cycle_k(const T *__r
 // fine ghost column / row (coarse index IICF1 = IIC); those points are updated the same way,
 // with the raw res value there since the reference divides res only in the interior.
 // ------------------------------------------------------------------------------------------
-// One 2 x 2 block of fine points (2m-1 .. 2m, 2n-1 .. 2n) of interp_add: the coarse point
-// (m, n), the x-edge point (2m, 2n-1), the y-edge point (2m-1, 2n) and the cell point (2m, 2n),
-// sharing the four coarse values around the cell.  Arrays of one problem.
-// Two adjacent floats moved by one 8-byte access.  On this GPU an 8-byte global access needs only
-// 4-byte alignment, so a pair may start at any float (rows of odd length included).
-struct __attribute__((aligned(4))) float_pair {
-    float a, b;
-};
-__device__ inline void load_pair(const float *p, float &a, float &b) {
-    float_pair v;
-    __builtin_memcpy(&v, p, sizeof(v));
-    a = v.a;
-    b = v.b;
-}
-__device__ inline void store_pair(float *p, float a, float b) {
-    const float_pair v{a, b};
-    __builtin_memcpy(p, &v, sizeof(v));
-}
-
-template <typename T>
-__device__ inline void interp_block(T *__restrict__ q, const T *__restrict__ qc,
-                                    const T *__restrict__ res, const T *__restrict__ so,
-                                    const T *__restrict__ ci, int iic, int jjc, int iif, int jjf,
-                                    int m, int n) {
-    const int imax = iif - 2 + ((iif - 2) % 2 == 0 ? 1 : 0);
-    const int jmax = jjf - 2 + ((jjf - 2) % 2 == 0 ? 1 : 0);
-    const int i0 = 2 * m - 1, j0 = 2 * n - 1;
-    if (i0 > imax || j0 > jmax) return;
-    const bool xe = i0 + 1 <= imax, ye = j0 + 1 <= jmax;  // the even fine points exist
-    const std::size_t Pc = (std::size_t)iic * jjc;
-    auto CI = [&](int a, int b, int k) { return ci[Pc * k + pidx(a, b, iic)]; };
-    auto QC = [&](int a, int b) { return qc[pidx(a, b, iic)]; };
-    auto R = [&](int i, int j, std::size_t p) {
-        return (i > iif - 2 || j > jjf - 2) ? res[p] : res[p] / so[p];
-    };
-    if constexpr (sizeof(T) == 4) {
-        // FP32: the same operations, with horizontally adjacent values moved as pairs where the
-        // point (2m, .) exists (xe): then i0 + 1 <= iif - 1 and m + 1 <= iic - 1, so every pair
-        // lies inside its row (for even sizes i0 can be the ghost column, where xe is false)
-        const std::size_t p = pidx(i0, j0, iif);
-        T c00, c10 = T(0), c01 = T(0), c11 = T(0);
-        if (xe) {
-            load_pair(qc + pidx(m, n, iic), c00, c10);
-            if (ye) load_pair(qc + pidx(m, n + 1, iic), c01, c11);
-        } else {
-            c00 = QC(m, n);
-            if (ye) c01 = QC(m, n + 1);
-        }
-        if (xe) {  // coarse point and (2m, 2n-1)
-            T q0, q1;
-            load_pair(q + p, q0, q1);
-            q0 = q0 + c00;
-            const T a = CI(m + 1, n, LR) * c10 + CI(m + 1, n, LL) * c00;
-            q1 = q1 + a + R(i0 + 1, j0, p + 1);
-            store_pair(q + p, q0, q1);
-        } else {
-            q[p] = q[p] + c00;
-        }
-        if (ye) {  // (2m-1, 2n) and (2m, 2n)
-            const std::size_t p2 = p + iif;
-            const T a = CI(m, n + 1, LA) * c01 + CI(m, n + 1, LB) * c00;
-            if (xe) {
-                T q2, q3, r2, r3, s2, s3;
-                load_pair(q + p2, q2, q3);
-                load_pair(res + p2, r2, r3);
-                load_pair(so + p2, s2, s3);
-                q2 = q2 + a + ((i0 > iif - 2 || j0 + 1 > jjf - 2) ? r2 : r2 / s2);
-                T b = CI(m + 1, n + 1, LSW) * c00;
-                b = b + CI(m + 1, n + 1, LNW) * c01;
-                b = b + CI(m + 1, n + 1, LNE) * c11;
-                b = b + CI(m + 1, n + 1, LSE) * c10;
-                q3 = q3 + b + ((i0 + 1 > iif - 2 || j0 + 1 > jjf - 2) ? r3 : r3 / s3);
-                store_pair(q + p2, q2, q3);
-            } else {
-                q[p2] = q[p2] + a + R(i0, j0 + 1, p2);
-            }
-        }
-        return;
-    }
-    const T q00 = QC(m, n);
-    {  // coarse point
-        const std::size_t p = pidx(i0, j0, iif);
-        q[p] = q[p] + q00;
-    }
-    if (xe) {  // (2m, 2n-1): between coarse (m, n) and (m+1, n)
-        const std::size_t p = pidx(i0 + 1, j0, iif);
-        const T a = CI(m + 1, n, LR) * QC(m + 1, n) + CI(m + 1, n, LL) * q00;
-        q[p] = q[p] + a + R(i0 + 1, j0, p);
-    }
-    if (ye) {  // (2m-1, 2n): between coarse (m, n) and (m, n+1)
-        const std::size_t p = pidx(i0, j0 + 1, iif);
-        const T a = CI(m, n + 1, LA) * QC(m, n + 1) + CI(m, n + 1, LB) * q00;
-        q[p] = q[p] + a + R(i0, j0 + 1, p);
-    }
-    if (xe && ye) {  // (2m, 2n): the cell of coarse (m..m+1, n..n+1)
-        const std::size_t p = pidx(i0 + 1, j0 + 1, iif);
-        T a = CI(m + 1, n + 1, LSW) * q00;
-        a = a + CI(m + 1, n + 1, LNW) * QC(m, n + 1);
-        a = a + CI(m + 1, n + 1, LNE) * QC(m + 1, n + 1);
-        a = a + CI(m + 1, n + 1, LSE) * QC(m + 1, n);
-        q[p] = q[p] + a + R(i0 + 1, j0 + 1, p);
-    }
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void interp_add_k(T *__restrict__ q, const T *__restrict__ qc,
                                                     const T *__restrict__ res,
@@ -1450,35 +652,6 @@ __global__ __launch_bounds__(256) void setup_cg_k(const double *__restrict__ so,
     __shared__ int bad;
     band_factor_upper(abd, n, kd, ld, bad);
     if (threadIdx.x == 0 && bad) atomicMax(info, bad);
-}
-
-// The coarsest level's band solve: one thread runs the two triangular solves, each step of which
-// reads what the previous one wrote.  Where the factor (ld * n) and the iterate (n) fit in
-// CG_LDS doubles, the workgroup first stages both into LDS, so that those steps wait on LDS and
-// not on global-memory round trips (4x4 coarsest grid of the 4095^2 hierarchy: 25 us per solve
-// through memory); otherwise the iterate lives in the global scratch x.  Same operations either
-// way.  tid / nt: this thread and the workgroup's thread count; sh: the LDS staging area.
-constexpr int CG_LDS = 1024;
-template <typename T>
-__device__ inline void coarse_band_solve(T *q, const T *qf, const double *abd, double *x, int ii,
-                                         int jj, int tid, int nt, double *sh) {
-    const int nx = ii - 2, ny = jj - 2, n = nx * ny, kd = ii - 1, ld = ii;
-    const bool lds = (std::size_t)n * (ld + 1) <= (std::size_t)CG_LDS;
-    double *xx = lds ? sh : x;
-    const double *ab = abd;
-    if (lds) {
-        for (int k = tid; k < ld * n; k += nt) sh[n + k] = abd[k];
-        ab = sh + n;
-    }
-    for (int kk = tid; kk < n; kk += nt) xx[kk] = (double)qf[pidx(kk % nx + 1, kk / nx + 1, ii)];
-    __syncthreads();
-    if (lds && kd < WAVE && nt >= WAVE) {  // bitwise the same sweeps, one wavefront
-        if (tid < WAVE) band_solve_upper_wave(ab, n, kd, ld, xx, tid);
-    } else if (tid == 0) {
-        band_solve_upper(ab, n, kd, ld, xx);
-    }
-    __syncthreads();
-    for (int kk = tid; kk < n; kk += nt) q[pidx(kk % nx + 1, kk / nx + 1, ii)] = (T)xx[kk];
 }
 
 template <typename T>
@@ -2013,864 +1186,11 @@ void transpose(const T *src, T *dst, int rows, int cols, hipStream_t s, int nb) 
     }
 }
 
-// ---- fused coarse-level V-cycle ---------------------------------------------------------------
-// One workgroup per problem runs the whole V-cycle below a level of at most 64*CH points per side
-// (smoothing, residual, restriction, coarsest band solve, interpolation) with workgroup barriers
-// between the steps instead of one launch per step.  Every point is computed by the same device
-// functions and in the same order as in the grid kernels, so the result is bitwise that of the
-// unfused cycle.  Levels of a fused cycle are always 9-point (Galerkin operators).
-
-// one x-line (row j) or y-line (column i) of at most 64*CH points, by one wavefront, in place
-template <typename T, int DIR, int CH>
-__device__ inline void wave_line(const T *__restrict__ so, const T *__restrict__ qf, T *q,
-                                 const T *__restrict__ sor, int ii, int jj, int fixed) {
-    const int lane = threadIdx.x % WAVE, rl = WAVE - 1 - lane;
-    const std::size_t P = (std::size_t)ii * jj;
-    const int n = DIR == 0 ? ii - 2 : jj - 2;
-    const std::size_t f0 = DIR == 0 ? (std::size_t)fixed * ii : (std::size_t)fixed * jj;
-    const T *D = sor + f0 + 1;
-    const T *E = sor + P + f0 + 2;
-    auto at = [&](int k) { return DIR == 0 ? pidx(k + 1, fixed, ii) : pidx(fixed, k + 1, ii); };
-    T a[CH], b[CH];
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-        const int k = u * WAVE + lane, kc = min(k, n - 1);
-        line_raw<T> r;
-        line_load<T, true, DIR>(r, so, qf, q, P, ii, at(kc));
-        b[u] = line_rhs<T, true>(r);
-        a[u] = (k > 0) ? -E[max(kc - 1, 0)] : T(0);
-    }
-#pragma unroll
-    for (int u = 0; u < CH; ++u) scan_affine_dpp(a[u], b[u]);
-    T carry = T(0);
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-        const T y = affine(a[u], carry, b[u]);
-        carry = last_lane(y);
-        b[u] = div_pivot(y, D[min(u * WAVE + lane, n - 1)]);
-    }
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-        const int k = u * WAVE + rl;
-        const T c = __shfl(b[u], rl, WAVE);
-        const T e = E[min(k, max(n - 2, 0))];
-        a[u] = (k < n - 1) ? -e : T(0);
-        a[u] = (k < n) ? a[u] : T(1);
-        b[u] = (k < n) ? c : T(0);
-    }
-#pragma unroll
-    for (int u = 0; u < CH; ++u) scan_affine_dpp(a[u], b[u]);
-    carry = T(0);
-#pragma unroll
-    for (int u = CH - 1; u >= 0; --u) {
-        const T x = affine(a[u], carry, b[u]);
-        carry = last_lane(x);
-        b[u] = x;
-    }
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-        const int k = u * WAVE + rl;
-        if (k < n) q[at(k)] = b[u];
-    }
-}
-
-// LDS bytes the fused cycle needs to hold the arrays of one level on chip (per level: the
-// operator, both relaxation factors, x, b, res and, below the first level, the interpolation),
-// each array rounded up to 16 bytes.  first_mode (the first level of lds_mode 2 or 3): x, b
-// and res (2) or x alone (3).
-template <typename T>
-__host__ __device__ inline std::size_t fused_level_bytes(int ii, int jj, bool has_ci,
-                                                        int first_mode = 1) {
-    const std::size_t plane = ((std::size_t)ii * jj * sizeof(T) + 15) / 16 * 16;
-    if (first_mode == 2) return 3 * plane;
-    if (first_mode == 3) return plane;
-    return plane * (5 + 2 + 2 + 3 + (has_ci ? 8 : 0));
-}
-
-template <typename T, int CH>
-__global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__restrict__ lv,
-                                                       int nlev, int relax, int npre, int npost,
-                                                       const double *__restrict__ abd,
-                                                       double *__restrict__ bbd, int rep,
-                                                       int lds_mode) {
-    constexpr int NT = 1024, NWAVE = NT / WAVE;
-    extern __shared__ __align__(16) unsigned char lds[];
-    const int tid = threadIdx.x, wave = tid / WAVE;
-    const std::size_t bz = blockIdx.x, bo = bz / rep;
-    auto level_global = [&](int l) {  // the level's arrays of problem bz (operator bo)
-        coarse_level<T> d = lv[l];
-        const std::size_t P = (std::size_t)d.ii * d.jj;
-        d.so += bo * 5 * P;
-        d.x += bz * P;
-        d.b += bz * P;
-        d.res += bz * P;
-        d.sor0 += bo * 2 * P;
-        d.sor1 += bo * 2 * P;
-        if (d.ci) d.ci += bo * 8 * P;
-        return d;
-    };
-    // lds_mode 1: every array of every level lives in LDS for the whole cycle (the launcher
-    // checked that they fit); the first level's b comes in from memory and its x goes back at the
-    // end, the only values the caller exchanges with the fused levels.  For a first level too
-    // large to hold whole, lds_mode 2 keeps only its x, b and res in LDS and lds_mode 3 its x
-    // alone; its other arrays stay in memory, where the sweeps only read them, so that a sweep no
-    // longer waits on memory for the previous sweep's writes.
-    const bool on_chip = lds_mode != 0;
-    const int m0 = lds_mode >= 2 ? lds_mode : 1;  // fused_level_bytes mode of the first level
-    auto level_lds = [&](int l) {
-        std::size_t off = 0;
-        for (int m = 0; m < l; ++m)
-            off += fused_level_bytes<T>(lv[m].ii, lv[m].jj, m > 0, m == 0 ? m0 : 1);
-        coarse_level<T> d = lv[l];
-        const std::size_t plane = ((std::size_t)d.ii * d.jj * sizeof(T) + 15) / 16 * 16;
-        unsigned char *base = lds + off;
-        if (l == 0 && m0 >= 2) {
-            d = level_global(0);
-            d.x = reinterpret_cast<T *>(base);
-            if (m0 == 2) {
-                d.b = reinterpret_cast<T *>(base + plane);
-                d.res = reinterpret_cast<T *>(base + 2 * plane);
-            }
-            return d;
-        }
-        d.so = reinterpret_cast<T *>(base);
-        d.sor0 = reinterpret_cast<T *>(base + 5 * plane);
-        d.sor1 = reinterpret_cast<T *>(base + 7 * plane);
-        d.x = reinterpret_cast<T *>(base + 9 * plane);
-        d.b = reinterpret_cast<T *>(base + 10 * plane);
-        d.res = reinterpret_cast<T *>(base + 11 * plane);
-        d.ci = l > 0 ? reinterpret_cast<T *>(base + 12 * plane) : nullptr;
-        return d;
-    };
-    auto level = [&](int l) { return on_chip ? level_lds(l) : level_global(l); };
-    if (on_chip) {
-        for (int l = 0; l < nlev; ++l) {
-            const coarse_level<T> g = level_global(l), d = level_lds(l);
-            const std::size_t P = (std::size_t)g.ii * g.jj;
-            if (l == 0 && m0 == 3) {  // the first level's x alone
-                for (std::size_t k = tid; k < P; k += NT) d.x[k] = g.x[k];
-                continue;
-            }
-            if (!(l == 0 && m0 == 2)) {
-                for (std::size_t k = tid; k < 5 * P; k += NT) const_cast<T *>(d.so)[k] = g.so[k];
-                for (std::size_t k = tid; k < 2 * P; k += NT) {
-                    const_cast<T *>(d.sor0)[k] = g.sor0[k];
-                    const_cast<T *>(d.sor1)[k] = g.sor1[k];
-                }
-                if (l > 0)
-                    for (std::size_t k = tid; k < 8 * P; k += NT)
-                        const_cast<T *>(d.ci)[k] = g.ci[k];
-            }
-            // res and, below the first level, b start at zero as in memory: their ghosts are
-            // never written, and interp_add adds the ghost res of an even-sized level to the
-            // ghost of x
-            for (std::size_t k = tid; k < P; k += NT) {
-                d.res[k] = T(0);
-                d.b[k] = l == 0 ? g.b[k] : T(0);
-                if (l == 0) d.x[k] = g.x[k];
-            }
-        }
-        __syncthreads();
-    }
-    auto lines = [&](const coarse_level<T> &d, const T *sor, int dir, int updown) {
-        const int nfix = dir == 0 ? d.jj - 2 : d.ii - 2;
-        for (int t = 0; t < 2; ++t) {
-            const int first = (updown == 0) ? (t == 0 ? 2 : 1) : (t == 0 ? 1 : 2);
-            if (first <= nfix) {
-                const int nlines = (nfix - first) / 2 + 1;
-                for (int line = wave; line < nlines; line += NWAVE) {
-                    if (dir == 0)
-                        wave_line<T, 0, CH>(d.so, d.b, d.x, sor, d.ii, d.jj, first + 2 * line);
-                    else
-                        wave_line<T, 1, CH>(d.so, d.b, d.x, sor, d.ii, d.jj, first + 2 * line);
-                }
-            }
-            __syncthreads();
-        }
-    };
-    auto gauss_seidel = [&](const coarse_level<T> &d, int updown) {
-        static constexpr int order[4][2] = {{1, 1}, {0, 1}, {1, 0}, {0, 0}};
-        const std::size_t P = (std::size_t)d.ii * d.jj;
-        const int nx = d.ii - 2, npts = nx * (d.jj - 2);
-        for (int t = 0; t < 4; ++t) {
-            const int c = updown == 0 ? t : 3 - t;
-            for (int k = tid; k < npts; k += NT) {
-                const int i = k % nx + 1, j = k / nx + 1;
-                if ((i & 1) != order[c][0] || (j & 1) != order[c][1]) continue;
-                const std::size_t p = pidx(i, j, d.ii);
-                const T v = apply_offdiag<T, true>(d.so, P, d.x, p, d.ii, d.b[p]);
-                d.x[p] = v * d.sor0[P + p];
-            }
-            __syncthreads();
-        }
-    };
-    auto smooth = [&](const coarse_level<T> &d, int updown) {
-        const int nrep = updown == 0 ? npre : npost;
-        for (int r = 0; r < nrep; ++r) {
-            if (relax == CDR_RELAX_POINT) {
-                gauss_seidel(d, updown);
-            } else if (relax == CDR_RELAX_LINE_X) {
-                lines(d, d.sor0, 0, updown);
-            } else if (relax == CDR_RELAX_LINE_Y) {
-                lines(d, d.sor0, 1, updown);
-            } else if (updown == 0) {
-                lines(d, d.sor0, 0, updown);
-                lines(d, d.sor1, 1, updown);
-            } else {
-                lines(d, d.sor1, 1, updown);
-                lines(d, d.sor0, 0, updown);
-            }
-        }
-    };
-    // down: smooth, residual, restrict to the next level's b, zero its x
-    for (int l = 0; l + 1 < nlev; ++l) {
-        const coarse_level<T> F = level(l), C = level(l + 1);
-        smooth(F, 0);
-        const std::size_t P = (std::size_t)F.ii * F.jj;
-        const int nx = F.ii - 2, npts = nx * (F.jj - 2);
-        for (int k = tid; k < npts; k += NT) {
-            const std::size_t p = pidx(k % nx + 1, k / nx + 1, F.ii);
-            T r = apply_offdiag<T, true>(F.so, P, F.x, p, F.ii, F.b[p]);
-            r = r - F.so[p] * F.x[p];
-            F.res[p] = r;
-        }
-        __syncthreads();
-        const std::size_t Pc = (std::size_t)C.ii * C.jj;
-        const int nxc = C.ii - 2, nc = nxc * (C.jj - 2);
-        for (int k = tid; k < nc; k += NT) {
-            const int ic = k % nxc + 1, jc = k / nxc + 1;
-            C.b[pidx(ic, jc, C.ii)] = restrict_point<T>(C.ci, F.res, F.ii, C.ii, Pc, ic, jc);
-        }
-        for (std::size_t k = tid; k < Pc; k += NT) C.x[k] = T(0);
-        __syncthreads();
-    }
-    // coarsest level: band Cholesky solve (as solve_cg_k)
-    {
-        __shared__ double cg_sh[CG_LDS];
-        const coarse_level<T> C = level(nlev - 1);
-        const int n = (C.ii - 2) * (C.jj - 2);
-        coarse_band_solve<T>(C.x, C.b, abd + bo * (std::size_t)C.ii * n, bbd + bz * n, C.ii, C.jj,
-                             tid, NT, cg_sh);
-        __syncthreads();
-    }
-    // up: interpolate and add, smooth
-    for (int l = nlev - 2; l >= 0; --l) {
-        const coarse_level<T> F = level(l), C = level(l + 1);
-        const int mb = F.ii / 2, nblk = mb * (F.jj / 2);
-        for (int k = tid; k < nblk; k += NT)
-            interp_block<T>(F.x, C.x, F.res, F.so, C.ci, C.ii, C.jj, F.ii, F.jj, k % mb + 1,
-                            k / mb + 1);
-        __syncthreads();
-        smooth(F, 1);
-    }
-    if (on_chip) {  // the smoothing ends with a workgroup barrier
-        const coarse_level<T> g = level_global(0), d = level_lds(0);
-        const std::size_t P = (std::size_t)g.ii * g.jj;
-        for (std::size_t k = tid; k < P; k += NT) g.x[k] = d.x[k];
-    }
-}
-
-// ---- line kernel shapes and their autotuner ---------------------------------------------------
-// A shape is (CPW, W, L) for x-lines (chunks per wavefront, wavefronts per line, lines per
-// workgroup) and (CPW, W, NC, G) for y-lines (..., columns per workgroup, chunk rows per LDS
-// round).  All shapes of a chunk class give bitwise identical results (see the segmented
-// kernels), so the shape of each (precision, stencil, direction, extents, batch) is picked by
-// timing: tune_lines() times every candidate once on the caller's data and records the fastest in
-// a process-wide table that the launchers consult; without an entry, candidate 0 runs.
-
-template <typename T, bool NINE, int CPW, int W, int L, bool TR>
-static void launch_x(const T *so, const T *qf, T *q, const T *sor, int ii, int jj, int first,
-                     int nlines, hipStream_t s, int nb, int rev, int rep) {
-    const int ntiles = (nlines + L - 1) / L;
-    const dim3 blocks((unsigned)(8 * ((ntiles + 7) / 8)), (unsigned)nb);
-    // rev bit 1: zero start (x-lines of the grid itself only)
-    if (!TR && (rev & 2))
-        relax_xlines_seg_k<T, NINE, CPW, W, L, TR, !TR><<<blocks, L * W * 64, 0, s>>>(
-            so, qf, q, sor, ii, jj, first, nlines, ntiles, rev & 1, rep);
-    else
-        relax_xlines_seg_k<T, NINE, CPW, W, L, TR, false><<<blocks, L * W * 64, 0, s>>>(
-            so, qf, q, sor, ii, jj, first, nlines, ntiles, rev & 1, rep);
-}
-
-template <typename T, bool NINE, int CPW, int W, int NC, int G>
-static void launch_y(const T *so, const T *qf, T *q, const T *sor, int ii, int jj, int first,
-                     int nlines, hipStream_t s, int nb, int rev, int rep) {
-    const int ntiles = (nlines + NC - 1) / NC;
-    const dim3 blocks((unsigned)(8 * ((ntiles + 7) / 8)), (unsigned)nb);
-    relax_ylines_seg_k<T, NINE, CPW, W, NC, G><<<blocks, NC * W * 64, 0, s>>>(
-        so, qf, q, sor, ii, jj, first, nlines, ntiles, rev, rep);
-}
-
-// Launches candidate c of chunk class NCH (lines of at most 64*NCH points); returns the number
-// of candidates of the class (c outside [0, count) launches nothing).
-static std::string shape_text(const char *k, int cpw, int w, const char *tn, int t, int g) {
-    char buf[96];
-    if (g > 0)
-        std::snprintf(buf, sizeof(buf), "%s<CPW=%d,W=%d,%s=%d,G=%d>", k, cpw, w, tn, t, g);
-    else
-        std::snprintf(buf, sizeof(buf), "%s<CPW=%d,W=%d,%s=%d>", k, cpw, w, tn, t);
-    return buf;
-}
-
-// With `name` non-null nothing is launched and *name receives candidate c's description.
-// DIR 0: x-lines, 1: y-lines, 2: x-lines of a transposed y-line problem.
-template <typename T, bool NINE, int DIR, int NCH>
-static int launch_shape(int c, const T *so, const T *qf, T *q, const T *sor, int ii, int jj,
-                        int first, int nlines, hipStream_t s, int nb, std::string *name = nullptr,
-                        int rev = 0, int rep = 1) {
-    constexpr bool TR = DIR == 2;
-    constexpr bool F64 = sizeof(T) == 8;
-#define CDR_X(k, C, W, L)                                                                       \
-    if (c == k) {                                                                               \
-        if (name)                                                                               \
-            *name = shape_text("relax_xlines_seg_k", C, W, "L", L, 0);                          \
-        else                                                                                    \
-            launch_x<T, NINE, C, W, L, TR>(so, qf, q, sor, ii, jj, first, nlines, s, nb, rev,   \
-                                           rep);                                                \
-    }
-#define CDR_Y(k, C, W, NC, G)                                                                   \
-    if (c == k) {                                                                               \
-        if (name)                                                                               \
-            *name = shape_text("relax_ylines_seg_k", C, W, "NC", NC, G);                        \
-        else                                                                                    \
-            launch_y<T, NINE, C, W, NC, G>(so, qf, q, sor, ii, jj, first, nlines, s, nb, rev,   \
-                                           rep);                                                \
-    }
-    // x: (CPW, W, L); y: (CPW, W, NC, G).  At most 16 wavefronts per workgroup.
-    if constexpr (DIR != 1) {
-        if constexpr (NCH <= 2) {
-            CDR_X(0, NCH, 1, 4);
-            return 1;
-        } else if constexpr (NCH == 4) {
-            CDR_X(0, 4, 1, 4);
-            CDR_X(1, 1, 4, 1);
-            return 2;
-        } else if constexpr (NCH == 8) {
-            CDR_X(0, 8, 1, 4);
-            CDR_X(1, 4, 2, 2);
-            CDR_X(2, 2, 4, 1);
-            CDR_X(3, 1, 8, 1);  // one chunk per wavefront: the shortest chain per line
-            return 4;
-        } else if constexpr (NCH == 16) {
-            CDR_X(0, 16, 1, 4);
-            CDR_X(1, 8, 2, 2);
-            CDR_X(2, 4, 4, 1);
-            CDR_X(3, 2, 8, 1);
-            CDR_X(4, 1, 16, 1);
-            return 5;
-        } else if constexpr (NCH == 32) {
-            CDR_X(0, 16, 2, 2);
-            CDR_X(1, 8, 4, 1);
-            CDR_X(2, 4, 8, 1);
-            CDR_X(3, F64 ? 2 : 32, F64 ? 16 : 1, F64 ? 1 : 4);
-            // two neighbouring lines of a colour per workgroup share the row of q between them
-            CDR_X(4, 8, 4, 2);
-            CDR_X(5, 4, 8, 2);
-            return 6;
-        } else if constexpr (NCH == 3) {  // classes of 2^k + 1 chunks: W * CPW >= NCH
-            CDR_X(0, 3, 1, 4);
-            CDR_X(1, 1, 3, 2);
-            return 2;
-        } else if constexpr (NCH == 5) {
-            CDR_X(0, 5, 1, 4);
-            CDR_X(1, 3, 2, 2);
-            CDR_X(2, 1, 5, 2);
-            return 3;
-        } else if constexpr (NCH == 9) {
-            CDR_X(0, 9, 1, 4);
-            CDR_X(1, 5, 2, 2);
-            CDR_X(2, 3, 3, 2);
-            CDR_X(3, 1, 9, 1);
-            return 4;
-        } else if constexpr (NCH == 17) {
-            CDR_X(0, 17, 1, 4);
-            CDR_X(1, 9, 2, 2);
-            CDR_X(2, 6, 3, 1);
-            CDR_X(3, 6, 3, 2);
-            CDR_X(4, 3, 6, 1);
-            return 5;
-        } else if constexpr (NCH == 33) {
-            CDR_X(0, 11, 3, 1);
-            CDR_X(1, 11, 3, 2);
-            CDR_X(2, 6, 6, 1);
-            CDR_X(3, 3, 11, 1);
-            CDR_X(4, 17, 2, 2);
-            return 5;
-        } else {
-            CDR_X(0, 16, 4, 1);
-            CDR_X(1, 8, 8, 1);
-            CDR_X(2, 4, 16, 1);
-            CDR_X(3, 64, 1, 4);
-            CDR_X(4, 8, 8, 2);
-            CDR_X(5, 16, 4, 2);
-            return 6;
-        }
-    } else {
-        // columns per workgroup for 64-byte (N1) and 128-byte (2 N1) row segments
-        constexpr int N1 = F64 ? 4 : 8;
-        // small levels: fewer columns per workgroup put more workgroups on the GPU (their rows
-        // come from the caches at these sizes)
-        if constexpr (NCH <= 2) {
-            CDR_Y(0, NCH, 1, N1, NCH);
-            CDR_Y(1, NCH, 1, 2 * N1, NCH);
-            CDR_Y(2, NCH, 1, N1 / 4, NCH);
-            return 3;
-        } else if constexpr (NCH == 4) {
-            CDR_Y(0, 4, 1, N1, 4);
-            CDR_Y(1, 4, 1, 2 * N1, 2);
-            CDR_Y(2, 1, 4, N1 / 2, 1);
-            CDR_Y(3, 4, 1, N1 / 4, 4);
-            CDR_Y(4, 2, 2, N1 / 4, 2);
-            // FP32: one column per workgroup as well (FP64 has it as N1 / 4): the levels of a few
-            // hundred columns are latency-bound, where more, smaller workgroups fill more CUs
-            if constexpr (!F64) {
-                CDR_Y(5, 2, 2, 1, 2);
-                CDR_Y(6, 1, 4, 1, 1);
-                return 7;
-            }
-            return 5;
-        } else if constexpr (NCH == 8) {
-            CDR_Y(0, 8, 1, N1, 4);
-            CDR_Y(1, 8, 1, 2 * N1, 2);
-            CDR_Y(2, 4, 2, N1, 4);
-            CDR_Y(3, 2, 4, N1 / 2, 2);
-            CDR_Y(4, 8, 1, N1 / 4, 4);
-            CDR_Y(5, 4, 2, N1 / 4, 4);
-            if constexpr (!F64) {
-                CDR_Y(6, 4, 2, 1, 4);
-                CDR_Y(7, 2, 4, 1, 2);
-                return 8;
-            }
-            return 6;
-        } else if constexpr (NCH == 16) {
-            CDR_Y(0, 16, 1, N1, 4);
-            CDR_Y(1, 8, 2, N1, 4);
-            CDR_Y(2, 16, 1, 2 * N1, 2);
-            CDR_Y(3, 4, 4, N1 / 2, 4);
-            if constexpr (!F64) {
-                CDR_Y(4, 4, 4, 1, 4);
-                CDR_Y(5, 8, 2, 1, 4);
-                return 6;
-            }
-            return 4;
-        } else if constexpr (NCH == 32) {
-            CDR_Y(0, 16, 2, N1, 2);
-            CDR_Y(1, 32, 1, N1, 4);
-            CDR_Y(2, 8, 4, N1 / 2, 2);
-            CDR_Y(3, 4, 8, N1 / 4, 4);
-            return 4;
-        } else {  // 16-wavefront workgroups get 128 VGPRs: narrower tiles for long segments
-            CDR_Y(0, 64, 1, N1, 2);
-            CDR_Y(1, 16, 4, N1 / 2, 2);
-            CDR_Y(2, 32, 2, N1 / 2, 2);
-            CDR_Y(3, 64, 1, 2 * N1, 2);
-            return 4;
-        }
-    }
-#undef CDR_X
-#undef CDR_Y
-}
-
-// chunk class of a line of n points: 1, 2, 4, ..., 64, or 0 beyond 4096 points.  With odd set
-// (x-line shapes), lines of 3, 5, 9, 17 or 33 chunks get a class of their own: the lines of the
-// 2^k + 1 grids (129 ... 2049 points) would otherwise leave almost half of the lanes of a
-// power-of-two class idle.
-static int chunk_class(int n, bool odd) {
-    const int nch = (n + WAVE - 1) / WAVE;
-    if (odd && (nch == 3 || nch == 5 || nch == 9 || nch == 17 || nch == 33)) return nch;
-    int c = 1;
-    while (c < nch && c < 64) c *= 2;
-    return nch > 64 ? 0 : c;
-}
-
-template <typename T, bool NINE, int DIR>
-static int launch_class(int c, const T *so, const T *qf, T *q, const T *sor, int ii, int jj,
-                        int first, int nlines, hipStream_t s, int nb, std::string *name = nullptr,
-                        int rev = 0, int rep = 1) {
-    const int n = (DIR != 1) ? ii - 2 : jj - 2;
-#define CDR_C(K)                                                                                  \
-    case K:                                                                                       \
-        return launch_shape<T, NINE, DIR, K>(c, so, qf, q, sor, ii, jj, first, nlines, s, nb, name, \
-                                             rev, rep)
-#define CDR_O(K)                                                                                  \
-    case K:                                                                                       \
-        if constexpr (DIR != 1)                                                                   \
-            return launch_shape<T, NINE, DIR, K>(c, so, qf, q, sor, ii, jj, first, nlines, s, nb,  \
-                                                 name, rev, rep);                                 \
-        else                                                                                      \
-            return 0;  /* not reached: y-lines use the power-of-two classes */
-    switch (chunk_class(n, DIR != 1)) {
-        CDR_C(1);
-        CDR_C(2);
-        CDR_O(3);
-        CDR_C(4);
-        CDR_O(5);
-        CDR_C(8);
-        CDR_O(9);
-        CDR_C(16);
-        CDR_O(17);
-        CDR_C(32);
-        CDR_O(33);
-        CDR_C(64);
-    default:  // lines longer than 4096: stage the forward results in q itself
-        if constexpr (DIR == 2) {
-            return 0;  // no transposed path for such lines
-        } else {
-            if (c == 0 && name) *name = "relax_lines_k";
-            if (c == 0 && !name)
-                relax_lines_k<T, NINE, DIR><<<dim3((unsigned)((nlines + 3) / 4), (unsigned)nb), 256,
-                                              0, s>>>(so, qf, q, sor, ii, jj, first, nlines, rep);
-            return 1;
-        }
-    }
-#undef CDR_C
-#undef CDR_O
-}
-
-namespace {
-using tune_key = std::array<int, 6>;  // direction, word size, 9-point, ii, jj, batch
-std::mutex g_tune_mu;
-std::map<tune_key, int> g_tune;
-std::atomic<int> g_autotune{1};
-}  // namespace
-
-template <typename T>
-static tune_key key_of(int dir, int nstncl, int ii, int jj, int nb) {
-    return tune_key{dir, (int)sizeof(T), nstncl == 5 ? 1 : 0, ii, jj, nb};
-}
-
-static int tuned_shape(const tune_key &k) {
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    const auto it = g_tune.find(k);
-    return it == g_tune.end() ? 0 : it->second;
-}
-
-template <typename T, int DIR>
-static int launch_colour(int c, const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii,
-                         int jj, int first, int nlines, hipStream_t s, int nb,
-                         std::string *name = nullptr, int rev = 0, int rep = 1) {
-    if (nstncl == 5)
-        return launch_class<T, true, DIR>(c, so, qf, q, sor, ii, jj, first, nlines, s, nb, name, rev,
-                                          rep);
-    return launch_class<T, false, DIR>(c, so, qf, q, sor, ii, jj, first, nlines, s, nb, name, rev,
-                                       rep);
-}
-
-static std::string shape_name(const std::array<int, 6> &k, int c) {
-    std::string name;
-    const int ns = k[2] ? 5 : 3;
-    // direction 2 (y-lines through the transposed grid): an x-line shape on the swapped extents
-    if (k[0] == 2 && c < 0) return "direct y-lines";
-    const int dir = k[0] == 1 ? 1 : 0;
-    const int ii = k[0] == 2 ? k[4] : k[3], jj = k[0] == 2 ? k[3] : k[4];
-    if (k[1] == 8)
-        (void)(dir == 0 ? launch_colour<double, 0>(c, nullptr, ns, nullptr, nullptr, nullptr, ii,
-                                                   jj, 1, 1, nullptr, 1, &name)
-                        : launch_colour<double, 1>(c, nullptr, ns, nullptr, nullptr, nullptr, ii,
-                                                   jj, 1, 1, nullptr, 1, &name));
-    else
-        (void)(dir == 0 ? launch_colour<float, 0>(c, nullptr, ns, nullptr, nullptr, nullptr, ii,
-                                                  jj, 1, 1, nullptr, 1, &name)
-                        : launch_colour<float, 1>(c, nullptr, ns, nullptr, nullptr, nullptr, ii,
-                                                  jj, 1, 1, nullptr, 1, &name));
-    return k[0] == 2 ? "transposed, " + name : name;
-}
-
-// zq (x-lines of at most 4096 points only): the sweep starts from q = 0 (see relax_xlines_seg_k)
-template <typename T, int DIR>
-static void relax_lines(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj,
-                        int updown, hipStream_t s, int nb, int rep = 1, int zq = 0) {
-    const int c = tuned_shape(key_of<T>(DIR, nstncl, ii, jj, nb));
-    // lines of one colour: DOWN relaxes the lines at even array index (odd Cedar index) first,
-    // UP the odd ones first (src/2d/ftn/BMG2_SymStd_relax_lines_x.f90:82-97)
-    const int nfix = (DIR == 0) ? jj - 2 : ii - 2;
-    for (int t = 0; t < 2; ++t) {
-        const int first = (updown == 0) ? (t == 0 ? 2 : 1) : (t == 0 ? 1 : 2);
-        if (first > nfix) continue;
-        const int nlines = (nfix - first) / 2 + 1;
-        // the second colour walks the lines in the opposite order (see xcd_tile)
-        const int z = (DIR == 0 && zq && t == 0) ? 2 : 0;
-        launch_colour<T, DIR>(c, so, nstncl, qf, q, sor, ii, jj, first, nlines, s, nb, nullptr,
-                              t | z, rep);
-    }
-}
-
-template <typename T>
-void relax_lines_x(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj,
-                   int updown, hipStream_t s, int nb, int rep, int zero_start) {
-    relax_lines<T, 0>(so, nstncl, qf, q, sor, ii, jj, updown, s, nb, rep,
-                      zero_start && chunk_class(ii - 2, true) != 0);
-}
-
-bool lines_zero_start(int ii) { return chunk_class(ii - 2, true) != 0; }
-
-template <typename T>
-void relax_lines_y(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj,
-                   int updown, hipStream_t s, int nb, int rep) {
-    relax_lines<T, 1>(so, nstncl, qf, q, sor, ii, jj, updown, s, nb, rep);
-}
-
-int set_autotune(int on) { return g_autotune.exchange(on ? 1 : 0); }
-bool autotune_enabled() { return g_autotune.load() != 0; }
-
-int line_shape_count(int dir, int wbytes, int nstncl, int ii, int jj) {
-    const hipStream_t s = nullptr;  // counting launches nothing
-    if (dir == 2) {  // x-line shapes of the transposed grid; none for lines over 4096 points
-        if (jj - 2 > 64 * WAVE) return 0;
-        dir = 0;
-        std::swap(ii, jj);
-    }
-    if (wbytes == 8)
-        return dir == 0 ? launch_colour<double, 0>(-1, nullptr, nstncl, nullptr, nullptr, nullptr,
-                                                   ii, jj, 1, 1, s, 1)
-                        : launch_colour<double, 1>(-1, nullptr, nstncl, nullptr, nullptr, nullptr,
-                                                   ii, jj, 1, 1, s, 1);
-    return dir == 0 ? launch_colour<float, 0>(-1, nullptr, nstncl, nullptr, nullptr, nullptr, ii,
-                                              jj, 1, 1, s, 1)
-                    : launch_colour<float, 1>(-1, nullptr, nstncl, nullptr, nullptr, nullptr, ii,
-                                              jj, 1, 1, s, 1);
-}
-
-void set_line_shape(int dir, int wbytes, int nstncl, int ii, int jj, int nb, int shape) {
-    const tune_key k{dir, wbytes, nstncl == 5 ? 1 : 0, ii, jj, nb};
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    if (shape < 0)
-        g_tune.erase(k);
-    else
-        g_tune[k] = shape;
-}
-
-template <typename T>
-int tune_lines(int dir, const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, int jj,
-               hipStream_t s, int nb, int rep) {
-    const tune_key k = key_of<T>(dir, nstncl, ii, jj, nb);
-    {
-        std::lock_guard<std::mutex> g(g_tune_mu);
-        if (g_tune.count(k)) return g_tune[k];
-    }
-    auto run = [&](int c) {
-        return dir == 0 ? launch_colour<T, 0>(c, so, nstncl, qf, q, sor, ii, jj, 1,
-                                              (jj - 2 + 1) / 2, s, nb, nullptr, 0, rep)
-                        : launch_colour<T, 1>(c, so, nstncl, qf, q, sor, ii, jj, 1,
-                                              (ii - 2 + 1) / 2, s, nb, nullptr, 0, rep);
-    };
-    const int ncand = run(-1);  // count only
-    if (!g_autotune.load() || ncand < 2) return 0;
-    int best = 0;
-    {
-        hipEvent_t e0, e1;
-        if (hipEventCreate(&e0) != hipSuccess) return -1;
-        if (hipEventCreate(&e1) != hipSuccess) {
-            (void)hipEventDestroy(e0);
-            return -1;
-        }
-        // two rounds over the candidates, each candidate's time the smaller of its two: shapes
-        // within a few percent of each other were otherwise picked by the noise of one timing
-        std::vector<float> tmin(ncand, -1.f);
-        for (int round = 0; round < 2; ++round)
-            for (int c = 0; c < ncand; ++c) {
-                run(c);  // warm-up
-                (void)hipEventRecord(e0, s);
-                for (int r = 0; r < 3; ++r) run(c);
-                (void)hipEventRecord(e1, s);
-                if (hipEventSynchronize(e1) != hipSuccess) break;
-                float ms = 0.f;
-                (void)hipEventElapsedTime(&ms, e0, e1);
-                if (tmin[c] < 0.f || ms < tmin[c]) tmin[c] = ms;
-            }
-        for (int c = 1; c < ncand; ++c)
-            if (tmin[c] >= 0.f && tmin[c] < tmin[best]) best = c;
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        if (hipGetLastError() != hipSuccess) return -1;
-    }
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    g_tune[k] = best;
-    return best;
-}
-
-// ---- y-lines through the transposed grid ------------------------------------------------------
-// With the operator transposed once at setup (soT: c, w, s, sw, nw of the transposed grid, i.e.
-// the transposes of c, s, w, sw, nw), a y-line sweep is an x-line sweep of the transposed grid:
-// q and f are transposed, both colours are relaxed with the x-line kernel (right-hand side terms in
-// the y-line order, the y-line factors are already stored column-contiguous), and q is transposed
-// back.  The result is bitwise that of relax_lines_y.
-
 template <typename T>
 void transpose_op(const T *so, T *soT, int nstncl, int ii, int jj, hipStream_t s, int nb) {
     // every stencil plane of every problem in one launch (z = problem * nstncl + plane)
     const dim3 g((unsigned)((ii + 63) / 64), (unsigned)((jj + 63) / 64), (unsigned)(nb * nstncl));
     transpose_op_k<T><<<g, 512, 0, s>>>(so, soT, jj, ii, nstncl);
-}
-
-template <typename T>
-static void relax_lines_ytr(const T *soT, int nstncl, const T *qf, T *q, const T *sory, T *qT,
-                            T *qfT, int ii, int jj, int updown, int shape, hipStream_t s, int nb,
-                            bool qfT_ready = false, bool q_in_T = false, bool keep_T = false,
-                            int rep = 1) {
-    if (!q_in_T) transpose<T>(q, qT, jj, ii, s, nb);
-    if (!qfT_ready) transpose<T>(qf, qfT, jj, ii, s, nb);
-    const int nfix = ii - 2;  // columns of the original grid = rows of the transposed one
-    for (int t = 0; t < 2; ++t) {
-        const int first = (updown == 0) ? (t == 0 ? 2 : 1) : (t == 0 ? 1 : 2);
-        if (first > nfix) continue;
-        const int nlines = (nfix - first) / 2 + 1;
-        if (nstncl == 5)
-            launch_class<T, true, 2>(shape, soT, qfT, qT, sory, jj, ii, first, nlines, s, nb,
-                                     nullptr, t, rep);
-        else
-            launch_class<T, false, 2>(shape, soT, qfT, qT, sory, jj, ii, first, nlines, s, nb,
-                                      nullptr, t, rep);
-    }
-    if (!keep_T) transpose<T>(qT, q, ii, jj, s, nb);
-}
-
-static int tuned_transposed(const tune_key &k) {
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    const auto it = g_tune.find(k);
-    return it == g_tune.end() ? -1 : it->second;
-}
-
-template <typename T>
-bool relax_lines_y_auto(const T *so, const T *soT, int nstncl, const T *qf, T *q, const T *sory,
-                        T *qT, T *qfT, int ii, int jj, int updown, hipStream_t s, int nb,
-                        bool qfT_ready, bool q_in_T, bool keep_T, int rep) {
-    const int c = uses_transposed_y<T>(soT, nstncl, ii, jj, nb);
-    if (c < 0) {
-        if (q_in_T) transpose<T>(qT, q, ii, jj, s, nb);
-        relax_lines<T, 1>(so, nstncl, qf, q, sory, ii, jj, updown, s, nb, rep);
-        return false;
-    }
-    relax_lines_ytr<T>(soT, nstncl, qf, q, sory, qT, qfT, ii, jj, updown, c, s, nb, qfT_ready,
-                       q_in_T, keep_T, rep);
-    return true;
-}
-
-template <typename T>
-int uses_transposed_y(const T *soT, int nstncl, int ii, int jj, int nb) {
-    return soT ? tuned_transposed(key_of<T>(2, nstncl, ii, jj, nb)) : -1;
-}
-
-// Milliseconds for 3 replays of what run(cs) launches, captured as a graph on the capture stream
-// cs and replayed on s, the way the solvers execute their cycles (eager back-to-back launches
-// would leave gaps that favour the variant with fewer launches); -1 if capture fails.
-template <typename F>
-static float time_captured(hipStream_t cs, hipStream_t s, hipEvent_t e0, hipEvent_t e1, F &&run) {
-    if (!cs || hipStreamSynchronize(s) != hipSuccess) return -1.f;
-    if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) return -1.f;
-    run(cs);
-    hipGraph_t g = nullptr;
-    if (hipStreamEndCapture(cs, &g) != hipSuccess || !g) {
-        if (g) (void)hipGraphDestroy(g);
-        return -1.f;
-    }
-    hipGraphExec_t ge = nullptr;
-    float ms = -1.f;
-    if (hipGraphInstantiate(&ge, g, nullptr, nullptr, 0) == hipSuccess) {
-        (void)hipGraphLaunch(ge, s);  // warm-up
-        (void)hipEventRecord(e0, s);
-        for (int r = 0; r < 3; ++r) (void)hipGraphLaunch(ge, s);
-        (void)hipEventRecord(e1, s);
-        if (hipEventSynchronize(e1) == hipSuccess) (void)hipEventElapsedTime(&ms, e0, e1);
-        (void)hipGraphExecDestroy(ge);
-    }
-    (void)hipGraphDestroy(g);
-    return ms;
-}
-
-template <typename T>
-int tune_lines_ytr(const T *so, const T *soT, int nstncl, const T *qf, T *q, const T *sory,
-                   T *qT, T *qfT, int ii, int jj, hipStream_t s, int nb, int sweeps, int rep) {
-    sweeps = sweeps < 1 ? 1 : sweeps;
-    const tune_key k = key_of<T>(2, nstncl, ii, jj, nb);
-    {
-        std::lock_guard<std::mutex> g(g_tune_mu);
-        if (g_tune.count(k)) return g_tune[k];
-    }
-    if (!g_autotune.load()) return -1;
-    if (tune_lines<T>(1, so, nstncl, qf, q, sory, ii, jj, s, nb, rep) < 0) return -2;
-    const int ncand = nstncl == 5 ? launch_class<T, true, 2>(-1, soT, qf, q, sory, jj, ii, 1, 1, s, nb)
-                                  : launch_class<T, false, 2>(-1, soT, qf, q, sory, jj, ii, 1, 1, s, nb);
-    hipEvent_t e0, e1;
-    if (hipEventCreate(&e0) != hipSuccess) return -2;
-    if (hipEventCreate(&e1) != hipSuccess) {
-        (void)hipEventDestroy(e0);
-        return -2;
-    }
-    hipStream_t cs = nullptr;
-    if (hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) != hipSuccess) cs = nullptr;
-    auto timed1 = [&](auto &&run) {  // run(stream) launches one timed unit on that stream
-        const float tc = time_captured(cs, s, e0, e1, run);
-        if (tc >= 0.f) return tc;
-        (void)hipGetLastError();  // eager timing when capture is not available
-        run(s);  // warm-up
-        (void)hipEventRecord(e0, s);
-        for (int r = 0; r < 3; ++r) run(s);
-        (void)hipEventRecord(e1, s);
-        float ms = -1.f;
-        if (hipEventSynchronize(e1) == hipSuccess) (void)hipEventElapsedTime(&ms, e0, e1);
-        return ms;
-    };
-    auto timed = [&](auto &&run) {  // the faster of two timings
-        const float a = timed1(run), b = timed1(run);
-        return a < 0.f ? b : (b < 0.f ? a : (b < a ? b : a));
-    };
-    // `sweeps` y sweeps share one right-hand side (one transpose of qf)
-    const float tdirect = timed([&](hipStream_t st) {
-        for (int k = 0; k < sweeps; ++k)
-            relax_lines<T, 1>(so, nstncl, qf, q, sory, ii, jj, 0, st, nb, rep);
-    });
-    int best = -1;
-    float tbest = tdirect;
-    for (int c = 0; c < ncand; ++c) {
-        const float t = timed([&](hipStream_t st) {
-            for (int k = 0; k < sweeps; ++k)
-                relax_lines_ytr<T>(soT, nstncl, qf, q, sory, qT, qfT, ii, jj, 0, c, st, nb, k > 0,
-                                   k > 0, k < sweeps - 1, rep);
-        });
-        if (t >= 0.f && t < tbest) {
-            tbest = t;
-            best = c;
-        }
-    }
-    if (cs) (void)hipStreamDestroy(cs);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (hipGetLastError() != hipSuccess) return -2;
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    g_tune[k] = best;
-    return best;
-}
-
-std::string tune_report() {
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    std::string out = "[";
-    for (const auto &kv : g_tune) {
-        const tune_key &k = kv.first;
-        char buf[160];
-        std::snprintf(buf, sizeof(buf),
-                      "%s{\"dir\":\"%c\",\"fp\":%d,\"stencil\":%d,\"ii\":%d,\"jj\":%d,\"nb\":%d,"
-                      "\"shape\":%d,\"kernel\":\"",
-                      out.size() > 1 ? "," : "", k[0] == 0 ? 'x' : (k[0] == 1 ? 'y' : 't'),
-                      8 * k[1], k[2] ? 9 : 5,
-                      k[3], k[4], k[5], kv.second);
-        out += buf;
-        out += shape_name(k, kv.second) + "\"}";
-    }
-    return out + "]";
-}
-
-template <typename T>
-void relax_lines_xy(const T *so, int nstncl, const T *qf, T *q, const T *sorx, const T *sory,
-                    T *work, int ii, int jj, int updown, hipStream_t s, int nb, int rep) {
-    (void)work;
-    if (updown == 0) {
-        relax_lines<T, 0>(so, nstncl, qf, q, sorx, ii, jj, updown, s, nb, rep);
-        relax_lines<T, 1>(so, nstncl, qf, q, sory, ii, jj, updown, s, nb, rep);
-    } else {
-        relax_lines<T, 1>(so, nstncl, qf, q, sory, ii, jj, updown, s, nb, rep);
-        relax_lines<T, 0>(so, nstncl, qf, q, sorx, ii, jj, updown, s, nb, rep);
-    }
 }
 
 template <typename T>
@@ -2958,37 +1278,6 @@ template <typename T>
 void solve_cg(T *q, const T *qf, const double *abd, double *bbd, int ii, int jj, hipStream_t s,
               int nb, int rep) {
     solve_cg_k<T><<<nb, 64, 0, s>>>(q, qf, abd, bbd, ii, jj, rep);
-}
-
-std::size_t fused_cycle_lds_bytes(int wbytes, const int *ii, const int *jj, int nlev,
-                                  int lds_mode) {
-    std::size_t b = 0;
-    for (int l = 0; l < nlev; ++l) {
-        const int m = l == 0 ? lds_mode : 1;
-        b += wbytes == 8 ? fused_level_bytes<double>(ii[l], jj[l], l > 0, m)
-                         : fused_level_bytes<float>(ii[l], jj[l], l > 0, m);
-    }
-    return b;
-}
-
-template <typename T>
-void coarse_cycle(const coarse_level<T> *lv, int nlev, int max_side, int relax, int npre,
-                  int npost, const double *abd, double *bbd, hipStream_t s, int nb, int rep,
-                  std::size_t lds_bytes, int lds_mode) {
-    const int mode = lds_bytes > 0 ? lds_mode : 0;
-    if (max_side <= 64) {
-        if (mode)
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(coarse_cycle_k<T, 1>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-        coarse_cycle_k<T, 1><<<nb, 1024, lds_bytes, s>>>(lv, nlev, relax, npre, npost, abd, bbd,
-                                                         rep, mode);
-    } else {
-        if (mode)
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(coarse_cycle_k<T, 2>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-        coarse_cycle_k<T, 2><<<nb, 1024, lds_bytes, s>>>(lv, nlev, relax, npre, npost, abd, bbd,
-                                                         rep, mode);
-    }
 }
 
 template <typename Tin, typename Tout>
@@ -3713,51 +2002,36 @@ void copy(const T *src, T *dst, std::size_t n, hipStream_t s) {
 
 // explicit instantiations
 #define CDR_INST(T)                                                                               \
-    template void residual<T>(const T *, int, const T *, const T *, T *, int, int, hipStream_t,   \
-                              int, int);                                                          \
-    template void residual_norm<T>(const T *, int, const T *, const T *, T *, int, int, double *, \
-                                   double *, hipStream_t, int, int);                              \
+    template void residual<T>(const T *, int, const T *, const T *, T *, int, int,                \
+        hipStream_t, int, int);                                                                   \
+    template void residual_norm<T>(const T *, int, const T *, const T *, T *, int, int, double    \
+        *, double *, hipStream_t, int, int);                                                      \
     template void sumsq<T>(const T *, int, int, double *, double *, hipStream_t, int);            \
     template void relax_gs<T>(const T *, int, const T *, T *, const T *, int, int, int,           \
-                              hipStream_t, int, int);                                             \
-    template void relax_lines_x<T>(const T *, int, const T *, T *, const T *, int, int, int,      \
-                                   hipStream_t, int, int, int);                                   \
-    template void relax_lines_y<T>(const T *, int, const T *, T *, const T *, int, int, int,      \
-                                   hipStream_t, int, int);                                        \
-    template void relax_lines_xy<T>(const T *, int, const T *, T *, const T *, const T *, T *, int,\
-                                    int, int, hipStream_t, int, int);                             \
-    template int tune_lines<T>(int, const T *, int, const T *, T *, const T *, int, int,          \
-                               hipStream_t, int, int);                                            \
+        hipStream_t, int, int);                                                                   \
     template void transpose<T>(const T *, T *, int, int, hipStream_t, int);                       \
-    template void coarse_cycle<T>(const coarse_level<T> *, int, int, int, int, int, const double *, \
-                                  double *, hipStream_t, int, int, std::size_t, int);             \
     template void transpose_op<T>(const T *, T *, int, int, int, hipStream_t, int);               \
-    template bool relax_lines_y_auto<T>(const T *, const T *, int, const T *, T *, const T *, T *, \
-                                        T *, int, int, int, hipStream_t, int, bool, bool, bool,   \
-                                        int);                                                     \
-    template int uses_transposed_y<T>(const T *, int, int, int, int);                           \
-    template void residual_qT<T>(const T *, int, const T *, const T *, T *, int, int, hipStream_t, \
-                                 int, int);                                                       \
-    template void interp_add_qT<T>(T *, const T *, const T *, const T *, int, const T *, int, int, \
-                                   int, int, hipStream_t, int, int);                              \
-    template int tune_lines_ytr<T>(const T *, const T *, int, const T *, T *, const T *, T *, T *, \
-                                   int, int, hipStream_t, int, int, int);                         \
-    template void restrict_<T>(const T *, const T *, T *, int, int, int, int, hipStream_t, int,   \
-                               int);                                                              \
-    template void restrict_cycle<T>(const T *, const T *, T *, T *, T *, int, int, int, int,       \
-                                    hipStream_t, int, int);                                       \
-    template void interp_add<T>(T *, const T *, const T *, const T *, int, const T *, int, int,   \
-                                int, int, hipStream_t, int, int);                                 \
+    template void residual_qT<T>(const T *, int, const T *, const T *, T *, int, int,             \
+        hipStream_t, int, int);                                                                   \
+    template void interp_add_qT<T>(T *, const T *, const T *, const T *, int, const T *, int,     \
+        int, int, int, hipStream_t, int, int);                                                    \
+    template void restrict_<T>(const T *, const T *, T *, int, int, int, int, hipStream_t,        \
+        int, int);                                                                                \
+    template void restrict_cycle<T>(const T *, const T *, T *, T *, T *, int, int, int, int,      \
+        hipStream_t, int, int);                                                                   \
+    template void interp_add<T>(T *, const T *, const T *, const T *, int, const T *, int,        \
+        int, int, int, hipStream_t, int, int);                                                    \
     template void solve_cg<T>(T *, const T *, const double *, double *, int, int, hipStream_t,    \
-                              int, int);                                                          \
-    template void fill<T>(T *, T, std::size_t, hipStream_t);                                     \
-    template void relax_gs_per<T>(const T *, int, const T *, T *, const T *, int, int, int, int,  \
-                                  hipStream_t, int);                                              \
-    template void restrict_per<T>(const T *, T *, T *, int, int, int, int, int, hipStream_t, int);\
+        int, int);                                                                                \
+    template void fill<T>(T *, T, std::size_t, hipStream_t);                                      \
+    template void relax_gs_per<T>(const T *, int, const T *, T *, const T *, int, int, int,       \
+        int, hipStream_t, int);                                                                   \
+    template void restrict_per<T>(const T *, T *, T *, int, int, int, int, int, hipStream_t,      \
+        int);                                                                                     \
     template void interp_add_per<T>(T *, const T *, const T *, const T *, int, const T *, int,    \
-                                    int, int, int, int, hipStream_t, int);                        \
+        int, int, int, int, hipStream_t, int);                                                    \
     template void solve_cg_per<T>(T *, const T *, const double *, double *, int, int, int,        \
-                                  hipStream_t, int);                                              \
+        hipStream_t, int);                                                                        \
     template void copy<T>(const T *, T *, std::size_t, hipStream_t);                              \
     template void periodic_images<T>(T *, int, int, int, hipStream_t, int);
 CDR_INST(double)

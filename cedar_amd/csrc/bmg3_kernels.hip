@@ -956,6 +956,17 @@ __global__ __launch_bounds__(256) void solve_cg3_k(T *__restrict__ q, const T *_
         for (int t = tid; t < ld * n; t += nt) sh[n + t] = abd[t];
         ab = sh + n;
     }
+    if (lds && n <= 64 && kd < 64) {
+        __syncthreads();
+        if (tid < 64) {
+            const bool own = tid < n;
+            const std::size_t p =
+                own ? ix3(tid % nx + 2, (tid / nx) % ny + 2, tid / (nx * ny) + 2, ii, jj) : 0;
+            const double v = band_solve_upper_regs(ab, n, kd, ld, own ? (double)qf[p] : 0.0, tid);
+            if (own) q[p] = (T)v;
+        }
+        return;
+    }
     for (int t = tid; t < n; t += nt)
         xx[t] = (double)Q3(qf, t % nx + 2, (t / nx) % ny + 2, t / (nx * ny) + 2);
     __syncthreads();
