@@ -256,80 +256,6 @@ __global__ __launch_bounds__(256) void gs_colour_k(const T *__restrict__ so, con
 }
 
 // ------------------------------------------------------------------------------------------
-// line relaxation
-//
-// setup (src/2d/ftn/BMG2_SymStd_SETUP_lines_{x,y}.f90): diag = c, off = -w (x) or -s (y), then
-// LAPACK DPTTRF per line; one thread walks one line sequentially (setup-time only).
-// x factors: sor[0][p] = D, sor[1][p] = E at (i, j) as in the reference; y factors stored
-// transposed: plane k element (j, i) at k*ii*jj + i*jj + j.
-// ------------------------------------------------------------------------------------------
-// per: the line direction is periodic, so its wrap couplings are added to the end diagonals
-// (src/2d/ftn/BMG2_SymStd_SETUP_lines_x.f90:75-82, _y.f90:77-84) before the factorisation
-__global__ void setup_lines_x_k(const double *__restrict__ so, double *__restrict__ sor, int ii,
-                                int jj, int ns, int *__restrict__ info, int per = 0) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (j > jj - 2) return;
-    const std::size_t P = (std::size_t)ii * jj;
-    so += (std::size_t)blockIdx.y * ns * P;
-    sor += (std::size_t)blockIdx.y * 2 * P;
-    const int n = ii - 2;
-    double *D = sor + pidx(1, j, ii);      // D[k] at i = k + 1
-    double *E = sor + P + pidx(2, j, ii);  // E[k] at i = k + 2
-    for (int i = 1; i <= n; ++i) {
-        const std::size_t p = pidx(i, j, ii);
-        sor[P + p] = -so[P * KW + p];
-        sor[p] = so[p];
-    }
-    if (per) {
-        D[0] = D[0] + so[P * KW + pidx(1, j, ii)];
-        D[n - 1] = D[n - 1] + so[P * KW + pidx(ii - 1, j, ii)];
-    }
-    for (int k = 0; k < n - 1; ++k) {
-        const double d = D[k];
-        if (!(d > 0.0)) {
-            atomicMax(info, k + 1);
-            return;
-        }
-        const double ei = E[k];
-        E[k] = ei / d;
-        D[k + 1] = D[k + 1] - E[k] * ei;
-    }
-    if (!(D[n - 1] > 0.0)) atomicMax(info, n);
-}
-
-__global__ void setup_lines_y_k(const double *__restrict__ so, double *__restrict__ sor, int ii,
-                                int jj, int ns, int *__restrict__ info, int per = 0) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (i > ii - 2) return;
-    const std::size_t P = (std::size_t)ii * jj;
-    so += (std::size_t)blockIdx.y * ns * P;
-    sor += (std::size_t)blockIdx.y * 2 * P;
-    const int n = jj - 2;
-    double *D = sor + (std::size_t)i * jj + 1;
-    double *E = sor + P + (std::size_t)i * jj + 2;
-    for (int j = 1; j <= n; ++j) {
-        const std::size_t p = pidx(i, j, ii);
-        sor[P + (std::size_t)i * jj + j] = -so[P * KS + p];
-        sor[(std::size_t)i * jj + j] = so[p];
-    }
-    if (per) {
-        D[0] = D[0] + so[P * KS + pidx(i, 1, ii)];
-        D[n - 1] = D[n - 1] + so[P * KS + pidx(i, jj - 1, ii)];
-    }
-    for (int k = 0; k < n - 1; ++k) {
-        const double d = D[k];
-        if (!(d > 0.0)) {
-            atomicMax(info, k + 1);
-            return;
-        }
-        const double ei = E[k];
-        E[k] = ei / d;
-        D[k + 1] = D[k + 1] - E[k] * ei;
-    }
-    if (!(D[n - 1] > 0.0)) atomicMax(info, n);
-}
-
-// ------------------------------------------------------------------------------------------
 // restriction qc = P^T q (src/2d/ftn/BMG2_SymStd_restrict.f90:76-92); coarse (ic, jc) sits on
 // fine (2ic-1, 2jc-1)
 // ------------------------------------------------------------------------------------------
@@ -827,18 +753,6 @@ void relax_gs(const T *so, int nstncl, const T *qf, T *q, const T *sor, int ii, 
             gs_colour_k<T, false><<<g, 256, 0, s>>>(so, qf, q, sor, ii, jj, parity, 0, rep, t & 1);
         }
     }
-}
-
-void setup_lines_x(const double *so, int nstncl, double *sor, int ii, int jj, int *info,
-                   hipStream_t s, int nb) {
-    const int n = jj - 2;
-    setup_lines_x_k<<<dim3((n + 63) / 64, nb), 64, 0, s>>>(so, sor, ii, jj, nstncl, info);
-}
-
-void setup_lines_y(const double *so, int nstncl, double *sor, int ii, int jj, int *info,
-                   hipStream_t s, int nb) {
-    const int n = ii - 2;
-    setup_lines_y_k<<<dim3((n + 63) / 64, nb), 64, 0, s>>>(so, sor, ii, jj, nstncl, info);
 }
 
 // dst (cols x rows) = transpose of src (rows x cols), row-major, for each problem of a batch;
@@ -1887,19 +1801,6 @@ void relax_gs_per(const T *so, int nstncl, const T *qf, T *q, const T *sor, int 
         }
     }
     if (per_y(jpn)) ghost_y<T>(q, ii, jj, 0, ii - 1, s, nb);
-}
-
-void setup_lines_per(int dir, const double *so, int nstncl, double *sor, int ii, int jj, int jpn,
-                     int *info, hipStream_t s, int nb) {
-    if (dir == 0) {
-        const int n = jj - 2;
-        setup_lines_x_k<<<dim3((n + 63) / 64, nb), 64, 0, s>>>(so, sor, ii, jj, nstncl, info,
-                                                               per_x(jpn) ? 1 : 0);
-    } else {
-        const int n = ii - 2;
-        setup_lines_y_k<<<dim3((n + 63) / 64, nb), 64, 0, s>>>(so, sor, ii, jj, nstncl, info,
-                                                               per_y(jpn) ? 1 : 0);
-    }
 }
 
 template <typename T>

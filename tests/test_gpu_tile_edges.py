@@ -132,3 +132,30 @@ def test_gs27_rows(dims, dtype):
             assert np.array_equal(g, ref), ud
         else:  # 27 products and sums a point, eight colours deep
             assert np.abs(g - ref).max() <= 100 * 2.0 ** -24 * np.abs(ref).max(), ud
+
+
+# tiles of 64 elements and groups of 16 lines, one less, one more; two and three tiles; a pivot that
+# is not positive in the first tile, at a tile's edge and in the last element
+@pytest.mark.parametrize("nx,ny", [(2, 3), (63, 15), (64, 16), (65, 17), (129, 33), (193, 5), (7, 130)])
+@pytest.mark.parametrize("ns", [3, 5])
+def test_line_setup(nx, ny, ns):
+    import cedar_amd as C
+    print(f"\nline setup {nx}x{ny} ns={ns}", flush=True)
+    so = _so2(np.random.default_rng(nx + ny + ns), nx, ny, ns)
+    for d in ("x", "y"):
+        sor = O.setup_lines(so, d)
+        sor = sor[0] if isinstance(sor, tuple) else sor
+        g = torch.zeros(sor.shape, dtype=torch.float64, device="cuda")
+        assert np.array_equal(host(C.setup_lines(dev(so), g, d)), sor), d
+
+
+@pytest.mark.parametrize("k", [0, 1, 63, 64, 128])
+@pytest.mark.parametrize("d", ["x", "y"])
+def test_line_setup_reports_the_failing_pivot(k, d):
+    import cedar_amd as C
+    n = 129
+    so = _so2(np.random.default_rng(k), n, n, 5)
+    so[(0,) + ((5, k + 1) if d == "x" else (k + 1, 5))] = -1.0
+    g = torch.zeros((2, n + 2, n + 2), dtype=torch.float64, device="cuda")
+    with pytest.raises(C.CedarHipError):
+        C.setup_lines(dev(so), g, d)
