@@ -120,6 +120,10 @@ struct coarse_level {
     const T *sor0, *sor1;
     const T *ci;
     int ii, jj;
+    // first level, where its operator stays in memory and its smoothing has y-lines: the operator of
+    // the transposed grid (transpose_op) and a scratch grid; null: y-lines read so with stride ii
+    const T *soT;
+    T *bT;
 };
 // Runs one V-cycle over nlev levels (lv: device array, finest first; the last level is the
 // coarsest, solved with the band factor abd) in one launch of one workgroup per problem, for x of
@@ -129,15 +133,17 @@ struct coarse_level {
 // lds_bytes > 0 (at least fused_cycle_lds_bytes of the levels for lds_mode): lds_mode 1, every
 // array of the fused levels is staged in LDS for the whole cycle (only the first level's b and x
 // cross memory); lds_mode 2 or 3, the same except that of the first level only x, b and res (2)
-// or x alone (3) are in LDS, its other arrays stay in memory.
+// or x alone (3) are in LDS, its other arrays stay in memory.  With kCiInMemory added, the
+// interpolation stays in memory on every level.
+constexpr int kCiInMemory = 4;
 template <typename T>
 void coarse_cycle(const coarse_level<T> *lv, int nlev, int max_side, int relax, int npre,
                   int npost, const double *abd, double *bbd, hipStream_t s, int nb = 1,
                   int rep = 1, std::size_t lds_bytes = 0, int lds_mode = 1);
 // LDS bytes that fused levels of these extents (first level first) need at word size wbytes
-// with lds_mode 1, 2 or 3
-std::size_t fused_cycle_lds_bytes(int wbytes, const int *ii, const int *jj, int nlev,
-                                  int lds_mode = 1);
+// with lds_mode and relax as above
+std::size_t fused_cycle_lds_bytes(int wbytes, const int *ii, const int *jj, int nlev, int lds_mode,
+                                  int relax);
 
 // dst (cols x rows) = transpose of src (rows x cols), row-major, per problem of a batch
 template <typename T>

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace cdr {
 namespace k2 {
@@ -20,49 +21,86 @@ namespace {
 // unfused cycle.  Levels of a fused cycle are always 9-point (Galerkin operators).
 //
 // A chain of 60 to 150 short steps, each waiting for the one before: bound by the latency of a
-// step.  The arrays sit in LDS as far as they fit, addressed as LDS (MODE is a template parameter
-// and no pointer may be either, or every access becomes a flat one that waits for memory and LDS
-// alike), and a step's threads are dealt to exactly the points it updates, by shifts.
+// step.  The arrays sit in LDS as far as they fit, addressed as LDS (what lies where is a template
+// parameter and no pointer may be either, or every access becomes a flat one that waits for memory
+// and LDS alike); a step's threads are dealt to exactly the points it updates, by shifts; a first
+// level whose operator stays in memory has the operands of its next sweep loaded during the
+// current one, y-lines from a transposed copy so that they arrive with unit stride.  V(2,1) point
+// relaxation in FP64 from 32^2 down: 62 us with flat accesses, 46 with the first level's operator in
+// memory, 38 with only the planes point relaxation needs on chip; from 64^2 down 127, 108, 80.
+
+// Operands of one element of a line (everything but the iterate): right-hand side, couplings to
+// the neighbouring lines, multipliers of the forward and backward pass, pivot.
+template <typename T>
+struct line_ops {
+    T qf, s0, s1, sw0, nw0, nw1, sw1, ef, eb, d;
+};
+
+// Where the operands of the lines of one direction lie: element k of line L at L * line + (k + 1) *
+// elem of the operator planes and of b, at L * flen + k of D and E.
+template <typename T>
+struct line_src {
+    const T *sc, *sw, *nw, *b, *D, *E;
+    int elem, line, flen, nw0, nw1;
+};
+
+// dir 0: rows, 1: columns.  so holds the grid itself, or with transposed (dir 1) the operator of the
+// transposed grid, b transposed likewise.  The factors of a line are contiguous either way.
+template <typename T>
+__device__ inline line_src<T> line_source(const T *so, const T *b, const T *sor, int ii, int jj,
+                                          int dir, bool transposed) {
+    line_src<T> r;
+    const int P = ii * jj;
+    r.elem = dir == 0 || transposed ? 1 : ii;
+    r.line = dir == 0 ? ii : transposed ? jj : 1;
+    r.flen = dir == 0 ? ii : jj;
+    r.sc = so + P * (dir == 0 || transposed ? KS : KW);
+    r.sw = so + P * KSW;
+    r.nw = so + P * KNW;
+    r.b = b;
+    r.D = sor + 1;
+    r.E = sor + P + 2;
+    r.nw0 = dir == 0 ? r.elem : r.line;
+    r.nw1 = dir == 0 ? r.line : r.elem;
+    return r;
+}
+
+// operands of element k of line L of n elements, and the backward multiplier of element kb
+template <typename T>
+__device__ inline void load_ops(line_ops<T> &o, const line_src<T> &r, int L, int k, int kb, int n) {
+    const int kc = min(k, n - 1), p = L * r.line + (kc + 1) * r.elem, f = L * r.flen;
+    o.qf = r.b[p];
+    o.s0 = r.sc[p];
+    o.s1 = r.sc[p + r.line];
+    o.sw0 = r.sw[p];
+    o.nw0 = r.nw[p + r.nw0];
+    o.nw1 = r.nw[p + r.nw1];
+    o.sw1 = r.sw[p + r.elem + r.line];
+    o.ef = r.E[f + max(kc - 1, 0)];
+    o.d = r.D[f + kc];
+    o.eb = r.E[f + min(kb, max(n - 2, 0))];
+}
 
 // Lines of one colour, in place, by one wavefront: 64 / w lines of at most w = 64, 32 or 16 points
-// side by side (one line of at most 64*CH points where CH > 1), lane k of a line owning its
-// element k.  The scans stop where the lines do: the steps left out of scan_affine_dpp would
-// combine with the identity only, so a line's result does not depend on w.  x-lines (dir 0) lie
-// along rows, y-lines (dir 1) along columns; line = the wavefront's first of them.
+// side by side (w = 1 << ws; one line of at most 64*CH points where CH > 1), lane k of a line
+// owning its element k.  The scans stop where the lines do: the steps left out of scan_affine_dpp
+// would combine with the identity only, so a line's result does not depend on w.  act: the
+// lane's line exists; L: its index.
 template <typename T, int CH>
-__device__ inline void wave_lines(const T *__restrict__ so, const T *__restrict__ qf, T *q,
-                                  const T *__restrict__ sor, int ii, int jj, int dir, int first,
-                                  int nlines, int line, int w) {
-    const int lane = threadIdx.x % WAVE, e = lane & (w - 1), sub = lane & ~(w - 1);
-    const int P = ii * jj, n = dir == 0 ? ii - 2 : jj - 2;
-    const int mine = line + (int)((unsigned)sub / (unsigned)w);
-    const bool act = mine < nlines;
-    const int fixed = first + 2 * (act ? mine : nlines - 1);
+__device__ inline void solve_lines(const line_ops<T> (&o)[CH], T *q, int ii, int jj, int dir, int L,
+                                   bool act, int ws) {
+    const int w = 1 << ws, lane = threadIdx.x % WAVE, e = lane & (w - 1), sub = lane - e;
+    const int n = dir == 0 ? ii - 2 : jj - 2;
     const int step = dir == 0 ? 1 : ii, cross = dir == 0 ? ii : 1;
-    const int base = fixed * cross + step;  // element 0
-    const T *D = sor + fixed * (dir == 0 ? ii : jj) + 1, *E = D + P + 1;
-    const T *sc = so + P * (dir == 0 ? KS : KW), *sw = so + P * KSW, *nw = so + P * KNW;
+    const int base = L * cross + step;  // element 0
     T a[CH], b[CH];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-        const int k = u * WAVE + e, kc = min(k, n - 1), p = base + kc * step;
-        line_raw<T> r;
-        r.qf = qf[p];
-        r.s0 = sc[p];
-        r.q0 = q[p - cross];
-        r.s1 = sc[p + cross];
-        r.q1 = q[p + cross];
-        r.sw0 = sw[p];
-        r.q0m = q[p - ii - 1];
-        r.nw0 = nw[p + 1];
-        r.q0p = q[p - ii + 1];
-        r.nw1 = nw[p + ii];
-        r.q1m = q[p + ii - 1];
-        r.sw1 = sw[p + ii + 1];
-        r.q1p = q[p + ii + 1];
-        const T m = E[max(kc - 1, 0)];
+        const int k = u * WAVE + e, p = base + min(k, n - 1) * step;
+        line_raw<T> r{o[u].qf, o[u].s0, q[p - cross],  o[u].s1, q[p + cross],  o[u].sw0, q[p - ii - 1],
+                      o[u].nw0, q[p - ii + 1], o[u].nw1, q[p + ii - 1], o[u].sw1, q[p + ii + 1]};
         b[u] = line_rhs<T, true>(r);
-        a[u] = (k > 0) ? -m : T(0);
+        a[u] = (k > 0) ? -o[u].ef : T(0);
     }
 #pragma unroll
     for (int u = 0; u < CH; ++u) scan_affine_rows(a[u], b[u], w);
@@ -71,15 +109,14 @@ __device__ inline void wave_lines(const T *__restrict__ so, const T *__restrict_
     for (int u = 0; u < CH; ++u) {
         const T y = affine(a[u], carry, b[u]);
         if (CH > 1) carry = last_lane(y);
-        b[u] = div_pivot(y, D[min(u * WAVE + e, n - 1)]);
+        b[u] = div_pivot(y, o[u].d);
     }
     const int r = w - 1 - e;  // the backward pass runs from a line's last element
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
         const int k = u * WAVE + r;
         const T c = __shfl(b[u], sub + r, WAVE);
-        const T m = E[min(k, max(n - 2, 0))];
-        a[u] = (k < n - 1) ? -m : T(0);
+        a[u] = (k < n - 1) ? -o[u].eb : T(0);
         a[u] = (k < n) ? a[u] : T(1);
         b[u] = (k < n) ? c : T(0);
     }
@@ -98,17 +135,55 @@ __device__ inline void wave_lines(const T *__restrict__ so, const T *__restrict_
     }
 }
 
-// LDS bytes the fused cycle needs to hold the arrays of one level on chip (per level: the
-// operator, both relaxation factors, x, b, res and, below the first level, the interpolation),
-// each array rounded up to 16 bytes.  first_mode (the first level of lds_mode 2 or 3): x, b
-// and res (2) or x alone (3).
+// operands of one point of a Gauss-Seidel colour
 template <typename T>
-__host__ __device__ inline std::size_t fused_level_bytes(int ii, int jj, bool has_ci,
-                                                        int first_mode = 1) {
+struct point_ops {
+    T b, w0, w1, s0, s1, sw0, nw0, nw1, sw1, rec;
+};
+template <typename T>
+__device__ inline void load_point(point_ops<T> &o, const T *so, const T *b, const T *sor, int P,
+                                  int p, int ii) {
+    o.b = b[p];
+    o.w0 = so[P * KW + p];
+    o.w1 = so[P * KW + p + 1];
+    o.s0 = so[P * KS + p];
+    o.s1 = so[P * KS + p + ii];
+    o.sw0 = so[P * KSW + p];
+    o.nw0 = so[P * KNW + p + 1];
+    o.nw1 = so[P * KNW + p + ii];
+    o.sw1 = so[P * KSW + p + ii + 1];
+    o.rec = sor[P + p];
+}
+// the new value of point p, in the order of apply_offdiag
+template <typename T>
+__device__ inline T relax_point(const point_ops<T> &o, const T *q, int p, int ii) {
+    T v = o.b + o.w0 * q[p - 1];
+    v = v + o.w1 * q[p + 1];
+    v = v + o.s0 * q[p - ii];
+    v = v + o.s1 * q[p + ii];
+    v = v + o.sw0 * q[p - ii - 1];
+    v = v + o.nw0 * q[p - ii + 1];
+    v = v + o.nw1 * q[p + ii - 1];
+    v = v + o.sw1 * q[p + ii + 1];
+    return v * o.rec;
+}
+
+// planes of the relaxation data a level keeps on chip: 1 / c, the factors of one direction, or
+// those of both
+__host__ __device__ inline int relax_planes(int relax) {
+    return relax == CDR_RELAX_POINT ? 1 : relax == CDR_RELAX_LINE_XY ? 4 : 2;
+}
+
+// LDS bytes of one level: the operator, the relaxation data, x, b, res and, where ci, the
+// interpolation stored on it; each array rounded up to 16 bytes.  first_mode (the first level of
+// lds_mode 2 or 3): x, b and res (2) or x alone (3).
+template <typename T>
+__host__ __device__ inline std::size_t fused_level_bytes(int ii, int jj, bool ci, int first_mode,
+                                                        int relax) {
     const std::size_t plane = ((std::size_t)ii * jj * sizeof(T) + 15) / 16 * 16;
     if (first_mode == 2) return 3 * plane;
     if (first_mode == 3) return plane;
-    return plane * (5 + 2 + 2 + 3 + (has_ci ? 8 : 0));
+    return plane * (5 + relax_planes(relax) + 3 + (ci ? 8 : 0));
 }
 
 // a pointer read from memory, known to point to memory (and not to LDS)
@@ -124,9 +199,9 @@ __device__ inline int log2_up(int n) { return n <= 1 ? 0 : 32 - __clz(n - 1); }
 // they fit); the first level's b comes in from memory and its x goes back at the end, the only
 // values the caller exchanges with the fused levels.  For a first level too large to hold whole,
 // MODE 2 keeps only its x, b and res in LDS and MODE 3 its x alone; its other arrays stay in
-// memory, where the sweeps only read them, so that a sweep does not wait on memory for the
-// previous sweep's writes.  MODE 0: everything in memory.
-template <typename T, int CH, int MODE>
+// memory.  MODE 0: everything in memory.  CI: the interpolation weights are on chip too (each is
+// used once going down and once going up).
+template <typename T, int CH, int MODE, bool CI>
 __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__restrict__ lv,
                                                        int nlev, int relax, int npre, int npost,
                                                        const double *__restrict__ abd,
@@ -137,6 +212,7 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
     __shared__ double cg_sh[CG_LDS];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const std::size_t bz = blockIdx.x, bo = bz / rep;
+    const int nsor = relax_planes(relax);
     auto in_memory = [&](int l) {  // the level's arrays of problem bz (operator bo)
         coarse_level<T> d = lv[l];
         const std::size_t P = (std::size_t)d.ii * d.jj;
@@ -151,21 +227,27 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
     };
     // offset of level l in LDS, given that of a neighbour (the levels lie one after another)
     auto bytes_of = [&](int l) {
-        return (unsigned)fused_level_bytes<T>(lv[l].ii, lv[l].jj, l > 0, l == 0 ? M0 : 1);
+        return (unsigned)fused_level_bytes<T>(lv[l].ii, lv[l].jj, CI && l > 0, l == 0 ? M0 : 1, relax);
     };
     auto on_chip = [&](int l, unsigned off) {
         coarse_level<T> d;
         d.ii = lv[l].ii;
         d.jj = lv[l].jj;
-        const unsigned plane = ((unsigned)(d.ii * d.jj) * sizeof(T) + 15) / 16 * 16;
-        unsigned char *base = lds + off;
-        d.so = reinterpret_cast<T *>(base);
-        d.sor0 = reinterpret_cast<T *>(base + 5 * plane);
-        d.sor1 = reinterpret_cast<T *>(base + 7 * plane);
-        d.x = reinterpret_cast<T *>(base + 9 * plane);
-        d.b = reinterpret_cast<T *>(base + 10 * plane);
-        d.res = reinterpret_cast<T *>(base + 11 * plane);
-        d.ci = reinterpret_cast<T *>(base + 12 * plane);  // not there on level 0
+        const int P = d.ii * d.jj;
+        const unsigned plane = ((unsigned)P * sizeof(T) + 15) / 16 * 16;
+        T *base = reinterpret_cast<T *>(lds + off);
+        const unsigned pl = plane / sizeof(T);
+        d.x = base;
+        d.b = base + pl;
+        d.res = base + 2 * pl;
+        d.so = base + 3 * pl;
+        T *sor = base + 8 * pl;
+        d.sor0 = relax == CDR_RELAX_POINT ? sor - P : sor;  // point: the reciprocals are plane 1
+        d.sor1 = sor + 2 * pl;
+        if constexpr (CI)
+            d.ci = base + (8 + nsor) * pl;
+        else
+            d.ci = global_ptr(lv[l].ci) + bo * 8 * (std::size_t)P;
         return d;
     };
     auto lower = [&](int l, unsigned off) {
@@ -176,14 +258,18 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
     };
     auto first_level = [&] {  // MODE 2 and 3
         coarse_level<T> d = in_memory(0);
-        const unsigned plane = ((unsigned)(d.ii * d.jj) * sizeof(T) + 15) / 16 * 16;
+        const unsigned pl = (((unsigned)(d.ii * d.jj) * sizeof(T) + 15) / 16 * 16) / sizeof(T);
         d.x = reinterpret_cast<T *>(lds);
         if constexpr (MODE == 2) {
-            d.b = reinterpret_cast<T *>(lds + plane);
-            d.res = reinterpret_cast<T *>(lds + 2 * plane);
+            d.b = d.x + pl;
+            d.res = d.x + 2 * pl;
         }
         return d;
     };
+    // MODE 2 and 3: the first level's operator and (3) b for its y-lines, transposed; b is
+    // transposed here, into the scratch the caller gives, as it is new in every cycle
+    const T *soT = nullptr;
+    T *bT = nullptr;
     {
         const int n = (lv[nlev - 1].ii - 2) * (lv[nlev - 1].jj - 2);
         coarse_band_stage(abd + bo * (std::size_t)lv[nlev - 1].ii * n, lv[nlev - 1].ii,
@@ -196,21 +282,33 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
             const int P = g.ii * g.jj;
             if (MODE >= 2 && l == 0) {
                 const coarse_level<T> d = first_level();
+                const bool tr = lv[0].soT != nullptr &&
+                                (relax == CDR_RELAX_LINE_Y || relax == CDR_RELAX_LINE_XY);
+                if (tr) {
+                    soT = global_ptr(lv[0].soT) + bo * 5 * (std::size_t)P;
+                    bT = global_ptr(lv[0].bT) + bz * (std::size_t)P;
+                }
                 for (int k = tid; k < P; k += NT) {
+                    const T v = g.b[k];
                     d.x[k] = g.x[k];
                     if constexpr (MODE == 2) {
-                        d.b[k] = g.b[k];
+                        d.b[k] = v;
                         d.res[k] = T(0);
+                    } else {
+                        if (tr) bT[(k % g.ii) * g.jj + k / g.ii] = v;
                     }
                 }
             } else {
                 const coarse_level<T> d = on_chip(l, off);
                 for (int k = tid; k < 5 * P; k += NT) const_cast<T *>(d.so)[k] = g.so[k];
-                for (int k = tid; k < 2 * P; k += NT) {
-                    const_cast<T *>(d.sor0)[k] = g.sor0[k];
-                    const_cast<T *>(d.sor1)[k] = g.sor1[k];
+                if (relax == CDR_RELAX_POINT) {
+                    for (int k = tid; k < P; k += NT) const_cast<T *>(d.sor0)[P + k] = g.sor0[P + k];
+                } else {
+                    for (int k = tid; k < 2 * P; k += NT) const_cast<T *>(d.sor0)[k] = g.sor0[k];
+                    if (nsor == 4)
+                        for (int k = tid; k < 2 * P; k += NT) const_cast<T *>(d.sor1)[k] = g.sor1[k];
                 }
-                if (l > 0)
+                if (CI && l > 0)
                     for (int k = tid; k < 8 * P; k += NT) const_cast<T *>(d.ci)[k] = g.ci[k];
                 // res and, below the first level, b start at zero as in memory: their ghosts are
                 // never written, and interp_add adds the ghost res of an even-sized level to the
@@ -225,47 +323,204 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
         }
     }
     __syncthreads();
-    // Steps over the points (i, j) = (i0 + di * c, j0 + dj * r), c < nc, r < nr: threads along a row
-    // of the smallest power of two that holds it
+    // after a step that writes the iterate alone: with x on chip the operands on their way from
+    // memory need not have arrived
+    auto x_barrier = [] {
+        if constexpr (MODE == 0)
+            __syncthreads();
+        else
+            lds_barrier();
+    };
+    // Steps over the points (c, r), c < nc, r < nr: threads along a row of the smallest power of two
+    // that holds it
     auto each = [&](int nc, int nr, auto &&f) {
         const int sh = min(log2_up(nc), 10);
         for (int r = tid >> sh; r < nr; r += NT >> sh)
             for (int c = tid & ((1 << sh) - 1); c < nc; c += 1 << sh) f(c, r);
     };
+    // sweep t of a smoothing: colour of a point sweep; direction and first line of a line sweep
+    // (line-xy: x then y going down, y then x going up; two colours each)
+    const bool xy = relax == CDR_RELAX_LINE_XY;
+    auto colour = [&](int t, int updown, int &pi, int &pj) {
+        // DOWN: (i odd, j odd), (even, odd), (odd, even), (even, even); UP: reverse
+        const int c = updown == 0 ? t & 3 : 3 - (t & 3);
+        pi = c & 1;
+        pj = c >> 1;
+    };
+    auto sweep = [&](int t, int updown, int &dir, int &first) {
+        dir = xy ? ((t >> 1) ^ updown) & 1 : relax == CDR_RELAX_LINE_Y;
+        first = (t & 1) == updown ? 2 : 1;
+    };
+    auto width = [](int n) { return n <= 16 ? 4 : n <= 32 ? 5 : 6; };  // log2 of lanes per line
+    // the lane's line of wavefront wv, counted along the colour
+    auto lane_line = [&](int wv, int ws) { return (wv << (6 - ws)) + ((tid % WAVE) >> ws); };
     auto smooth = [&](const coarse_level<T> &d, int updown) {
         const int nrep = updown == 0 ? npre : npost;
         const int nx = d.ii - 2, ny = d.jj - 2, P = d.ii * d.jj;
         if (relax == CDR_RELAX_POINT) {
             for (int t = 0; t < 4 * nrep; ++t) {
-                // DOWN: (i odd, j odd), (even, odd), (odd, even), (even, even); UP: reverse
-                const int c = updown == 0 ? t & 3 : 3 - (t & 3), pi = c & 1, pj = c >> 1;
+                int pi, pj;
+                colour(t, updown, pi, pj);
                 each((nx + 1 - pi) / 2, (ny + 1 - pj) / 2, [&](int ic, int jc) {
                     const int p = (2 * jc + 1 + pj) * d.ii + 2 * ic + 1 + pi;
-                    const T v = apply_offdiag<T, true>(d.so, P, d.x, p, d.ii, d.b[p]);
-                    d.x[p] = v * d.sor0[P + p];
+                    point_ops<T> o;
+                    load_point(o, d.so, d.b, d.sor0, P, p, d.ii);
+                    d.x[p] = relax_point(o, d.x, p, d.ii);
                 });
-                __syncthreads();
+                x_barrier();
             }
             return;
         }
-        const bool xy = relax == CDR_RELAX_LINE_XY;
         for (int t = 0; t < nrep * (xy ? 4 : 2); ++t) {
-            // line-xy: x then y going down, y then x going up; two colours each
-            const int dir = xy ? ((t >> 1) ^ updown) & 1 : relax == CDR_RELAX_LINE_Y;
-            const int first = (t & 1) == updown ? 2 : 1;
+            int dir, first;
+            sweep(t, updown, dir, first);
             const int nfix = dir == 0 ? ny : nx, n = dir == 0 ? nx : ny;
-            if (first <= nfix) {
-                const int nlines = (nfix - first) / 2 + 1;
-                const int w = n <= 16 ? 16 : n <= 32 ? 32 : 64, per = WAVE / w;
-                const T *sor = xy && dir ? d.sor1 : d.sor0;
-                for (int line = wave * per; line < nlines; line += NWAVE * per) {
-                    if (CH > 1 && n > WAVE)
-                        wave_lines<T, CH>(d.so, d.b, d.x, sor, d.ii, d.jj, dir, first, nlines, line, WAVE);
-                    else
-                        wave_lines<T, 1>(d.so, d.b, d.x, sor, d.ii, d.jj, dir, first, nlines, line, w);
+            const int nlines = first <= nfix ? (nfix - first) / 2 + 1 : 0;
+            const line_src<T> src =
+                line_source<T>(d.so, d.b, xy && dir ? d.sor1 : d.sor0, d.ii, d.jj, dir, false);
+            const int ws = width(n), e = tid & ((1 << ws) - 1);
+            for (int wv = wave; wv << (6 - ws) < nlines; wv += NWAVE) {
+                const int m = lane_line(wv, ws);
+                const bool act = m < nlines;
+                const int L = first + 2 * (act ? m : nlines - 1);
+                if (CH > 1 && n > WAVE) {
+                    line_ops<T> o[CH];
+#pragma unroll
+                    for (int u = 0; u < CH; ++u)
+                        load_ops(o[u], src, L, u * WAVE + e, u * WAVE + WAVE - 1 - e, n);
+                    solve_lines<T, CH>(o, d.x, d.ii, d.jj, dir, L, act, 6);
+                } else {
+                    line_ops<T> o[1];
+                    load_ops(o[0], src, L, e, (1 << ws) - 1 - e, n);
+                    solve_lines<T, 1>(o, d.x, d.ii, d.jj, dir, L, act, ws);
                 }
             }
-            __syncthreads();
+            x_barrier();
+        }
+    };
+    // smooth() of a first level whose operator is in memory.  Up to 64 points a side a thread has at
+    // most one point of a colour and a wavefront at most two groups of lines, whose operands are
+    // loaded a sweep ahead; larger levels load them when they need them.
+    auto smooth_first = [&](const coarse_level<T> &d, int updown) {
+        const int nrep = updown == 0 ? npre : npost;
+        const int nx = d.ii - 2, ny = d.jj - 2, P = d.ii * d.jj;
+        if (relax == CDR_RELAX_POINT) {
+            if constexpr (CH > 1) {
+                smooth(d, updown);
+            } else {
+                auto point = [&](int t, int &p) {  // this thread's point of sweep t
+                    int pi, pj;
+                    colour(t, updown, pi, pj);
+                    const int nc = (nx + 1 - pi) / 2, nr = (ny + 1 - pj) / 2, sh = log2_up(nc);
+                    const int ic = tid & ((1 << sh) - 1), jc = tid >> sh;
+                    p = (2 * jc + 1 + pj) * d.ii + 2 * ic + 1 + pi;
+                    return ic < nc && jc < nr;
+                };
+                point_ops<T> cur{}, nxt{};
+                int p = 0, pn = 0;
+                bool on = point(0, p), onn = false;
+                if (on) load_point(cur, d.so, d.b, d.sor0, P, p, d.ii);
+                for (int t = 0; t < 4 * nrep; ++t) {
+                    onn = t + 1 < 4 * nrep && point(t + 1, pn);
+                    if (onn) load_point(nxt, d.so, d.b, d.sor0, P, pn, d.ii);
+                    if (on) d.x[p] = relax_point(cur, d.x, p, d.ii);
+                    x_barrier();
+                    cur = nxt;
+                    p = pn;
+                    on = onn;
+                }
+            }
+            return;
+        }
+        // two groups of lines per wavefront; FP64 has registers for the next operands of one
+        constexpr int SLOTS = 2, AHEAD = sizeof(T) == 8 ? 1 : 2;
+        // operands of this wavefront's groups of lines of sweep t
+        auto load = [&](int t, line_ops<T>(&o)[CH], int slot, int &L, bool &act, bool &any) {
+            int dir, first;
+            sweep(t, updown, dir, first);
+            const int nfix = dir == 0 ? ny : nx, n = dir == 0 ? nx : ny;
+            const int nlines = first <= nfix ? (nfix - first) / 2 + 1 : 0;
+            const int ws = width(n), e = tid & ((1 << ws) - 1), wv = wave + slot * NWAVE;
+            any = wv << (6 - ws) < nlines;
+            if (!any) return;
+            const int m = lane_line(wv, ws);
+            act = m < nlines;
+            L = first + 2 * (act ? m : nlines - 1);
+            const bool tr = dir == 1 && soT != nullptr;
+            const T *sor = xy && dir ? d.sor1 : d.sor0;
+            auto fetch = [&](const line_src<T> &src) {
+#pragma unroll
+                for (int u = 0; u < CH; ++u)
+                    load_ops(o[u], src, L, u * WAVE + e, u * WAVE + (1 << ws) - 1 - e, n);
+            };
+            // three sources whose arrays lie in different places; the transposed one of MODE 2
+            // reads b from LDS, where its order does not matter
+            line_src<T> src = line_source<T>(tr ? soT : d.so, d.b, sor, d.ii, d.jj, dir, tr);
+            if constexpr (MODE == 3) {
+                if (tr) src.b = bT;
+                fetch(src);
+            } else {
+                fetch(src);
+                if (tr)
+#pragma unroll
+                    for (int u = 0; u < CH; ++u)
+                        o[u].qf = d.b[(min(u * WAVE + e, n - 1) + 1) * d.ii + L];
+            }
+        };
+        const int total = nrep * (xy ? 4 : 2);
+        if constexpr (CH == 1) {
+            line_ops<T> cur[AHEAD][1] = {}, nxt[AHEAD][1] = {};
+            int L[AHEAD] = {}, Ln[AHEAD] = {};
+            bool act[AHEAD] = {}, actn[AHEAD] = {}, any[AHEAD] = {}, anyn[AHEAD] = {};
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s) load(0, cur[s], s, L[s], act[s], any[s]);
+            for (int t = 0; t < total; ++t) {
+                int dir, first;
+                sweep(t, updown, dir, first);
+                const int ws = width(dir == 0 ? nx : ny);
+                if (t + 1 < total)
+#pragma unroll
+                    for (int s = 0; s < AHEAD; ++s) load(t + 1, nxt[s], s, Ln[s], actn[s], anyn[s]);
+#pragma unroll
+                for (int s = 0; s < AHEAD; ++s)
+                    if (any[s]) solve_lines<T, 1>(cur[s], d.x, d.ii, d.jj, dir, L[s], act[s], ws);
+#pragma unroll
+                for (int s = AHEAD; s < SLOTS; ++s) {
+                    line_ops<T> o[1];
+                    int Lo = 0;
+                    bool acto = false, anyo = false;
+                    load(t, o, s, Lo, acto, anyo);
+                    if (anyo) solve_lines<T, 1>(o, d.x, d.ii, d.jj, dir, Lo, acto, ws);
+                }
+                x_barrier();
+#pragma unroll
+                for (int s = 0; s < AHEAD; ++s) {
+                    cur[s][0] = nxt[s][0];
+                    L[s] = Ln[s];
+                    act[s] = actn[s];
+                    any[s] = anyn[s];
+                }
+            }
+        } else {
+            for (int t = 0; t < total; ++t) {
+                int dir, first;
+                sweep(t, updown, dir, first);
+                bool any = true;
+                for (int s = 0; any; ++s) {
+                    line_ops<T> o[CH];
+                    int L = 0;
+                    bool act = false;
+                    load(t, o, s, L, act, any);
+                    const int n = dir == 0 ? nx : ny;
+                    if (!any) break;
+                    if (n > WAVE)
+                        solve_lines<T, CH>(o, d.x, d.ii, d.jj, dir, L, act, 6);
+                    else
+                        solve_lines<T, 1>(reinterpret_cast<line_ops<T>(&)[1]>(o[0]), d.x, d.ii, d.jj, dir,
+                                          L, act, width(n));
+                }
+                x_barrier();
+            }
         }
     };
     // going down: residual and restriction to the next level's b, whose x becomes zero
@@ -323,7 +578,7 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
         for (int s = 0; s < 2; ++s) {
             const coarse_level<T> C = on_chip(1, off);
             if (s == 1) up(F, C);
-            smooth(F, s);
+            smooth_first(F, s);
             if (s == 0) {
                 down(F, C);
                 cycle(1, off);
@@ -341,13 +596,14 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
 
 }  // namespace
 
-std::size_t fused_cycle_lds_bytes(int wbytes, const int *ii, const int *jj, int nlev,
-                                  int lds_mode) {
+std::size_t fused_cycle_lds_bytes(int wbytes, const int *ii, const int *jj, int nlev, int lds_mode,
+                                  int relax) {
     std::size_t b = 0;
+    const bool ci = !(lds_mode & kCiInMemory);
     for (int l = 0; l < nlev; ++l) {
-        const int m = l == 0 ? lds_mode : 1;
-        b += wbytes == 8 ? fused_level_bytes<double>(ii[l], jj[l], l > 0, m)
-                         : fused_level_bytes<float>(ii[l], jj[l], l > 0, m);
+        const int m = l == 0 ? lds_mode & ~kCiInMemory : 1;
+        b += wbytes == 8 ? fused_level_bytes<double>(ii[l], jj[l], ci && l > 0, m, relax)
+                         : fused_level_bytes<float>(ii[l], jj[l], ci && l > 0, m, relax);
     }
     return b;
 }
@@ -363,13 +619,22 @@ void coarse_cycle(const coarse_level<T> *lv, int nlev, int max_side, int relax, 
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
         kernel<<<nb, 1024, lds_bytes, s>>>(lv, nlev, relax, npre, npost, abd, bbd, rep);
     };
-    const bool one = max_side <= 64;  // lines of one 64-element chunk
-    switch (mode) {
-    case 0: one ? launch(coarse_cycle_k<T, 1, 0>) : launch(coarse_cycle_k<T, 2, 0>); break;
-    case 1: one ? launch(coarse_cycle_k<T, 1, 1>) : launch(coarse_cycle_k<T, 2, 1>); break;
-    case 2: one ? launch(coarse_cycle_k<T, 1, 2>) : launch(coarse_cycle_k<T, 2, 2>); break;
-    default: one ? launch(coarse_cycle_k<T, 1, 3>) : launch(coarse_cycle_k<T, 2, 3>); break;
-    }
+    auto pick = [&](auto ch) {  // lines of at most ch chunks of 64 elements
+        constexpr int CH = decltype(ch)::value;
+        switch (mode) {
+        case 0: return launch(coarse_cycle_k<T, CH, 0, false>);
+        case 1: return launch(coarse_cycle_k<T, CH, 1, true>);
+        case 2: return launch(coarse_cycle_k<T, CH, 2, true>);
+        case 3: return launch(coarse_cycle_k<T, CH, 3, true>);
+        case 1 | kCiInMemory: return launch(coarse_cycle_k<T, CH, 1, false>);
+        case 2 | kCiInMemory: return launch(coarse_cycle_k<T, CH, 2, false>);
+        default: return launch(coarse_cycle_k<T, CH, 3, false>);
+        }
+    };
+    if (max_side <= 64)
+        pick(std::integral_constant<int, 1>{});
+    else
+        pick(std::integral_constant<int, 2>{});
 }
 
 #define CDR_INST(T)                                                                               \

@@ -272,6 +272,8 @@ private:
     std::size_t fuse_lds_ = 0;  // LDS bytes of the on-chip fused cycle (0: arrays in memory)
     int fuse_lds_mode_ = 0;     // its lds_mode (k2::coarse_cycle)
     dbuf<unsigned char> fuse64_, fuse32_;
+    dbuf<double> fuse_soT64_, fuse_bT64_;  // of the fused cycle's first level (build_fused)
+    dbuf<float> fuse_soT32_, fuse_bT32_;
     int *host_active_ = nullptr;   // nb flags (pinned)
     hipEvent_t ev0_{}, ev1_{};
     double setup_s_ = 0, solve_s_ = 0;
@@ -488,7 +490,25 @@ private:
         for (int l = lt; l < nl; ++l) {
             const level_data<T> &D = L[l];
             v.push_back(k2::coarse_level<T>{D.A.p, D.x.p, D.b.p, D.res.p, D.SOR[0].p, D.SOR[1].p,
-                                            l == lt ? nullptr : D.P.p, D.ext.ii, D.ext.jj});
+                                            l == lt ? nullptr : D.P.p, D.ext.ii, D.ext.jj, nullptr,
+                                            nullptr});
+        }
+        pick_lds_mode<T>(L, lt);
+        // a first level whose operator stays in memory reads it for its y-lines from a transposed
+        // copy
+        const bool ylines = set_.relaxation == CDR_RELAX_LINE_Y || set_.relaxation == CDR_RELAX_LINE_XY;
+        dbuf<T> &soT = fuse_soT<T>(), &bT = fuse_bT<T>();
+        if (ylines && (fuse_lds_mode_ & 3) >= 2) {
+            const level_data<T> &D = L[lt];
+            soT = dbuf<T>(D.A.ext.total() * 5, stream_);
+            bT = dbuf<T>(D.ext.total(), stream_);
+            k2::transpose_op<T>(D.A.p, soT.data(), 5, D.ext.ii, D.ext.jj, stream_, D.A.ext.nb);
+            check_hip(hipGetLastError(), "transpose_op");
+            v[0].soT = soT.data();
+            v[0].bT = bT.data();
+        } else {
+            soT = dbuf<T>();
+            bT = dbuf<T>();
         }
         const std::size_t bytes = v.size() * sizeof(k2::coarse_level<T>);
         dst = dbuf<unsigned char>(bytes, stream_);
@@ -497,28 +517,46 @@ private:
         check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
         fuse_lvl_ = lt;
         fuse_side_ = std::max(L[lt].ext.nx(), L[lt].ext.ny());
-        // the fused levels run out of LDS where all their arrays fit in one workgroup's share
+    }
+
+    // The fused levels run out of LDS as far as their arrays fit: every array, else all but the
+    // interpolation, else all but the first level's read-only arrays, else of the first level its x
+    // alone, else these without the interpolation, else none.
+    template <typename T>
+    void pick_lds_mode(const std::vector<level_data<T>> &L, int lt) {
         std::vector<int> ii, jj;
-        for (int l = lt; l < nl; ++l) {
+        for (std::size_t l = lt; l < L.size(); ++l) {
             ii.push_back(L[l].ext.ii);
             jj.push_back(L[l].ext.jj);
         }
-        // every array on chip where they fit, else all but the first level's read-only arrays,
-        // else all but everything of the first level except its x, else none
         fuse_lds_mode_ = 0;
         fuse_lds_ = 0;
-        for (int mode = 1; mode <= 3 && !fuse_lds_mode_; ++mode) {
-            const std::size_t need = k2::fused_cycle_lds_bytes((int)sizeof(T), ii.data(),
-                                                               jj.data(), nl - lt, mode);
-            if (need <= kFusedLdsMax) {
-                fuse_lds_mode_ = mode;
-                fuse_lds_ = need;
-            }
+        for (int mode : {1, 1 | k2::kCiInMemory, 2, 3, 2 | k2::kCiInMemory, 3 | k2::kCiInMemory}) {
+            const std::size_t need = k2::fused_cycle_lds_bytes(
+                (int)sizeof(T), ii.data(), jj.data(), (int)ii.size(), mode, set_.relaxation);
+            if (need > kFusedLdsMax) continue;
+            fuse_lds_mode_ = mode;
+            fuse_lds_ = need;
+            break;
         }
+    }
+    template <typename T>
+    dbuf<T> &fuse_soT() {
+        if constexpr (std::is_same<T, double>::value)
+            return fuse_soT64_;
+        else
+            return fuse_soT32_;
+    }
+    template <typename T>
+    dbuf<T> &fuse_bT() {
+        if constexpr (std::is_same<T, double>::value)
+            return fuse_bT64_;
+        else
+            return fuse_bT32_;
     }
     // of the 160 KiB per workgroup; the kernel's static 8 KiB staging area of the coarsest
     // solve comes on top
-    static constexpr std::size_t kFusedLdsMax = 150 * 1024;
+    static constexpr std::size_t kFusedLdsMax = 152 * 1024;
 
     // Milliseconds per replay of what body() launches, captured as a graph on the capture stream
     // and replayed 3 times on the solver's stream after a warm-up; -1 if capture fails.

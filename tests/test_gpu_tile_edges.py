@@ -159,3 +159,22 @@ def test_line_setup_reports_the_failing_pivot(k, d):
     g = torch.zeros((2, n + 2, n + 2), dtype=torch.float64, device="cuda")
     with pytest.raises(C.CedarHipError):
         C.setup_lines(dev(so), g, d)
+
+
+# first levels of the fused coarse cycle that lie in LDS whole, but for the interpolation, for the
+# operator, with the iterate alone, not at all, in both word sizes; lines of 16, 32, 64 points and
+# more, several to a wavefront, odd and even.  num_levels = 3 leaves one level to start at.
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+@pytest.mark.parametrize("relax", ["point", "line-x", "line-y", "line-xy"])
+@pytest.mark.parametrize("nx,ny", [(31, 33), (33, 18), (63, 64), (66, 61), (95, 90), (127, 128),
+                                   (130, 60), (163, 150), (200, 199), (60, 250)])
+def test_fused_cycle_memory_modes(nx, ny, relax, precision):
+    import cedar_amd as C
+    print(f"\nfused {nx}x{ny} {relax} {precision}", flush=True)
+    rng = np.random.default_rng(nx + ny)
+    so, b = dev(_so2(rng, nx, ny, 5)), dev(rng.standard_normal((ny + 2, nx + 2)))
+    kw = dict(relaxation=relax, nrelax_pre=2, nrelax_post=1, num_levels=3, maxiter=3, tol=1e-30,
+              precision=precision)
+    x, h = C.Solver(so, **kw).solve(b)
+    y, g = C.Solver(so, fused_coarse=False, **kw).solve(b)
+    assert torch.equal(x, y) and np.array_equal(h, g)
