@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "../../include/cedar_hip.h"
+#include "device_pool.hpp"
 
 namespace cedar {
 namespace hip {
@@ -49,7 +50,9 @@ public:
     dbuf() = default;
     explicit dbuf(std::size_t n, hipStream_t s = nullptr) : n_(n) {
         if (n_ == 0) return;
-        check_hip(hipMalloc(&p_, n_ * sizeof(T)), "hipMalloc");
+        hipError_t e = hipSuccess;
+        p_ = static_cast<T *>(pool_malloc(n_ * sizeof(T), &e));
+        check_hip(e, "hipMalloc");
         check_hip(hipMemsetAsync(p_, 0, n_ * sizeof(T), s), "hipMemsetAsync");
     }
     dbuf(const dbuf &) = delete;
@@ -67,7 +70,7 @@ public:
     }
     ~dbuf() { reset(); }
     void reset() {
-        if (p_) (void)hipFree(p_);
+        pool_free(p_);
         p_ = nullptr;
         n_ = 0;
     }

@@ -1,0 +1,58 @@
+// Device memory and capture streams kept from one solver to the next.
+//
+// A solver allocates some fifty buffers and frees them together, and every hipFree waits for the
+// device and unmaps: 10 of the 31 ms of a differentiated solve of 4 x 1025^2, which builds a solver
+// per call, went into it and 2 ms into hipMalloc.  Blocks of a destroyed solver are therefore kept
+// for the next one of the same sizes, per device and byte count, up to kPoolBytes in all; beyond
+// that the ones kept longest are freed, and when an allocation fails all of them are.
+//
+// A block may be handed to any thread and stream, so it is only kept while no queued work can still
+// use it: inside a pool_idle_scope.  Outside one pool_free is hipFree.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <optional>
+
+namespace cedar {
+namespace hip {
+
+constexpr std::size_t kPoolBytes = std::size_t(4) << 30;
+
+// nullptr and the error in *e on failure
+void *pool_malloc(std::size_t bytes, hipError_t *e);
+void pool_free(void *p);
+
+// While alive, blocks of the current device that this thread frees are idle: nothing queued uses
+// them.  The constructor waits for the device, or for the stream that alone used them.
+class pool_idle_scope {
+public:
+    pool_idle_scope();
+    explicit pool_idle_scope(hipStream_t s);
+    ~pool_idle_scope();
+    pool_idle_scope(const pool_idle_scope &) = delete;
+    pool_idle_scope &operator=(const pool_idle_scope &) = delete;
+
+private:
+    void enter(hipError_t waited);
+    int prev_;
+};
+
+// First member of a class that owns buffers: its destructor calls enter(), and as the first member
+// is destroyed last, the members after it give their blocks back idle.
+class pool_guard {
+public:
+    void enter() { scope_.emplace(); }
+
+private:
+    std::optional<pool_idle_scope> scope_;
+};
+
+// A non-blocking stream of the current device for captures alone (no work runs on it, so the next
+// solver can take it over); nullptr and the error in *e on failure.  At most 16 are kept.
+hipStream_t pool_capture_stream(hipError_t *e);
+void pool_return_capture_stream(hipStream_t s);
+
+}  // namespace hip
+}  // namespace cedar

@@ -6,7 +6,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -142,6 +144,19 @@ private:
 };
 
 }  // namespace
+
+int fused_start(const fused_start_key &key, int record) {
+    static std::mutex mu;
+    static std::map<fused_start_key, int> table;
+    std::lock_guard<std::mutex> g(mu);
+    if (record < 0) {
+        const auto it = table.find(key);
+        return it == table.end() ? -1 : it->second;
+    }
+    if (table.size() >= 1024) table.clear();
+    table[key] = record;
+    return record;
+}
 
 void register_hip_kernels(kernel_manager &km, int *info) {
     km.add<kernels::residual<double>, hip_residual<double>>("hip");

@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -49,6 +50,12 @@ struct level_data {
     relax_stencil<T> SOR[2];
 };
 
+// First level of the fused coarse cycle by word size, smoothing, extents, levels, batch and
+// right-hand sides per operator: the recorded one (record < 0; -1 if none), or records `record`.  One
+// table per process, guarded by a mutex, emptied when it holds 1024 entries.
+using fused_start_key = std::array<int, 9>;
+int fused_start(const fused_start_key &key, int record);
+
 class solver2d {
 public:
     // nb operators of the same extents (so_dev holds them back to back), each with rep
@@ -69,9 +76,10 @@ public:
     }
 
     ~solver2d() {
+        guard_.enter();
         for (auto *g : {&g64_, &g32_})
             if (g->exec) (void)hipGraphExecDestroy(g->exec);
-        if (cap_stream_) (void)hipStreamDestroy(cap_stream_);
+        pool_return_capture_stream(cap_stream_);
         (void)hipEventDestroy(ev0_);
         (void)hipEventDestroy(ev1_);
         if (host_norm_) (void)hipHostFree(host_norm_);
@@ -244,6 +252,7 @@ private:
         check_hip(hipGetLastError(), "periodic_images");
     }
 
+    pool_guard guard_;  // before every buffer
     int jpn_ = 0;
     int rep_ = 1;  // right-hand sides per operator
     cdr_solver_settings set_;
@@ -293,9 +302,7 @@ private:
                 check_hip(hipGraphExecDestroy(g.exec), "hipGraphExecDestroy");
                 g.exec = nullptr;
             }
-            if (!cap_stream_)
-                check_hip(hipStreamCreateWithFlags(&cap_stream_, hipStreamNonBlocking),
-                          "hipStreamCreateWithFlags");
+            need_capture_stream();
             check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
             set_stream(cap_stream_);
             check_hip(hipStreamBeginCapture(cap_stream_, hipStreamCaptureModeThreadLocal),
@@ -318,6 +325,13 @@ private:
             g.k2 = k2;
         }
         check_hip(hipGraphLaunch(g.exec, stream_), "hipGraphLaunch");
+    }
+
+    void need_capture_stream() {
+        if (cap_stream_) return;
+        hipError_t e = hipSuccess;
+        cap_stream_ = pool_capture_stream(&e);
+        check_hip(e, "hipStreamCreateWithFlags");
     }
 
     void read_norms() {
@@ -461,6 +475,17 @@ private:
         if (cand.empty()) return;
         int lt = cand[0];
         if (cand.size() > 1 && k2::autotune_enabled()) {
+            // the choice depends on sizes and settings alone, so the next solver with the same ones
+            // takes it over instead of capturing and timing five cycles again (4 of 25 ms of a 1500 x
+            // 1100 setup and solve)
+            const extents &e = L[0].ext;
+            const fused_start_key key{(int)sizeof(T), set_.relaxation, set_.nrelax_pre,
+                                      set_.nrelax_post, e.ii, e.jj, nl, e.nb, rep_};
+            const int known = fused_start(key, -1);
+            if (known >= 0) {
+                build_fused<T>(L, known, dst);
+                return;
+            }
             const int top = *std::min_element(cand.begin(), cand.end());
             float tbest = -1.f;
             for (int c : cand) {
@@ -478,6 +503,7 @@ private:
                     lt = c;
                 }
             }
+            if (tbest >= 0.f) fused_start(key, lt);
         }
         build_fused<T>(L, lt, dst);
     }
@@ -498,6 +524,7 @@ private:
         // copy
         const bool ylines = set_.relaxation == CDR_RELAX_LINE_Y || set_.relaxation == CDR_RELAX_LINE_XY;
         dbuf<T> &soT = fuse_soT<T>(), &bT = fuse_bT<T>();
+        const pool_idle_scope idle(stream_);  // the buffers of the start level tried before
         if (ylines && (fuse_lds_mode_ & 3) >= 2) {
             const level_data<T> &D = L[lt];
             soT = dbuf<T>(D.A.ext.total() * 5, stream_);
@@ -562,9 +589,7 @@ private:
     // and replayed 3 times on the solver's stream after a warm-up; -1 if capture fails.
     template <typename F>
     float time_graph(F body) {
-        if (!cap_stream_)
-            check_hip(hipStreamCreateWithFlags(&cap_stream_, hipStreamNonBlocking),
-                      "hipStreamCreateWithFlags");
+        need_capture_stream();
         check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
         set_stream(cap_stream_);
         if (hipStreamBeginCapture(cap_stream_, hipStreamCaptureModeThreadLocal) != hipSuccess) {
@@ -645,11 +670,15 @@ private:
                                                 rep_);
             if (c == -2) throw error(CDR_ERR_HIP, "line-kernel tuning failed");
             if (c < 0) {  // direct y-lines: the transposed workspace is not needed
+                const pool_idle_scope idle(stream_);
                 D.soT_buf = dbuf<T>();
                 D.xT_buf = dbuf<T>();
                 D.bT_buf = dbuf<T>();
             }
         }
+        const pool_idle_scope idle(stream_);
+        q.reset();
+        f.reset();
     }
 
     void setup_relax(level_data<double> &F) {

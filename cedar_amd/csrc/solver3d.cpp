@@ -361,6 +361,7 @@ public:
         build(so_dev, ns, nx, ny, nz);
     }
     ~solver3d() {
+        guard_.enter();
         (void)hipEventDestroy(ev0_);
         (void)hipEventDestroy(ev1_);
         if (host_norm_) (void)hipHostFree(host_norm_);
@@ -467,6 +468,7 @@ public:
     }
 
 private:
+    pool_guard guard_;  // before every buffer
     cdr_solver3_settings set_;
     hipStream_t stream_;
     kernel_manager km_;

@@ -1,0 +1,80 @@
+"""Solvers built from the memory of destroyed ones, on one and on several threads and streams."""
+import threading
+
+import numpy as np
+import pytest
+
+from cedar_amd import gallery as G
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _problem(n, seed):
+    so, b, _ = G.heterogeneous_9pt(n, seed=seed, block=8, sigma=1.0)
+    return torch.as_tensor(so).cuda(), torch.as_tensor(b).cuda()
+
+
+KW = dict(relaxation="line-xy", nrelax_pre=1, nrelax_post=1, maxiter=30, tol=1e-10)
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+def test_a_rebuilt_solver_gives_the_same_solution(precision):
+    import cedar_amd as C
+    first = {}
+    for rnd in range(3):
+        for n in (65, 96, 130):
+            so, b = _problem(n, n)
+            s = C.Solver(so, precision=precision, **KW)
+            x, h = s.solve(b)
+            s.close()
+            if rnd == 0:
+                first[n] = (x, h)
+            else:
+                assert torch.equal(x, first[n][0]) and np.array_equal(h, first[n][1])
+
+
+def test_rebuilt_3d_solvers():
+    import cedar_amd as C
+    so, b, _ = G.poisson3_sine(33)
+    so, b = torch.as_tensor(so).cuda(), torch.as_tensor(b).cuda()
+    ref = None
+    for relax in ("point", "plane-xy", "point", "plane-xy"):
+        s = C.Solver3(so, relaxation=relax, maxiter=4)
+        x, h = s.solve(b)
+        s.close()
+        ref = ref or {}
+        if relax in ref:
+            assert torch.equal(x, ref[relax][0]) and np.array_equal(h, ref[relax][1])
+        ref[relax] = (x, h)
+
+
+def test_threads_and_streams_that_build_and_destroy_solvers():
+    import cedar_amd as C
+    sizes = (65, 66, 96, 97)
+    probs = {n: _problem(n, n) for n in sizes}
+    ref = {n: C.Solver(probs[n][0], **KW).solve(probs[n][1]) for n in sizes}
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(k):
+        try:
+            st = torch.cuda.Stream()
+            with torch.cuda.stream(st):
+                for r in range(4):
+                    n = sizes[(k + r) % len(sizes)]
+                    s = C.Solver(probs[n][0], **KW)
+                    x, h = s.solve(probs[n][1])
+                    s.close()
+                    if not (torch.equal(x, ref[n][0]) and np.array_equal(h, ref[n][1])):
+                        bad.append((k, r, n))
+                st.synchronize()
+        except BaseException as exc:  # reported by the main thread
+            bad.append(exc)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad
