@@ -54,20 +54,40 @@ __device__ inline void block_sum_store(double v, double *dst) {
     }
 }
 
+// Left to itself the compiler issues the operands of a long sum a few at a time and waits in
+// between.  Where a launch is short (every level of at most 512 points a side) those waits are its
+// whole time, so the point functions below issue all loads before the first product
+// (loads_issued): a 511^2 Poisson solve 1.91 -> 1.84 ms, the 27-point FP32 residual at
+// 127 x 127 x 95 15.2 -> 8.2 us.
+__device__ inline void loads_issued() { __builtin_amdgcn_sched_barrier(0); }
+
 // f + the couplings of point p to its neighbours, in the reference's order
 // (src/2d/ftn/BMG2_SymStd_residual.f90:85-119)
 template <typename T, bool NINE>
 __device__ inline T apply_offdiag(const T *__restrict__ so, std::size_t P, const T *__restrict__ q,
                                   std::size_t p, int ii, T acc) {
-    acc = acc + so[P * KW + p] * q[p - 1];
-    acc = acc + so[P * KW + p + 1] * q[p + 1];
-    acc = acc + so[P * KS + p] * q[p - ii];
-    acc = acc + so[P * KS + p + ii] * q[p + ii];
-    if (NINE) {
-        acc = acc + so[P * KSW + p] * q[p - ii - 1];
-        acc = acc + so[P * KNW + p + 1] * q[p - ii + 1];
-        acc = acc + so[P * KNW + p + ii] * q[p + ii - 1];
-        acc = acc + so[P * KSW + p + ii + 1] * q[p + ii + 1];
+    const T w0 = so[P * KW + p], w1 = so[P * KW + p + 1];
+    const T s0 = so[P * KS + p], s1 = so[P * KS + p + ii];
+    const T qw = q[p - 1], qe = q[p + 1], qs = q[p - ii], qn = q[p + ii];
+    if constexpr (NINE) {
+        const T sw0 = so[P * KSW + p], nw0 = so[P * KNW + p + 1];
+        const T nw1 = so[P * KNW + p + ii], sw1 = so[P * KSW + p + ii + 1];
+        const T qsw = q[p - ii - 1], qse = q[p - ii + 1], qnw = q[p + ii - 1], qne = q[p + ii + 1];
+        loads_issued();
+        acc = acc + w0 * qw;
+        acc = acc + w1 * qe;
+        acc = acc + s0 * qs;
+        acc = acc + s1 * qn;
+        acc = acc + sw0 * qsw;
+        acc = acc + nw0 * qse;
+        acc = acc + nw1 * qnw;
+        acc = acc + sw1 * qne;
+    } else {
+        loads_issued();
+        acc = acc + w0 * qw;
+        acc = acc + w1 * qe;
+        acc = acc + s0 * qs;
+        acc = acc + s1 * qn;
     }
     return acc;
 }
@@ -283,21 +303,46 @@ __device__ inline void line_load(line_raw<T> &r, const T *__restrict__ so, const
 
 // coarse point (ic, jc) of qc = P^T q (the reference's operation order); ci, q, qc of one problem
 template <typename T>
-__device__ inline T restrict_point(const T *__restrict__ ci, const T *__restrict__ q, int iif,
-                                   int iic, std::size_t Pc, int ic, int jc) {
+struct restrict_ops {
+    T w[8], q[9];
+};
+template <typename T>
+__device__ inline void load_restrict(restrict_ops<T> &o, const T *__restrict__ ci,
+                                     const T *__restrict__ q, int iif, int iic, std::size_t Pc,
+                                     int ic, int jc) {
     const int i = 2 * ic - 1, j = 2 * jc - 1;
     auto CI = [&](int a, int b, int k) { return ci[Pc * k + pidx(a, b, iic)]; };
     auto Q = [&](int a, int b) { return q[pidx(a, b, iif)]; };
-    T v = CI(ic, jc, LNE) * Q(i - 1, j - 1);
-    v = v + CI(ic, jc, LA) * Q(i, j - 1);
-    v = v + CI(ic + 1, jc, LNW) * Q(i + 1, j - 1);
-    v = v + CI(ic, jc, LR) * Q(i - 1, j);
-    v = v + Q(i, j);
-    v = v + CI(ic + 1, jc, LL) * Q(i + 1, j);
-    v = v + CI(ic, jc + 1, LSE) * Q(i - 1, j + 1);
-    v = v + CI(ic, jc + 1, LB) * Q(i, j + 1);
-    v = v + CI(ic + 1, jc + 1, LSW) * Q(i + 1, j + 1);
+    o.w[0] = CI(ic, jc, LNE), o.q[0] = Q(i - 1, j - 1);
+    o.w[1] = CI(ic, jc, LA), o.q[1] = Q(i, j - 1);
+    o.w[2] = CI(ic + 1, jc, LNW), o.q[2] = Q(i + 1, j - 1);
+    o.w[3] = CI(ic, jc, LR), o.q[3] = Q(i - 1, j);
+    o.q[8] = Q(i, j);
+    o.w[4] = CI(ic + 1, jc, LL), o.q[4] = Q(i + 1, j);
+    o.w[5] = CI(ic, jc + 1, LSE), o.q[5] = Q(i - 1, j + 1);
+    o.w[6] = CI(ic, jc + 1, LB), o.q[6] = Q(i, j + 1);
+    o.w[7] = CI(ic + 1, jc + 1, LSW), o.q[7] = Q(i + 1, j + 1);
+}
+template <typename T>
+__device__ inline T sum_restrict(const restrict_ops<T> &o) {
+    T v = o.w[0] * o.q[0];
+    v = v + o.w[1] * o.q[1];
+    v = v + o.w[2] * o.q[2];
+    v = v + o.w[3] * o.q[3];
+    v = v + o.q[8];
+    v = v + o.w[4] * o.q[4];
+    v = v + o.w[5] * o.q[5];
+    v = v + o.w[6] * o.q[6];
+    v = v + o.w[7] * o.q[7];
     return v;
+}
+template <typename T>
+__device__ inline T restrict_point(const T *__restrict__ ci, const T *__restrict__ q, int iif,
+                                   int iic, std::size_t Pc, int ic, int jc) {
+    restrict_ops<T> o;
+    load_restrict(o, ci, q, iif, iic, Pc, ic, jc);
+    loads_issued();
+    return sum_restrict(o);
 }
 
 // One 2 x 2 block of fine points (2m-1 .. 2m, 2n-1 .. 2n) of interp_add: the coarse point
@@ -319,7 +364,8 @@ __device__ inline void store_pair(float *p, float a, float b) {
     __builtin_memcpy(p, &v, sizeof(v));
 }
 
-template <typename T>
+// PAIRS: in FP32, blocks inside the grid move horizontally adjacent values as pairs.
+template <typename T, bool PAIRS = true>
 __device__ inline void interp_block(T *__restrict__ q, const T *__restrict__ qc,
                                     const T *__restrict__ res, const T *__restrict__ so,
                                     const T *__restrict__ ci, int iic, int jjc, int iif, int jjf,
@@ -332,76 +378,67 @@ __device__ inline void interp_block(T *__restrict__ q, const T *__restrict__ qc,
     const std::size_t Pc = (std::size_t)iic * jjc;
     auto CI = [&](int a, int b, int k) { return ci[Pc * k + pidx(a, b, iic)]; };
     auto QC = [&](int a, int b) { return qc[pidx(a, b, iic)]; };
-    auto R = [&](int i, int j, std::size_t p) {
-        return (i > iif - 2 || j > jjf - 2) ? res[p] : res[p] / so[p];
-    };
-    if constexpr (sizeof(T) == 4) {
-        // FP32: the same operations, with horizontally adjacent values moved as pairs where the
-        // point (2m, .) exists (xe): then i0 + 1 <= iif - 1 and m + 1 <= iic - 1, so every pair
-        // lies inside its row (for even sizes i0 can be the ghost column, where xe is false)
-        const std::size_t p = pidx(i0, j0, iif);
-        T c00, c10 = T(0), c01 = T(0), c11 = T(0);
-        if (xe) {
+    if constexpr (PAIRS && sizeof(T) == 4) {
+        if (xe && ye && i0 + 1 <= iif - 2 && j0 + 1 <= jjf - 2) {
+            const std::size_t p = pidx(i0, j0, iif), p2 = p + iif;
+            T q0, q1, q2, q3, c00, c10, c01, c11, r2, r3, s2, s3;
             load_pair(qc + pidx(m, n, iic), c00, c10);
-            if (ye) load_pair(qc + pidx(m, n + 1, iic), c01, c11);
-        } else {
-            c00 = QC(m, n);
-            if (ye) c01 = QC(m, n + 1);
-        }
-        if (xe) {  // coarse point and (2m, 2n-1)
-            T q0, q1;
+            load_pair(qc + pidx(m, n + 1, iic), c01, c11);
             load_pair(q + p, q0, q1);
+            load_pair(q + p2, q2, q3);
+            load_pair(res + p2, r2, r3);
+            load_pair(so + p2, s2, s3);
+            const T r1 = res[p + 1], s1 = so[p + 1];
+            const T wr = CI(m + 1, n, LR), wl = CI(m + 1, n, LL);
+            const T wa = CI(m, n + 1, LA), wb = CI(m, n + 1, LB);
+            const T wsw = CI(m + 1, n + 1, LSW), wnw = CI(m + 1, n + 1, LNW);
+            const T wne = CI(m + 1, n + 1, LNE), wse = CI(m + 1, n + 1, LSE);
+            loads_issued();
             q0 = q0 + c00;
-            const T a = CI(m + 1, n, LR) * c10 + CI(m + 1, n, LL) * c00;
-            q1 = q1 + a + R(i0 + 1, j0, p + 1);
+            const T a = wr * c10 + wl * c00;
+            q1 = q1 + a + r1 / s1;
+            const T b = wa * c01 + wb * c00;
+            q2 = q2 + b + r2 / s2;
+            T c = wsw * c00;
+            c = c + wnw * c01;
+            c = c + wne * c11;
+            c = c + wse * c10;
+            q3 = q3 + c + r3 / s3;
             store_pair(q + p, q0, q1);
-        } else {
-            q[p] = q[p] + c00;
+            store_pair(q + p2, q2, q3);
+            return;
         }
-        if (ye) {  // (2m-1, 2n) and (2m, 2n)
-            const std::size_t p2 = p + iif;
-            const T a = CI(m, n + 1, LA) * c01 + CI(m, n + 1, LB) * c00;
-            if (xe) {
-                T q2, q3, r2, r3, s2, s3;
-                load_pair(q + p2, q2, q3);
-                load_pair(res + p2, r2, r3);
-                load_pair(so + p2, s2, s3);
-                q2 = q2 + a + ((i0 > iif - 2 || j0 + 1 > jjf - 2) ? r2 : r2 / s2);
-                T b = CI(m + 1, n + 1, LSW) * c00;
-                b = b + CI(m + 1, n + 1, LNW) * c01;
-                b = b + CI(m + 1, n + 1, LNE) * c11;
-                b = b + CI(m + 1, n + 1, LSE) * c10;
-                q3 = q3 + b + ((i0 + 1 > iif - 2 || j0 + 1 > jjf - 2) ? r3 : r3 / s3);
-                store_pair(q + p2, q2, q3);
-            } else {
-                q[p2] = q[p2] + a + R(i0, j0 + 1, p2);
-            }
-        }
-        return;
     }
-    const T q00 = QC(m, n);
-    {  // coarse point
-        const std::size_t p = pidx(i0, j0, iif);
-        q[p] = q[p] + q00;
-    }
-    if (xe) {  // (2m, 2n-1): between coarse (m, n) and (m+1, n)
-        const std::size_t p = pidx(i0 + 1, j0, iif);
-        const T a = CI(m + 1, n, LR) * QC(m + 1, n) + CI(m + 1, n, LL) * q00;
-        q[p] = q[p] + a + R(i0 + 1, j0, p);
-    }
-    if (ye) {  // (2m-1, 2n): between coarse (m, n) and (m, n+1)
-        const std::size_t p = pidx(i0, j0 + 1, iif);
-        const T a = CI(m, n + 1, LA) * QC(m, n + 1) + CI(m, n + 1, LB) * q00;
-        q[p] = q[p] + a + R(i0, j0 + 1, p);
-    }
-    if (xe && ye) {  // (2m, 2n): the cell of coarse (m..m+1, n..n+1)
-        const std::size_t p = pidx(i0 + 1, j0 + 1, iif);
-        T a = CI(m + 1, n + 1, LSW) * q00;
-        a = a + CI(m + 1, n + 1, LNW) * QC(m, n + 1);
-        a = a + CI(m + 1, n + 1, LNE) * QC(m + 1, n + 1);
-        a = a + CI(m + 1, n + 1, LSE) * QC(m + 1, n);
-        q[p] = q[p] + a + R(i0 + 1, j0 + 1, p);
-    }
+    // where a point does not exist, its operands are those of its neighbour in the block and its
+    // result is dropped, so that all loads come before the first branch
+    const int mx = m + (xe ? 1 : 0), ny = n + (ye ? 1 : 0);
+    const std::size_t p0 = pidx(i0, j0, iif), p1 = p0 + (xe ? 1 : 0);
+    const std::size_t p2 = p0 + (ye ? iif : 0), p3 = p2 + (xe ? 1 : 0);
+    const T c00 = QC(m, n), c10 = QC(mx, n), c01 = QC(m, ny), c11 = QC(mx, ny);
+    T q0 = q[p0], q1 = q[p1], q2 = q[p2], q3 = q[p3];
+    const T r2 = res[p2], r3 = res[p3], s2 = so[p2], s3 = so[p3];
+    const T r1 = res[p1], s1 = so[p1];
+    const T wr = CI(mx, n, LR), wl = CI(mx, n, LL);
+    const T wa = CI(m, ny, LA), wb = CI(m, ny, LB);
+    const T wsw = CI(mx, ny, LSW), wnw = CI(mx, ny, LNW);
+    const T wne = CI(mx, ny, LNE), wse = CI(mx, ny, LSE);
+    loads_issued();
+    // a ghost point reached by an even extent takes the raw res
+    auto R = [&](int i, int j, T r, T s) { return (i > iif - 2 || j > jjf - 2) ? r : r / s; };
+    q0 = q0 + c00;  // coarse point
+    const T a = wr * c10 + wl * c00;  // (2m, 2n-1): between coarse (m, n) and (m+1, n)
+    q1 = q1 + a + R(i0 + 1, j0, r1, s1);
+    const T b = wa * c01 + wb * c00;  // (2m-1, 2n): between coarse (m, n) and (m, n+1)
+    q2 = q2 + b + R(i0, j0 + 1, r2, s2);
+    T c = wsw * c00;  // (2m, 2n): the cell of coarse (m..m+1, n..n+1)
+    c = c + wnw * c01;
+    c = c + wne * c11;
+    c = c + wse * c10;
+    q3 = q3 + c + R(i0 + 1, j0 + 1, r3, s3);
+    q[p0] = q0;
+    if (xe) q[p1] = q1;
+    if (ye) q[p2] = q2;
+    if (xe && ye) q[p3] = q3;
 }
 
 // The coarsest level's band solve, q = A^-1 qf, by the threads tid < nt of one workgroup.  Where

@@ -87,8 +87,9 @@ __global__ __launch_bounds__(256) void residual_k(const T *__restrict__ so, cons
     double sq = 0.0;
     if (i <= ii - 2 && j <= jj - 2) {
         const std::size_t p = pidx(i, j, ii);
+        const T c = so[p], x = q[p];
         T r = apply_offdiag<T, NINE>(so, P, q, p, ii, qf[p]);
-        r = r - so[p] * q[p];
+        r = r - c * x;
         res[p] = r;
         if (NORM) sq = (double)r * (double)r;
     }
@@ -251,8 +252,9 @@ __global__ __launch_bounds__(256) void gs_colour_k(const T *__restrict__ so, con
     q += bz * P;
     sor += bo * 2 * P;
     const std::size_t p = pidx(i, j, ii);
-    T v = apply_offdiag<T, NINE>(so, P, q, p, ii, qf[p]);
-    q[p] = v * sor[P + p];
+    const T rec = sor[P + p];
+    const T v = apply_offdiag<T, NINE>(so, P, q, p, ii, qf[p]);
+    q[p] = v * rec;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -303,15 +305,23 @@ __global__ __launch_bounds__(64 * rc_rows<T>) void restrict_cycle_k(const T *__r
     qc += bz * Pc;
     xc += bz * Pc;
     const int tx = threadIdx.x % 64, ic = ic0 + tx;
+    constexpr int U = 16 / rc_rows<T>;
+    restrict_ops<T> o[U];  // of the thread's rows, clamped into the interior
 #pragma unroll
-    for (int u = 0; u < 16 / rc_rows<T>; ++u) {
+    for (int u = 0; u < U; ++u) {
+        const int jc = jc0 + threadIdx.x / 64 + u * rc_rows<T>;
+        load_restrict(o[u], ci, q, iif, iic, Pc, min(max(ic, 1), iic - 2), min(max(jc, 1), jjc - 2));
+    }
+    loads_issued();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
         const int k = threadIdx.x / 64 + u * rc_rows<T>;
         const int jc = jc0 + k;
         if (ic >= iic || jc >= jjc) continue;
         const std::size_t pc = pidx(ic, jc, iic);
         xc[pc] = T(0);
         if (ic >= 1 && ic <= iic - 2 && jc >= 1 && jc <= jjc - 2) {
-            const T v = restrict_point<T>(ci, q, iif, iic, Pc, ic, jc);
+            const T v = sum_restrict(o[u]);
             qc[pc] = v;
             tile[k][tx] = v;
         }

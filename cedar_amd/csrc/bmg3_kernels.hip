@@ -56,20 +56,28 @@ __device__ inline double lumpd(double dp, double s, double ep) {
     return dp + (s - dp) * dmax2(s - (1.0 + ep) * dp, 0.0) / (fabs(s - (1.0 + ep) * dp) + EMACH);
 }
 
-#define CDR3_ADD(si, sj, sk, d, oi, oj, ok)                                                       \
-    v = v + S3(i + (si), j + (sj), k + (sk), d) * Q3(q, i + (oi), j + (oj), k + (ok));
-
-// qf + sum of the off-diagonal terms at Fortran point (i, j, k)
+// qf + sum of the off-diagonal terms at Fortran point (i, j, k).  Every operand is on its way
+// before the first product (loads_issued of the 2D path has the reason).
 template <typename T, bool NINE>
 __device__ inline T offdiag3(const T *__restrict__ so, const T *__restrict__ qf,
                              const T *__restrict__ q, int i, int j, int k, int ii, int jj,
                              std::size_t P) {
+    constexpr int N = NINE ? 26 : 6;
+    T c[N], x[N];
+    int n = 0;
     T v = Q3(qf, i, j, k);
+#define CDR3_LOAD(si, sj, sk, d, oi, oj, ok)                                                      \
+    c[n] = S3(i + (si), j + (sj), k + (sk), d);                                                   \
+    x[n++] = Q3(q, i + (oi), j + (oj), k + (ok));
     if (NINE) {
-        NB27_LIST(CDR3_ADD)
+        NB27_LIST(CDR3_LOAD)
     } else {
-        NB7_LIST(CDR3_ADD)
+        NB7_LIST(CDR3_LOAD)
     }
+#undef CDR3_LOAD
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < N; ++t) v = v + c[t] * x[t];
     return v;
 }
 
@@ -104,7 +112,8 @@ __global__ __launch_bounds__(256) void residual3_k(const T *__restrict__ so, con
     const std::size_t P = (std::size_t)ii * jj * kk;
     double sq = 0.0;
     if (i <= ii - 1 && j <= jj - 1) {
-        const T r = offdiag3<T, NINE>(so, qf, q, i, j, k, ii, jj, P) - S3(i, j, k, kp) * Q3(q, i, j, k);
+        const T c = S3(i, j, k, kp), x = Q3(q, i, j, k);
+        const T r = offdiag3<T, NINE>(so, qf, q, i, j, k, ii, jj, P) - c * x;
         Q3(res, i, j, k) = r;
         sq = (double)r * (double)r;
     }
@@ -177,7 +186,8 @@ __global__ __launch_bounds__(256) void gs27_colour_k(const T *__restrict__ so, c
     const int k = pk + 2 * bz;
     if (i > ii - 1 || j > jj - 1 || k > kk - 1) return;
     const std::size_t P = (std::size_t)ii * jj * kk;
-    Q3(q, i, j, k) = offdiag3<T, true>(so, qf, q, i, j, k, ii, jj, P) * sor[P + ix3(i, j, k, ii, jj)];
+    const T rec = sor[P + ix3(i, j, k, ii, jj)];
+    Q3(q, i, j, k) = offdiag3<T, true>(so, qf, q, i, j, k, ii, jj, P) * rec;
 }
 
 template <typename T>
@@ -190,7 +200,8 @@ __global__ __launch_bounds__(256) void gs7_colour_k(const T *__restrict__ so, co
     const int i = (j + k + pts) % 2 + 2 + 2 * (int)(blockIdx.x * 64 + (threadIdx.x % 64));
     if (i > ii - 1) return;
     const std::size_t P = (std::size_t)ii * jj * kk;
-    Q3(q, i, j, k) = offdiag3<T, false>(so, qf, q, i, j, k, ii, jj, P) * sor[P + ix3(i, j, k, ii, jj)];
+    const T rec = sor[P + ix3(i, j, k, ii, jj)];
+    Q3(q, i, j, k) = offdiag3<T, false>(so, qf, q, i, j, k, ii, jj, P) * rec;
 }
 
 // ------------------------------------------------------------------------------------------

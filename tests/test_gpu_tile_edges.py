@@ -178,3 +178,28 @@ def test_fused_cycle_memory_modes(nx, ny, relax, precision):
     x, h = C.Solver(so, **kw).solve(b)
     y, g = C.Solver(so, fused_coarse=False, **kw).solve(b)
     assert torch.equal(x, y) and np.array_equal(h, g)
+
+
+# FP32 transfers move blocks inside the grid as pairs and those at its last points one by one: the
+# smallest grids, odd and even extents, one tile of 64 x 16 coarse points and a remainder.  Every
+# result is a sum of at most 9 products with one quotient, so at most 12 roundings of 2^-24 of the
+# sum of its terms' sizes.
+@pytest.mark.parametrize("nx,ny", [(3, 3), (4, 3), (3, 4), (5, 6), (31, 33), (127, 17), (128, 34),
+                                   (129, 65), (130, 66)])
+@pytest.mark.parametrize("ns", [3, 5])
+def test_fp32_transfers(nx, ny, ns):
+    import cedar_amd as C
+    print(f"\nFP32 transfers {nx}x{ny} ns={ns}", flush=True)
+    rng = np.random.default_rng(5 * nx + ny + ns)
+    r32 = lambda a: np.asarray(a, dtype=np.float32).astype(np.float64)
+    so = r32(_so2(rng, nx, ny, ns))
+    ci = r32(O.setup_interp(so))
+    q, res, qc = (r32(rng.standard_normal(s)) for s in (so.shape[1:], so.shape[1:], ci.shape[1:]))
+    f = lambda a: dev(a, torch.float32)
+    g, h = f(q), torch.zeros(ci.shape[1:], dtype=torch.float32, device="cuda")
+    C.interp_add(g, f(qc), f(res), f(so), f(ci))
+    C.restrict(f(ci), f(res), h)
+    size = [O.interp_add(*map(np.abs, (q, qc, res, so, ci)))[0], O.restrict(abs(ci), abs(res))]
+    want = [O.interp_add(q, qc, res, so, ci)[0], O.restrict(ci, res)]
+    for got, w, s in zip((host(g), host(h)), want, size):
+        assert (np.abs(got - w) <= 12 * 2.0 ** -24 * np.abs(s)).all()
