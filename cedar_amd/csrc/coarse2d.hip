@@ -23,11 +23,15 @@ namespace {
 // A chain of 60 to 150 short steps, each waiting for the one before: bound by the latency of a
 // step.  The arrays sit in LDS as far as they fit, addressed as LDS (what lies where is a template
 // parameter and no pointer may be either, or every access becomes a flat one that waits for memory
-// and LDS alike); a step's threads are dealt to exactly the points it updates, by shifts; a first
-// level whose operator stays in memory has the operands of its next sweep loaded during the
-// current one, y-lines from a transposed copy so that they arrive with unit stride.  V(2,1) point
-// relaxation in FP64 from 32^2 down: 62 us with flat accesses, 46 with the first level's operator in
-// memory, 38 with only the planes point relaxation needs on chip; from 64^2 down 127, 108, 80.
+// and LDS alike); a step's threads are dealt to exactly the points it updates, by shifts; the
+// operands of a smoothing are loaded once and held in registers where they fit, y-lines of a
+// first level in memory from a transposed copy so that they arrive with unit stride; a wavefront
+// without points in a step goes straight to its barrier (four wavefronts share a SIMD, and what
+// the idle ones executed on the way was most of a small level's step); the arrays come in as
+// chunks dealt over the wavefronts, all of a chunk's loads in flight.  V(2,1) point relaxation
+// in FP64 from 32^2 down: 62 us with flat accesses, 38 addressed as LDS, 33 as it is; from 64^2
+// down 127, 80, 69; xy-lines in FP32 from 64^2 down 83 -> 71; 12 problems, lines from 66^2 down,
+// 152 -> 120.
 
 // Operands of one element of a line (everything but the iterate): right-hand side, couplings to
 // the neighbouring lines, multipliers of the forward and backward pass, pivot.
@@ -276,55 +280,66 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
                           lv[nlev - 1].jj, tid, NT, cg_sh);
     }
     if constexpr (MODE != 0) {
+        constexpr int U = 16;  // elements of a chunk per lane
+        int job = 0;           // chunks dealt so far
+        auto copy_in = [&](const T *src, T *dst, int n) {
+            const int lane = tid % WAVE, chunks = (n + WAVE * U - 1) / (WAVE * U);
+            for (int c = (wave - job) & (NWAVE - 1); c < chunks; c += NWAVE) {
+                T v[U];
+                const int k0 = c * WAVE * U + lane;
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = src[min(k0 + u * WAVE, n - 1)];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (k0 + u * WAVE < n) dst[k0 + u * WAVE] = v[u];
+            }
+            job += chunks;
+        };
         unsigned off = 0;
         for (int l = 0; l < nlev; ++l) {
             const coarse_level<T> g = in_memory(l);
             const int P = g.ii * g.jj;
             if (MODE >= 2 && l == 0) {
                 const coarse_level<T> d = first_level();
-                const bool tr = lv[0].soT != nullptr &&
-                                (relax == CDR_RELAX_LINE_Y || relax == CDR_RELAX_LINE_XY);
-                if (tr) {
+                copy_in(g.x, d.x, P);
+                if constexpr (MODE == 2) {
+                    copy_in(g.b, d.b, P);
+                    for (int k = tid; k < P; k += NT) d.res[k] = T(0);
+                }
+                if (lv[0].soT != nullptr &&
+                    (relax == CDR_RELAX_LINE_Y || relax == CDR_RELAX_LINE_XY)) {
                     soT = global_ptr(lv[0].soT) + bo * 5 * (std::size_t)P;
                     bT = global_ptr(lv[0].bT) + bz * (std::size_t)P;
-                }
-                for (int k = tid; k < P; k += NT) {
-                    const T v = g.b[k];
-                    d.x[k] = g.x[k];
-                    if constexpr (MODE == 2) {
-                        d.b[k] = v;
-                        d.res[k] = T(0);
-                    } else {
-                        if (tr) bT[(k % g.ii) * g.jj + k / g.ii] = v;
-                    }
+                    if constexpr (MODE == 3)
+                        for (int k = tid; k < P; k += NT) bT[(k % g.ii) * g.jj + k / g.ii] = g.b[k];
                 }
             } else {
                 const coarse_level<T> d = on_chip(l, off);
-                for (int k = tid; k < 5 * P; k += NT) const_cast<T *>(d.so)[k] = g.so[k];
-                if (relax == CDR_RELAX_POINT) {
-                    for (int k = tid; k < P; k += NT) const_cast<T *>(d.sor0)[P + k] = g.sor0[P + k];
-                } else {
-                    for (int k = tid; k < 2 * P; k += NT) const_cast<T *>(d.sor0)[k] = g.sor0[k];
-                    if (nsor == 4)
-                        for (int k = tid; k < 2 * P; k += NT) const_cast<T *>(d.sor1)[k] = g.sor1[k];
-                }
-                if (CI && l > 0)
-                    for (int k = tid; k < 8 * P; k += NT) const_cast<T *>(d.ci)[k] = g.ci[k];
+                copy_in(g.so, const_cast<T *>(d.so), 5 * P);
+                if (relax == CDR_RELAX_POINT)
+                    copy_in(g.sor0 + P, const_cast<T *>(d.sor0) + P, P);
+                else
+                    copy_in(g.sor0, const_cast<T *>(d.sor0), 2 * P);
+                if (nsor == 4) copy_in(g.sor1, const_cast<T *>(d.sor1), 2 * P);
+                if (CI && l > 0) copy_in(g.ci, const_cast<T *>(d.ci), 8 * P);
                 // res and, below the first level, b start at zero as in memory: their ghosts are
                 // never written, and interp_add adds the ghost res of an even-sized level to the
                 // ghost of x
+                if (l == 0) {
+                    copy_in(g.x, d.x, P);
+                    copy_in(g.b, d.b, P);
+                }
                 for (int k = tid; k < P; k += NT) {
                     d.res[k] = T(0);
-                    d.b[k] = l == 0 ? g.b[k] : T(0);
-                    if (l == 0) d.x[k] = g.x[k];
+                    if (l > 0) d.b[k] = T(0);
                 }
             }
             off += bytes_of(l);
         }
     }
     __syncthreads();
-    // after a step that writes the iterate alone: with x on chip the operands on their way from
-    // memory need not have arrived
+    // after a step that writes on chip alone: operands on their way from memory need not have arrived
     auto x_barrier = [] {
         if constexpr (MODE == 0)
             __syncthreads();
@@ -335,6 +350,7 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
     // that holds it
     auto each = [&](int nc, int nr, auto &&f) {
         const int sh = min(log2_up(nc), 10);
+        if ((wave * WAVE) >> sh >= nr) return;
         for (int r = tid >> sh; r < nr; r += NT >> sh)
             for (int c = tid & ((1 << sh) - 1); c < nc; c += 1 << sh) f(c, r);
     };
@@ -371,178 +387,172 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
             }
             return;
         }
-        for (int t = 0; t < nrep * (xy ? 4 : 2); ++t) {
+        for (int t = 0; t < nrep * (xy ? 4 : 2); t += 2) {  // the two colours of a direction
             int dir, first;
             sweep(t, updown, dir, first);
             const int nfix = dir == 0 ? ny : nx, n = dir == 0 ? nx : ny;
-            const int nlines = first <= nfix ? (nfix - first) / 2 + 1 : 0;
             const line_src<T> src =
                 line_source<T>(d.so, d.b, xy && dir ? d.sor1 : d.sor0, d.ii, d.jj, dir, false);
             const int ws = width(n), e = tid & ((1 << ws) - 1);
+            for (int c = 0; c < 2; ++c, first = 3 - first) {
+                const int nlines = (nfix - first + 2) / 2;
+                for (int wv = wave; wv << (6 - ws) < nlines; wv += NWAVE) {
+                    const int m = lane_line(wv, ws);
+                    const bool act = m < nlines;
+                    const int L = first + 2 * (act ? m : nlines - 1);
+                    if (CH > 1 && n > WAVE) {
+                        line_ops<T> o[CH];
+#pragma unroll
+                        for (int u = 0; u < CH; ++u)
+                            load_ops(o[u], src, L, u * WAVE + e, u * WAVE + WAVE - 1 - e, n);
+                        solve_lines<T, CH>(o, d.x, d.ii, d.jj, dir, L, act, 6);
+                    } else {
+                        line_ops<T> o[1];
+                        load_ops(o[0], src, L, e, (1 << ws) - 1 - e, n);
+                        solve_lines<T, 1>(o, d.x, d.ii, d.jj, dir, L, act, ws);
+                    }
+                }
+                x_barrier();
+            }
+        }
+    };
+    // smooth() of a level so small that a thread has at most one point of a colour (64 points a
+    // side) or a wavefront one group of lines: the operands of all its sweeps are loaded before the
+    // first one and stay in registers, so that a sweep waits for the iterate alone.
+    auto smooth_points = [&](const coarse_level<T> &d, int updown) {
+        const int nrep = updown == 0 ? npre : npost;
+        const int nx = d.ii - 2, ny = d.jj - 2, P = d.ii * d.jj;
+        point_ops<T> o[4];
+        int p[4];
+        bool on[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            int pi, pj;
+            colour(t, updown, pi, pj);
+            const int nc = (nx + 1 - pi) / 2, nr = (ny + 1 - pj) / 2, sh = log2_up(nc);
+            const int ic = tid & ((1 << sh) - 1), jc = tid >> sh;
+            p[t] = (2 * jc + 1 + pj) * d.ii + 2 * ic + 1 + pi;
+            on[t] = ic < nc && jc < nr;
+            if (!on[t]) p[t] = d.ii + 1;
+        }
+        const bool work = (wave * WAVE) >> log2_up((nx + 1) / 2) < (ny + 1) / 2;
+        if (work)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) load_point(o[t], d.so, d.b, d.sor0, P, p[t], d.ii);
+        for (int r = 0; r < nrep; ++r)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (work) {
+                    const T v = relax_point(o[t], d.x, p[t], d.ii);
+                    if (on[t]) d.x[p[t]] = v;
+                }
+                x_barrier();
+            }
+    };
+    auto smooth_lines = [&](const coarse_level<T> &d, int updown) {  // at most 32 points a side
+        const int nrep = updown == 0 ? npre : npost;
+        const int nx = d.ii - 2, ny = d.jj - 2;
+        line_ops<T> o[4][1];
+        int L[4];
+        bool act[4], any[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (t >= 2 && !xy) continue;
+            int dir, first;
+            sweep(t, updown, dir, first);
+            const int n = dir == 0 ? nx : ny, nlines = ((dir == 0 ? ny : nx) - first + 2) / 2;
+            const int ws = width(n), e = tid & ((1 << ws) - 1), m = lane_line(wave, ws);
+            any[t] = wave << (6 - ws) < nlines;
+            if (!any[t]) continue;
+            act[t] = m < nlines;
+            L[t] = first + 2 * (act[t] ? m : nlines - 1);
+            load_ops(o[t][0],
+                     line_source<T>(d.so, d.b, xy && dir ? d.sor1 : d.sor0, d.ii, d.jj, dir, false),
+                     L[t], e, (1 << ws) - 1 - e, n);
+        }
+        for (int r = 0; r < nrep; ++r)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (t >= 2 && !xy) continue;
+                int dir, first;
+                sweep(t, updown, dir, first);
+                if (any[t])
+                    solve_lines<T, 1>(o[t], d.x, d.ii, d.jj, dir, L[t], act[t],
+                                      width(dir == 0 ? nx : ny));
+                x_barrier();
+            }
+    };
+    auto smooth_level = [&](const coarse_level<T> &d, int updown) {
+        if constexpr (CH == 1 && MODE != 0) {
+            if (relax == CDR_RELAX_POINT) return smooth_points(d, updown);
+            if constexpr (sizeof(T) == 4)  // FP64 operands of four sweeps do not fit the registers
+                if (max(d.ii, d.jj) - 2 <= 32) return smooth_lines(d, updown);
+        }
+        smooth(d, updown);
+    };
+    // the smoothing of a first level whose operator is in memory
+    auto smooth_first = [&](const coarse_level<T> &d, int updown) {
+        if constexpr (CH == 1) {
+            if (relax == CDR_RELAX_POINT) return smooth_points(d, updown);
+        }
+        const int nrep = updown == 0 ? npre : npost;
+        const int nx = d.ii - 2, ny = d.jj - 2;
+        if (relax == CDR_RELAX_POINT) return smooth(d, updown);
+        for (int t = 0; t < nrep * (xy ? 4 : 2); ++t) {
+            int dir, first;
+            sweep(t, updown, dir, first);
+            const int n = dir == 0 ? nx : ny, nlines = ((dir == 0 ? ny : nx) - first + 2) / 2;
+            const int ws = width(n), e = tid & ((1 << ws) - 1);
+            const bool trans = dir == 1 && soT != nullptr;
+            const T *sor = xy && dir ? d.sor1 : d.sor0;
+            line_src<T> src = line_source<T>(trans ? soT : d.so, d.b, sor, d.ii, d.jj, dir, trans);
+            if constexpr (MODE == 3)
+                if (trans) src.b = bT;
             for (int wv = wave; wv << (6 - ws) < nlines; wv += NWAVE) {
                 const int m = lane_line(wv, ws);
                 const bool act = m < nlines;
                 const int L = first + 2 * (act ? m : nlines - 1);
-                if (CH > 1 && n > WAVE) {
-                    line_ops<T> o[CH];
+                line_ops<T> o[CH];
 #pragma unroll
-                    for (int u = 0; u < CH; ++u)
-                        load_ops(o[u], src, L, u * WAVE + e, u * WAVE + WAVE - 1 - e, n);
-                    solve_lines<T, CH>(o, d.x, d.ii, d.jj, dir, L, act, 6);
-                } else {
-                    line_ops<T> o[1];
-                    load_ops(o[0], src, L, e, (1 << ws) - 1 - e, n);
-                    solve_lines<T, 1>(o, d.x, d.ii, d.jj, dir, L, act, ws);
+                for (int u = 0; u < CH; ++u) {
+                    load_ops(o[u], src, L, u * WAVE + e, u * WAVE + (1 << ws) - 1 - e, n);
+                    if constexpr (MODE == 2)
+                        if (trans) o[u].qf = d.b[(min(u * WAVE + e, n - 1) + 1) * d.ii + L];
                 }
+                if (CH > 1 && n > WAVE)
+                    solve_lines<T, CH>(o, d.x, d.ii, d.jj, dir, L, act, 6);
+                else
+                    solve_lines<T, 1>(reinterpret_cast<line_ops<T>(&)[1]>(o[0]), d.x, d.ii, d.jj, dir,
+                                      L, act, ws);
             }
             x_barrier();
         }
     };
-    // smooth() of a first level whose operator is in memory.  Up to 64 points a side a thread has at
-    // most one point of a colour and a wavefront at most two groups of lines, whose operands are
-    // loaded a sweep ahead; larger levels load them when they need them.
-    auto smooth_first = [&](const coarse_level<T> &d, int updown) {
-        const int nrep = updown == 0 ? npre : npost;
-        const int nx = d.ii - 2, ny = d.jj - 2, P = d.ii * d.jj;
-        if (relax == CDR_RELAX_POINT) {
-            if constexpr (CH > 1) {
-                smooth(d, updown);
-            } else {
-                auto point = [&](int t, int &p) {  // this thread's point of sweep t
-                    int pi, pj;
-                    colour(t, updown, pi, pj);
-                    const int nc = (nx + 1 - pi) / 2, nr = (ny + 1 - pj) / 2, sh = log2_up(nc);
-                    const int ic = tid & ((1 << sh) - 1), jc = tid >> sh;
-                    p = (2 * jc + 1 + pj) * d.ii + 2 * ic + 1 + pi;
-                    return ic < nc && jc < nr;
-                };
-                point_ops<T> cur{}, nxt{};
-                int p = 0, pn = 0;
-                bool on = point(0, p), onn = false;
-                if (on) load_point(cur, d.so, d.b, d.sor0, P, p, d.ii);
-                for (int t = 0; t < 4 * nrep; ++t) {
-                    onn = t + 1 < 4 * nrep && point(t + 1, pn);
-                    if (onn) load_point(nxt, d.so, d.b, d.sor0, P, pn, d.ii);
-                    if (on) d.x[p] = relax_point(cur, d.x, p, d.ii);
-                    x_barrier();
-                    cur = nxt;
-                    p = pn;
-                    on = onn;
-                }
-            }
-            return;
-        }
-        // two groups of lines per wavefront; FP64 has registers for the next operands of one
-        constexpr int SLOTS = 2, AHEAD = sizeof(T) == 8 ? 1 : 2;
-        // operands of this wavefront's groups of lines of sweep t
-        auto load = [&](int t, line_ops<T>(&o)[CH], int slot, int &L, bool &act, bool &any) {
-            int dir, first;
-            sweep(t, updown, dir, first);
-            const int nfix = dir == 0 ? ny : nx, n = dir == 0 ? nx : ny;
-            const int nlines = first <= nfix ? (nfix - first) / 2 + 1 : 0;
-            const int ws = width(n), e = tid & ((1 << ws) - 1), wv = wave + slot * NWAVE;
-            any = wv << (6 - ws) < nlines;
-            if (!any) return;
-            const int m = lane_line(wv, ws);
-            act = m < nlines;
-            L = first + 2 * (act ? m : nlines - 1);
-            const bool tr = dir == 1 && soT != nullptr;
-            const T *sor = xy && dir ? d.sor1 : d.sor0;
-            auto fetch = [&](const line_src<T> &src) {
-#pragma unroll
-                for (int u = 0; u < CH; ++u)
-                    load_ops(o[u], src, L, u * WAVE + e, u * WAVE + (1 << ws) - 1 - e, n);
-            };
-            // three sources whose arrays lie in different places; the transposed one of MODE 2
-            // reads b from LDS, where its order does not matter
-            line_src<T> src = line_source<T>(tr ? soT : d.so, d.b, sor, d.ii, d.jj, dir, tr);
-            if constexpr (MODE == 3) {
-                if (tr) src.b = bT;
-                fetch(src);
-            } else {
-                fetch(src);
-                if (tr)
-#pragma unroll
-                    for (int u = 0; u < CH; ++u)
-                        o[u].qf = d.b[(min(u * WAVE + e, n - 1) + 1) * d.ii + L];
-            }
-        };
-        const int total = nrep * (xy ? 4 : 2);
-        if constexpr (CH == 1) {
-            line_ops<T> cur[AHEAD][1] = {}, nxt[AHEAD][1] = {};
-            int L[AHEAD] = {}, Ln[AHEAD] = {};
-            bool act[AHEAD] = {}, actn[AHEAD] = {}, any[AHEAD] = {}, anyn[AHEAD] = {};
-#pragma unroll
-            for (int s = 0; s < AHEAD; ++s) load(0, cur[s], s, L[s], act[s], any[s]);
-            for (int t = 0; t < total; ++t) {
-                int dir, first;
-                sweep(t, updown, dir, first);
-                const int ws = width(dir == 0 ? nx : ny);
-                if (t + 1 < total)
-#pragma unroll
-                    for (int s = 0; s < AHEAD; ++s) load(t + 1, nxt[s], s, Ln[s], actn[s], anyn[s]);
-#pragma unroll
-                for (int s = 0; s < AHEAD; ++s)
-                    if (any[s]) solve_lines<T, 1>(cur[s], d.x, d.ii, d.jj, dir, L[s], act[s], ws);
-#pragma unroll
-                for (int s = AHEAD; s < SLOTS; ++s) {
-                    line_ops<T> o[1];
-                    int Lo = 0;
-                    bool acto = false, anyo = false;
-                    load(t, o, s, Lo, acto, anyo);
-                    if (anyo) solve_lines<T, 1>(o, d.x, d.ii, d.jj, dir, Lo, acto, ws);
-                }
-                x_barrier();
-#pragma unroll
-                for (int s = 0; s < AHEAD; ++s) {
-                    cur[s][0] = nxt[s][0];
-                    L[s] = Ln[s];
-                    act[s] = actn[s];
-                    any[s] = anyn[s];
-                }
-            }
-        } else {
-            for (int t = 0; t < total; ++t) {
-                int dir, first;
-                sweep(t, updown, dir, first);
-                bool any = true;
-                for (int s = 0; any; ++s) {
-                    line_ops<T> o[CH];
-                    int L = 0;
-                    bool act = false;
-                    load(t, o, s, L, act, any);
-                    const int n = dir == 0 ? nx : ny;
-                    if (!any) break;
-                    if (n > WAVE)
-                        solve_lines<T, CH>(o, d.x, d.ii, d.jj, dir, L, act, 6);
-                    else
-                        solve_lines<T, 1>(reinterpret_cast<line_ops<T>(&)[1]>(o[0]), d.x, d.ii, d.jj, dir,
-                                          L, act, width(n));
-                }
-                x_barrier();
-            }
-        }
-    };
     // going down: residual and restriction to the next level's b, whose x becomes zero
-    auto down = [&](const coarse_level<T> &F, const coarse_level<T> &C) {
+    // (res of a MODE 3 first level is in memory)
+    auto down = [&](const coarse_level<T> &F, const coarse_level<T> &C, bool first) {
         const int P = F.ii * F.jj, Pc = C.ii * C.jj;
         each(F.ii - 2, F.jj - 2, [&](int c, int r) {
             const int p = (r + 1) * F.ii + c + 1;
-            T v = apply_offdiag<T, true>(F.so, P, F.x, p, F.ii, F.b[p]);
-            F.res[p] = v - F.so[p] * F.x[p];
+            const T co = F.so[p], x = F.x[p];
+            const T v = apply_offdiag<T, true>(F.so, P, F.x, p, F.ii, F.b[p]);
+            F.res[p] = v - co * x;
         });
-        __syncthreads();
+        if (MODE == 3 && first)
+            __syncthreads();
+        else
+            x_barrier();
         each(C.ii - 2, C.jj - 2, [&](int c, int r) {
             C.b[(r + 1) * C.ii + c + 1] = restrict_point<T>(C.ci, F.res, F.ii, C.ii, Pc, c + 1, r + 1);
         });
         for (int k = tid; k < Pc; k += NT) C.x[k] = T(0);
-        __syncthreads();
+        x_barrier();
     };
     auto up = [&](const coarse_level<T> &F, const coarse_level<T> &C) {
         each(F.ii / 2, F.jj / 2, [&](int c, int r) {
-            interp_block<T>(F.x, C.x, F.res, F.so, C.ci, C.ii, C.jj, F.ii, F.jj, c + 1, r + 1);
+            interp_block<T, false>(F.x, C.x, F.res, F.so, C.ci, C.ii, C.jj, F.ii, F.jj, c + 1, r + 1);
         });
-        __syncthreads();
+        x_barrier();
     };
     // the levels l0 .. nlev - 1, all addressed alike, at off; one copy of each step for all of them
     auto cycle = [&](int l0, unsigned off) {
@@ -564,9 +574,9 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
             }
             const coarse_level<T> F = lower(l, off), C = lower(l + 1, off + bytes_of(l));
             if (rise) up(F, C);
-            smooth(F, rise ? 1 : 0);
+            smooth_level(F, rise ? 1 : 0);
             if (!rise) {
-                down(F, C);
+                down(F, C, false);
                 off += bytes_of(l);
                 ++l;
             }
@@ -580,7 +590,7 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
             if (s == 1) up(F, C);
             smooth_first(F, s);
             if (s == 0) {
-                down(F, C);
+                down(F, C, true);
                 cycle(1, off);
             }
         }
