@@ -175,7 +175,7 @@ public:
             double *bT0 = bT_target<double>(L64_[0]);
             if (bT0) k2::transpose<double>(b.p, bT0, e.jj, e.ii, stream_, nb);
             check(api2::residual_norm(A.p, A.nstncl, b.p, x.p, L64_[0].res.p, e.ii, e.jj,
-                                      work_.data(), sumsq_.data(), stream_, nb, rep_),
+                                      work_.data(), host_norm_, stream_, nb, rep_),
                   "residual_norm");
             read_norms();
             for (int p = 0; p < nb; ++p) res0[p] = std::sqrt(host_norm_[p]);
@@ -192,7 +192,7 @@ public:
                                 [&] { run_cycle<double>(L64_, x, b, bT0 != nullptr); });
                 if (masked) k2::keep_inactive(x.p, xprev_.data(), active_.data(), e.points(), nb, stream_);
                 check(api2::residual_norm(A.p, A.nstncl, b.p, x.p, L64_[0].res.p, e.ii, e.jj,
-                                          work_.data(), sumsq_.data(), stream_, nb, rep_),
+                                          work_.data(), host_norm_, stream_, nb, rep_),
                       "residual_norm");
                 read_norms();
                 if (!record(i)) break;
@@ -206,7 +206,7 @@ public:
             // level's y sweeps run through the transposed grid
             float *r32T = bT_target<float>(F);
             k2::residual_ir(A.p, A.nstncl, b_dev, x_dev, nullptr, xa, F.b.p, e.ii, e.jj,
-                            work_.data(), sumsq_.data(), stream_, nb, nullptr, rep_, r32T);
+                            work_.data(), host_norm_, stream_, nb, nullptr, rep_, r32T);
             check_hip(hipGetLastError(), "residual_ir");
             periodic_images(xa, e, nb);
             read_norms();
@@ -219,7 +219,7 @@ public:
                 });
                 push_mask();
                 k2::residual_ir(A.p, A.nstncl, b_dev, xa, F.x.p, xb, F.b.p, e.ii, e.jj,
-                                work_.data(), sumsq_.data(), stream_, nb,
+                                work_.data(), host_norm_, stream_, nb,
                                 nactive < nb ? active_.data() : nullptr, rep_, r32T);
                 check_hip(hipGetLastError(), "residual_ir");
                 std::swap(xa, xb);
@@ -266,7 +266,7 @@ private:
     } g64_, g32_;
     std::vector<level_data<double>> L64_;
     std::vector<level_data<float>> L32_;
-    dbuf<double> abd_, bbd_, work_, sumsq_, xa_, xb_, xprev_;
+    dbuf<double> abd_, bbd_, work_, xa_, xb_, xprev_;
     dbuf<int> info_, active_;
     grid_func<double> abd_g_;
     double *host_norm_ = nullptr;  // nb squared norms (pinned)
@@ -334,11 +334,9 @@ private:
         check_hip(e, "hipStreamCreateWithFlags");
     }
 
-    void read_norms() {
-        check_hip(hipMemcpyAsync(host_norm_, sumsq_.data(), sumsq_.size() * sizeof(double),
-                                 hipMemcpyDeviceToHost, stream_), "read norm");
-        check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-    }
+    // the reduction of a norm writes into host_norm_ itself (pinned, so mapped): a copy back was
+    // one more operation of 3.7 us on the device between a cycle and the host's look at it
+    void read_norms() { check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize"); }
 
     template <typename T>
     // e: extents of the level's grid functions (e.nb problems); the operator-side arrays hold
@@ -408,7 +406,6 @@ private:
         abd_ = dbuf<double>((jpn_ ? ncg : (std::size_t)ec.ii) * ncg * nops, stream_);
         bbd_ = dbuf<double>((std::size_t)ec.nx() * ec.ny() * nb, stream_);
         work_ = dbuf<double>(cdr_hip_norm_work2d(L64_[0].ext.ii, L64_[0].ext.jj) * nb, stream_);
-        sumsq_ = dbuf<double>(nb, stream_);
         active_ = dbuf<int>(nb, stream_);
         // the FP64 loop of a batch saves the iterate of a cycle in which some problems have
         // stopped, so that they keep theirs; allocated here, solve() allocates nothing

@@ -421,12 +421,12 @@ public:
             xa = xa_.data();
             xb = xb_.data();
             k3::residual_ir(F.d.A.p, F.ns, b_dev, x_dev, nullptr, xa, F.f.b.p, e.ii, e.jj, e.kk,
-                            work_.data(), sumsq_.data(), stream_);
+                            work_.data(), host_norm_, stream_);
             // the outer iterate keeps its periodic images (residual_ir writes the interior)
             if (jpn_) k3::images<double>(xa, e.ii, e.jj, e.kk, jpn_, 0, stream_);
         } else {
             k3::residual_norm(F.d.A.p, F.ns, b_dev, x_dev, F.d.res.p, e.ii, e.jj, e.kk,
-                              work_.data(), sumsq_.data(), stream_);
+                              work_.data(), host_norm_, stream_);
         }
         check_hip(hipGetLastError(), "residual");
         const double res0 = std::sqrt(read_norm2());
@@ -437,13 +437,13 @@ public:
                 k2::fill<float>(F.f.x.p, 0.0f, e.points(), stream_);
                 cycle<float>(F.f.x.p, F.f.b.p);
                 k3::residual_ir(F.d.A.p, F.ns, b_dev, xa, F.f.x.p, xb, F.f.b.p, e.ii, e.jj, e.kk,
-                                work_.data(), sumsq_.data(), stream_);
+                                work_.data(), host_norm_, stream_);
                 if (jpn_) k3::images<double>(xb, e.ii, e.jj, e.kk, jpn_, 0, stream_);
                 std::swap(xa, xb);
             } else {
                 cycle<double>(x_dev, b_dev);
                 k3::residual_norm(F.d.A.p, F.ns, b_dev, x_dev, F.d.res.p, e.ii, e.jj, e.kk,
-                                  work_.data(), sumsq_.data(), stream_);
+                                  work_.data(), host_norm_, stream_);
             }
             check_hip(hipGetLastError(), "residual");
             const double rel = std::sqrt(read_norm2()) / res0;
@@ -474,16 +474,14 @@ private:
     kernel_manager km_;
     int jpn_ = 0;  // BoxMG boundary id of set_.periodic (BMG_get_bc)
     std::vector<level3> L_;
-    dbuf<double> abd_, bbd_, work_, sumsq_, xa_, xb_;
+    dbuf<double> abd_, bbd_, work_, xa_, xb_;
     dbuf<int> info_;
     int ldab_ = 0;
     double *host_norm_ = nullptr;
     hipEvent_t ev0_{}, ev1_{};
     double setup_s_ = 0, solve_s_ = 0;
 
-    double read_norm2() {
-        check_hip(hipMemcpyAsync(host_norm_, sumsq_.data(), sizeof(double), hipMemcpyDeviceToHost,
-                                 stream_), "read norm");
+    double read_norm2() {  // written by the reduction itself (host_norm_ is pinned, so mapped)
         check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
         return *host_norm_;
     }
@@ -558,7 +556,6 @@ private:
         abd_ = dbuf<double>((std::size_t)ldab_ * n, stream_);
         bbd_ = dbuf<double>(n, stream_);
         work_ = dbuf<double>(k3::norm_partials(L_[0].e.ii, L_[0].e.jj, L_[0].e.kk), stream_);
-        sumsq_ = dbuf<double>(1, stream_);
         check_hip(hipHostMalloc(&host_norm_, sizeof(double)), "hipHostMalloc");
 
         check_hip(hipEventRecord(ev0_, stream_), "hipEventRecord");
