@@ -18,7 +18,7 @@ OBJDIR = os.path.join(HERE, "_build")
 
 SOURCES = ["lines2d.hip", "bmg2_kernels.hip", "capi2d.hip", "solver2d.cpp", "bmg3_kernels.hip", "capi3d.hip",
            "solver3d.cpp", "adjoint2d.hip", "matvec.hip", "capi_handles.cpp", "device_pool.cpp", "noalloc2d.hip",
-           "lines_per2d.hip", "gs_rows2d.hip", "gs_rows3d.hip",
+           "lines_per2d.hip", "gs_rows2d.hip", "gs_rows3d.hip", "gs_planes3d.hip",
            "coarse2d.hip", "line_setup2d.hip"]
 ARCH = os.environ.get("CEDAR_AMD_ARCH", "gfx950")
 

@@ -248,9 +248,10 @@ __global__ __launch_bounds__(256) void restrict3_k(const T *__restrict__ ci, con
 // index ranges reach the fine ghost layer for even extents (coarse index IIC = IICF1); those
 // points take the raw res there, as the reference divides res only in the interior.
 // ------------------------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void interp3_k(T *__restrict__ q, const T *__restrict__ qc,
-                                                 const T *__restrict__ res, const T *__restrict__ so,
+// TO: the interior's result goes to out (which may be res), that of ghosts into q.
+template <typename T, bool TO>
+__global__ __launch_bounds__(256) void interp3_k(T *__restrict__ q, T *out, const T *__restrict__ qc,
+                                                 const T *res, const T *__restrict__ so,
                                                  const T *__restrict__ ci, int iic, int jjc, int kkc,
                                                  int iif, int jjf, int kkf) {
     const int i = blockIdx.x * 64 + (threadIdx.x % 64) + 2;
@@ -260,20 +261,23 @@ __global__ __launch_bounds__(256) void interp3_k(T *__restrict__ q, const T *__r
     const std::size_t P = (std::size_t)iif * jjf * kkf, Pc = (std::size_t)iic * jjc * kkc;
     const int iicf1 = (iif - 2) / 2 + 2, jjcf1 = (jjf - 2) / 2 + 2, kkcf1 = (kkf - 2) / 2 + 2;
     const int imax1 = 2 * (iicf1 - 1), jmax1 = 2 * (jjcf1 - 1);
-    if (j > jmax1) return;
-    const bool keven = (k % 2) == 0;
-    if (keven) {
-        if (k > 2 * (kkc - 2) || i > imax1) return;
-    } else {
-        if (k < 3 || k > 2 * kkcf1 - 3) return;
-        if ((i % 2) == 0 ? i > 2 * (iic - 2) : (i < 3 || i > 2 * iicf1 - 3)) return;
-    }
     const bool interior = i <= iif - 1 && j <= jjf - 1 && k <= kkf - 1;
+    const bool keven = (k % 2) == 0, ie = (i % 2) == 0, je = (j % 2) == 0;
+    const std::size_t p = ix3(i, j, k, ii, jj);
+    bool on = j <= jmax1;
+    if (keven)
+        on = on && k <= 2 * (kkc - 2) && i <= imax1;
+    else
+        on = on && k >= 3 && k <= 2 * kkcf1 - 3 && (ie ? i <= 2 * (iic - 2) : i >= 3 && i <= 2 * iicf1 - 3);
+    if (!on) {
+        if (TO && interior) out[p] = q[p];
+        return;
+    }
     const T r = interior ? Q3(res, i, j, k) / S3(i, j, k, kp) : Q3(res, i, j, k);
-    T &qv = Q3(q, i, j, k);
+    T qv = q[p];
+    auto store = [&](T v) { (TO && interior ? out : q)[p] = v; };
     if (keven) {
         const int kc = k / 2 + 1;
-        const bool ie = (i % 2) == 0, je = (j % 2) == 0;
         if (ie && je) {
             qv = qv + QC3(qc, i / 2 + 1, j / 2 + 1, kc);
         } else if (!ie && je) {
@@ -292,11 +296,11 @@ __global__ __launch_bounds__(256) void interp3_k(T *__restrict__ q, const T *__r
                         CI3(ic, jc, kc, lxyse) * QC3(qc, ic, jc - 1, kc);
             qv = qv + a + r;
         }
+        store(qv);
         return;
     }
     const int kc = (k + 3) / 2;
-    const bool je = (j % 2) == 0;
-    if ((i % 2) == 0) {
+    if (ie) {
         const int ic = i / 2 + 1;
         if (je) {
             const int jc = j / 2 + 1;
@@ -325,6 +329,7 @@ __global__ __launch_bounds__(256) void interp3_k(T *__restrict__ q, const T *__r
                  CI3(ic, jc, kc, lbse) * QC3(qc, ic, jc - 1, kc - 1) + r;
         }
     }
+    store(qv);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1555,7 +1560,15 @@ template <typename T>
 void interp_add(T *q, const T *qc, const T *res, const T *so, int nstncl, const T *ci, int iic,
                 int jjc, int kkc, int iif, int jjf, int kkf, hipStream_t s) {
     (void)nstncl;
-    interp3_k<T><<<grid3(iif - 1, jjf - 1, kkf - 1), 256, 0, s>>>(q, qc, res, so, ci, iic, jjc, kkc, iif, jjf, kkf);
+    interp3_k<T, false><<<grid3(iif - 1, jjf - 1, kkf - 1), 256, 0, s>>>(q, q, qc, res, so, ci, iic, jjc,
+                                                                          kkc, iif, jjf, kkf);
+}
+
+template <typename T>
+void interp_to(T *q, T *out, const T *qc, const T *res, const T *so, const T *ci, int iic, int jjc,
+               int kkc, int iif, int jjf, int kkf, hipStream_t s) {
+    interp3_k<T, true><<<grid3(iif - 1, jjf - 1, kkf - 1), 256, 0, s>>>(q, out, qc, res, so, ci, iic, jjc,
+                                                                         kkc, iif, jjf, kkf);
 }
 
 void setup_interp(const double *so, int nstncl, double *ci, int iif, int jjf, int kkf, int iic,
@@ -1925,6 +1938,8 @@ void copy_rhs(int dir, const T *so3, int nstncl3, const T *x, const T *b, T *b2,
     template void restrict_<T>(const T *, const T *, T *, int, int, int, int, int, int, hipStream_t); \
     template void interp_add<T>(T *, const T *, const T *, const T *, int, const T *, int, int, int, \
                                 int, int, int, hipStream_t);                                        \
+    template void interp_to<T>(T *, T *, const T *, const T *, const T *, const T *, int, int, int, \
+                               int, int, int, hipStream_t);                                         \
     template void solve_cg<T>(T *, const T *, const double *, int, double *, int, int, int,         \
                               hipStream_t);                                                         \
     template void copy32<T>(int, const T *, T *, int, int, int, int, int, hipStream_t);             \

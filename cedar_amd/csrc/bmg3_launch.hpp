@@ -44,6 +44,14 @@ template <typename T>
 bool relax_gs27_rows(const T *so, const T *qf, T *q, const T *sor, int ii, int jj, int kk,
                      int updown, hipStream_t s);
 
+// A 7-point sweep in one launch, from q to out (another array).  The ghosts read are those of g and
+// no ghost is written, so a sweep to a scratch array and one back leave what two sweeps in place do.
+// gs7_sweep_pays: whether it is expected to take less time than relax_gs.
+bool gs7_sweep_pays(int ii, int jj, int kk);
+template <typename T>
+void relax_gs7_sweep(const T *so, const T *qf, const T *q, T *out, const T *g, const T *sor, int ii,
+                     int jj, int kk, int updown, hipStream_t s);
+
 template <typename T>
 void restrict_(const T *ci, const T *q, T *qc, int iif, int jjf, int kkf, int iic, int jjc,
                int kkc, hipStream_t s);
@@ -51,6 +59,10 @@ void restrict_(const T *ci, const T *q, T *qc, int iif, int jjf, int kkf, int ii
 template <typename T>
 void interp_add(T *q, const T *qc, const T *res, const T *so, int nstncl, const T *ci, int iic,
                 int jjc, int kkc, int iif, int jjf, int kkf, hipStream_t s);
+// interp_add whose result in the interior goes to out (another array than q; may be res)
+template <typename T>
+void interp_to(T *q, T *out, const T *qc, const T *res, const T *so, const T *ci, int iic, int jjc,
+               int kkc, int iif, int jjf, int kkf, hipStream_t s);
 
 void setup_interp(const double *so, int nstncl, double *ci, int iif, int jjf, int kkf, int iic,
                   int jjc, int kkc, hipStream_t s);

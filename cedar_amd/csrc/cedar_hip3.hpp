@@ -67,6 +67,12 @@ struct point_relax : kernel_base {
     virtual void setup(const stencil_op3<double> &so, relax_stencil3<double> &sor) = 0;
     virtual void run(const stencil_op3<T> &so, grid_func3<T> &x, const grid_func3<T> &b,
                      const relax_stencil3<T> &sor, Dir d) = 0;
+    // One sweep from x to out, another array; ghosts are read from g and not written.  Called where
+    // out_of_place says so.
+    virtual bool out_of_place(const stencil_op3<T> &) const { return false; }
+    virtual void run_to(const stencil_op3<T> &, const grid_func3<T> & /* x */,
+                        grid_func3<T> & /* out */, const grid_func3<T> & /* g */,
+                        const grid_func3<T> & /* b */, const relax_stencil3<T> &, Dir) {}
 };
 
 // include/cedar/kernels/plane_relax.h:11-31: setup(so) builds the plane solvers of the
@@ -106,6 +112,12 @@ struct interp_add : kernel_base {
     static const char *name() { return "interp-add (3D)"; }
     virtual void run(const prolong_op3<T> &P, const grid_func3<T> &coarse,
                      const grid_func3<T> &residual, grid_func3<T> &fine) = 0;
+    // the interior's result goes to out, which may be residual; false: nothing done
+    virtual bool run_to(const prolong_op3<T> &, const grid_func3<T> & /* coarse */,
+                        const grid_func3<T> & /* residual */, grid_func3<T> & /* fine */,
+                        grid_func3<T> & /* out */) {
+        return false;
+    }
 };
 
 // the band ABD(ldab, nx*ny*nz) is FP64 in both precisions

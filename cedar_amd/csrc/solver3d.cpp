@@ -160,6 +160,17 @@ struct hip_rbgs3 : kernels3::point_relax<T> {
             k3::relax_gs<T>(so.p, so.nstncl, b.p, x.p, sor.p, e.ii, e.jj, e.kk, (int)d, this->stream);
         launched3("relax_gs3");
     }
+    bool out_of_place(const stencil_op3<T> &so) const override {
+        return !jpn && so.nstncl == 4 && k3::gs7_sweep_pays(so.ext.ii, so.ext.jj, so.ext.kk);
+    }
+    void run_to(const stencil_op3<T> &so, const grid_func3<T> &x, grid_func3<T> &out,
+                const grid_func3<T> &g, const grid_func3<T> &b, const relax_stencil3<T> &sor,
+                Dir d) override {
+        const extents3 e = so.ext;
+        k3::relax_gs7_sweep<T>(so.p, b.p, x.p, out.p, g.p, sor.p, e.ii, e.jj, e.kk, (int)d,
+                               this->stream);
+        launched3("relax_gs3");
+    }
 };
 
 // The plane solvers of one family, per level (keyed by the level's extents, which differ from
@@ -256,6 +267,15 @@ struct hip_interp3 : kernels3::interp_add<T> {
             k3::interp_add<T>(fine.p, coarse.p, residual.p, P.fine_op->p, P.fine_op->nstncl, P.p,
                               c.ii, c.jj, c.kk, f.ii, f.jj, f.kk, this->stream);
         launched3("interp_add3");
+    }
+    bool run_to(const prolong_op3<T> &P, const grid_func3<T> &coarse, const grid_func3<T> &residual,
+                grid_func3<T> &fine, grid_func3<T> &out) override {
+        if (jpn || !P.fine_op) return false;
+        const extents3 f = fine.ext, c = coarse.ext;
+        k3::interp_to<T>(fine.p, out.p, coarse.p, residual.p, P.fine_op->p, P.p, c.ii, c.jj, c.kk,
+                         f.ii, f.jj, f.kk, this->stream);
+        launched3("interp_add3");
+        return true;
     }
 };
 
@@ -627,14 +647,34 @@ private:
         km_.run<kernels3::plane_relax<T, PD>>(L.v<T>().A, x, b, d);
     }
 
-    // smoother sequencing (include/cedar/multilevel.h:165-222)
     template <typename T>
-    void smooth(level3 &L, grid_func3<T> &x, const grid_func3<T> &b, Dir d) {
-        const int nrep = d == Dir::DOWN ? set_.nrelax_pre : set_.nrelax_post;
+    void sweep_to(lvl3v<T> &V, const grid_func3<T> &x, grid_func3<T> &out, const grid_func3<T> &g,
+                  const grid_func3<T> &b, Dir d) {
+        km_.get<kernels3::point_relax<T>>().run_to(V.A, x, out, g, b, V.sor, d);
+    }
+    template <typename T>
+    bool out_of_place(lvl3v<T> &V) {
+        return set_.relaxation == CDR_RELAX_POINT &&
+               km_.get<kernels3::point_relax<T>>().out_of_place(V.A);
+    }
+
+    // smoother sequencing (include/cedar/multilevel.h:165-222).  The level's residual is free
+    // meanwhile: out-of-place sweeps go there and back.
+    template <typename T>
+    void smooth(level3 &L, grid_func3<T> &x, const grid_func3<T> &b, Dir d, int nrep) {
         lvl3v<T> &V = L.v<T>();
+        const bool pairs = out_of_place<T>(V);
         for (int rep = 0; rep < nrep; ++rep) {
             switch (set_.relaxation) {
-            case CDR_RELAX_POINT: km_.run<kernels3::point_relax<T>>(V.A, x, b, V.sor, d); break;
+            case CDR_RELAX_POINT:
+                if (pairs && nrep - rep >= 2) {
+                    sweep_to<T>(V, x, V.res, x, b, d);
+                    sweep_to<T>(V, V.res, x, x, b, d);
+                    ++rep;
+                } else {
+                    km_.run<kernels3::point_relax<T>>(V.A, x, b, V.sor, d);
+                }
+                break;
             case CDR_RELAX_PLANE_XY: planes<T, plane_dir::xy>(L, x, b, d); break;
             case CDR_RELAX_PLANE_XZ: planes<T, plane_dir::xz>(L, x, b, d); break;
             case CDR_RELAX_PLANE_YZ: planes<T, plane_dir::yz>(L, x, b, d); break;
@@ -701,7 +741,7 @@ private:
         level3 &C = L_[l + 1];
         lvl3v<T> &fv = F.v<T>();
         lvl3v<T> &cv = C.v<T>();
-        smooth<T>(F, x, b, Dir::DOWN);
+        smooth<T>(F, x, b, Dir::DOWN, set_.nrelax_pre);
         km_.run<kernels3::residual<T>>(fv.A, x, b, fv.res);
         km_.run<kernels3::restriction<T>>(cv.P, fv.res, cv.b);
         k2::fill<T>(cv.x.p, T(0), C.e.points(), stream_);
@@ -709,8 +749,16 @@ private:
             coarse_solve<T>(cv.x, cv.b);
         else
             ncycle<T>(l + 1, cv.x, cv.b);
-        km_.run<kernels3::interp_add<T>>(cv.P, cv.x, fv.res, x);
-        smooth<T>(F, x, b, Dir::UP);
+        // an odd number of out-of-place sweeps starts from the residual's array
+        int up = set_.nrelax_post;
+        if (up % 2 == 1 && out_of_place<T>(fv) &&
+            km_.get<kernels3::interp_add<T>>().run_to(cv.P, cv.x, fv.res, x, fv.res)) {
+            sweep_to<T>(fv, fv.res, x, x, b, Dir::UP);
+            --up;
+        } else {
+            km_.run<kernels3::interp_add<T>>(cv.P, cv.x, fv.res, x);
+        }
+        smooth<T>(F, x, b, Dir::UP, up);
     }
 };
 

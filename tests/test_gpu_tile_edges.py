@@ -203,3 +203,68 @@ def test_fp32_transfers(nx, ny, ns):
     want = [O.interp_add(q, qc, res, so, ci)[0], O.restrict(ci, res)]
     for got, w, s in zip((host(g), host(h)), want, size):
         assert (np.abs(got - w) <= 12 * 2.0 ** -24 * np.abs(s)).all()
+
+
+def _cycle3(C, lv, abd, l, x, b, pre, post):
+    """One V-cycle, every sweep in place, level by level."""
+    so, ci, sor = lv[l]
+    if l == len(lv) - 1:
+        C.cdr3.solve_cg(x, b, abd)
+        return
+    for _ in range(pre):
+        C.cdr3.relax_gs(so, b, x, sor, 0)
+    res, ci = torch.zeros_like(x), lv[l + 1][1]
+    C.cdr3.residual(so, b, x, res)
+    xc, bc = torch.zeros_like(lv[l + 1][0][0]), torch.zeros_like(lv[l + 1][0][0])
+    C.cdr3.restrict(ci, res, bc)
+    _cycle3(C, lv, abd, l + 1, xc, bc, pre, post)
+    C.cdr3.interp_add(x, xc, res, so, ci)
+    for _ in range(post):
+        C.cdr3.relax_gs(so, b, x, sor, 1)
+
+
+# 7-point sweeps that take both colours in one launch: one to three groups of 62 pairs along a row,
+# the last one full, nearly full or short, odd and even; tiles of 14 rows with and without a
+# remainder, slabs likewise; couplings to the ghosts of a nonzero boundary; odd and even numbers of
+# sweeps.  The sizes are about the smallest that take this path.
+@pytest.mark.parametrize("dims", [(125, 96, 104), (126, 167, 59), (126, 65, 152), (117, 70, 152),
+                                  (249, 70, 71), (248, 94, 53), (373, 53, 62)])
+@pytest.mark.parametrize("pre,post", [(2, 1), (1, 2), (3, 0)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_gs7_sweeps(dims, pre, post, dtype):
+    import cedar_amd as C
+    print(f"\n7-point sweeps {dims} {pre},{post} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(sum(dims) + pre)
+    shape = tuple(n + 2 for n in dims[::-1])
+    rand = lambda *s: torch.rand(*s, generator=g, device="cuda", dtype=torch.float64)
+    so = torch.zeros((4,) + shape, device="cuda", dtype=torch.float64)
+    so[0, 1:-1, 1:-1, 1:-1] = 7.0
+    so[1, 1:-1, 1:-1, 1:] = 0.1 + 0.9 * rand(shape[0] - 2, shape[1] - 2, shape[2] - 1)
+    so[2, 1:-1, 1:, 1:-1] = 0.1 + 0.9 * rand(shape[0] - 2, shape[1] - 1, shape[2] - 2)
+    so[3, 1:, 1:-1, 1:-1] = 0.1 + 0.9 * rand(shape[0] - 1, shape[1] - 2, shape[2] - 2)
+    b, x = rand(*shape) - 0.5, rand(*shape) - 0.5
+    f64 = dtype == torch.float64
+    s = C.Solver3(so, nrelax_pre=pre, nrelax_post=post, maxiter=1, tol=1e-30,
+                  precision="f64" if f64 else "mixed")
+    lv = []
+    for l in range(s.nlevels):
+        a, ci = s.level_arrays(l)
+        a = dev(a)
+        sor = torch.zeros((2,) + tuple(a.shape[1:]), device="cuda", dtype=torch.float64)
+        C.cdr3.setup_recip(a, sor)
+        lv.append(tuple(None if v is None else v.to(dtype)
+                        for v in (a, None if ci is None else dev(ci), sor)))
+        abd = C.cdr3.setup_cg(a) if l == s.nlevels - 1 else None
+    want, got = x.clone(), x.clone()
+    if f64:
+        s.vcycle(got, b)
+        _cycle3(C, lv, abd, 0, want, b, pre, post)
+    else:
+        s.solve(b, got)
+        r = torch.zeros_like(b)
+        C.cdr3.residual(so, b, x, r)
+        e = torch.zeros_like(r, dtype=dtype)
+        _cycle3(C, lv, abd, 0, e, r.to(dtype), pre, post)
+        inner = (slice(1, -1),) * 3  # the outer iterate's ghosts are those of its own arrays
+        want, got = (want + e.double())[inner], got[inner]
+    assert torch.equal(got, want)
