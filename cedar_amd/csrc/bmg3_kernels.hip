@@ -823,12 +823,27 @@ __device__ inline double row_weight(const row_ctx &c) {
     }
 }
 
-template <bool NINE, int F, int O, int... T>
+// entries of the row that part PART of PARTS forms
+template <int PARTS, int PART>
+constexpr bool row_part(int t) {
+    return t % PARTS == PART;
+}
+// whether f + o (x, y, z from C) interpolates from C + D of entry T
+template <int T>
+constexpr bool row_reaches(int x, int y, int z) {
+    using D = row_dir<T>;
+    const int gx = x - 2 * D::x, gy = y - 2 * D::y, gz = z - 2 * D::z;
+    return gx >= -1 && gx <= 1 && gy >= -1 && gy <= 1 && gz >= -1 && gz <= 1;
+}
+
+template <bool NINE, int PARTS, int PART, int F, int O, int... T>
 __device__ inline void row_neighbour(const row_ctx &c, double (&inner)[14],
                                      std::integer_sequence<int, T...>) {
     constexpr int fx = F % 3 - 1, fy = F / 3 % 3 - 1, fz = F / 9 - 1;
     constexpr int ox = O % 3 - 1, oy = O / 3 % 3 - 1, oz = O / 9 - 1;
-    if constexpr (NINE || (ox != 0) + (oy != 0) + (oz != 0) <= 1) {
+    constexpr bool any =
+        ((row_part<PARTS, PART>(T) && row_reaches<T>(fx + ox, fy + oy, fz + oz)) || ...);
+    if constexpr (any && (NINE || (ox != 0) + (oy != 0) + (oz != 0) <= 1)) {
         const bool ok = c.vx[fx + ox + 2] && c.vy[fy + oy + 2] && c.vz[fz + oz + 2];
         double a = c.so[(std::size_t)(A_PL[O] - 1) * c.P +
                         (c.zf[fz + A_SK[O] + 1] + c.yf[fy + A_SJ[O] + 1] + c.xf[fx + A_SI[O] + 1])];
@@ -837,7 +852,7 @@ __device__ inline void row_neighbour(const row_ctx &c, double (&inner)[14],
             [&] {
                 using D = row_dir<T>;
                 constexpr int gx = fx + ox - 2 * D::x, gy = fy + oy - 2 * D::y, gz = fz + oz - 2 * D::z;
-                if constexpr (gx >= -1 && gx <= 1 && gy >= -1 && gy <= 1 && gz >= -1 && gz <= 1) {
+                if constexpr (row_part<PARTS, PART>(T) && row_reaches<T>(fx + ox, fy + oy, fz + oz)) {
                     const double t = a * row_weight<D::x, D::y, D::z, gx, gy, gz>(c);
                     inner[T] += ok ? t : 0.0;  // a point outside carries no unknown
                 }
@@ -846,34 +861,84 @@ __device__ inline void row_neighbour(const row_ctx &c, double (&inner)[14],
     }
 }
 
-template <bool NINE, int F, int... O>
+template <bool NINE, int PARTS, int PART, int F, int... O>
 __device__ inline void row_fine_point(const row_ctx &c, double (&sum)[14],
                                       std::integer_sequence<int, O...>) {
     constexpr int fx = F % 3 - 1, fy = F / 3 % 3 - 1, fz = F / 9 - 1;
     if (!(c.vx[fx + 2] && c.vy[fy + 2] && c.vz[fz + 2])) return;
     double inner[14] = {0.0};
-    (row_neighbour<NINE, F, O>(c, inner, std::make_integer_sequence<int, 14>{}), ...);
+    (row_neighbour<NINE, PARTS, PART, F, O>(c, inner, std::make_integer_sequence<int, 14>{}), ...);
     const double w = row_weight<0, 0, 0, fx, fy, fz>(c);
 #pragma unroll
-    for (int t = 0; t < 14; ++t) sum[t] += w * inner[t];  // a direction out of reach adds zero
+    for (int t = 0; t < 14; ++t)
+        if (row_part<PARTS, PART>(t)) sum[t] += w * inner[t];  // a direction out of reach adds zero
 }
 
-template <bool NINE, int... F>
+template <bool NINE, int PARTS, int PART, int... F>
 __device__ inline void row_sums(const row_ctx &c, double (&sum)[14],
                                 std::integer_sequence<int, F...>) {
-    (row_fine_point<NINE, F>(c, sum, std::make_integer_sequence<int, 27>{}), ...);
+    (row_fine_point<NINE, PARTS, PART, F>(c, sum, std::make_integer_sequence<int, 27>{}), ...);
 }
 
 // One thread per coarse point C: its row, each entry stored at the point g = C - a where the
-// plane keeps it (zero where g couples a point outside the grid).
-template <bool NINE>
+// plane keeps it (zero where g couples a point outside the grid).  A row is a chain of some 2000
+// loads, 100 to 140 us however few the points.  Levels of at most 256 workgroups deal the 14 entries of
+// a row to PARTS = 7 workgroups each, which read a few of its operands (25^3 145 -> 95 us, 13^3
+// 145 -> 44); at 50^3 that reads too much again (355 -> 450).
+template <bool NINE, int PARTS, int... PART>
+__device__ inline void row_parts(int part, const row_ctx &c, double (&sum)[14],
+                                 std::integer_sequence<int, PART...>) {
+    ((part == PART ? row_sums<NINE, PARTS, PART>(c, sum, std::make_integer_sequence<int, 27>{})
+                   : void()),
+     ...);
+}
+
+// One thread per coarse point C: its row, each entry stored at the point g = C - a where the
+// plane keeps it (zero where g couples a point outside the grid).  A row is a chain of some 2000
+// loads, 100 to 140 us however few the points.  Levels of at most 256 workgroups deal the 14 entries of
+// a row to PARTS = 7 workgroups each, which read a few of its operands (25^3 145 -> 95 us, 13^3
+// 145 -> 44); at 50^3 that reads too much again (355 -> 450).
+template <bool NINE, int PARTS, int PART>
+__device__ inline void row_of(const row_ctx &c, double *soc, int ic, int jc, int kc,
+                              int iic, int jjc, int kkc) {
+    double sum[14] = {0.0};
+    row_sums<NINE, PARTS, PART>(c, sum, std::make_integer_sequence<int, 27>{});
+    const std::size_t Pc = c.Pc, pc = ix3(ic, jc, kc, iic, jjc);
+    if (row_part<PARTS, PART>(13)) soc[pc] = sum[13];
+#pragma unroll
+    for (int t = 0; t < 13; ++t) {
+        if (!row_part<PARTS, PART>(t)) continue;
+        const int ax = CP_A[t][0], ay = CP_A[t][1], az = CP_A[t][2];
+        const int gx = ic - ax, gy = jc - ay, gz = kc - az;  // where the coupling is kept
+        double *d = soc + (std::size_t)(CP_D[t] - 1) * Pc;
+        if (gx <= iic - 1 && gy <= jjc - 1 && gz <= kkc - 1)
+            d[ix3(gx, gy, gz, iic, jjc)] =
+                (gx + CP_B[t][0] >= 2 && gy + CP_B[t][1] >= 2 && gz + CP_B[t][2] >= 2) ? -sum[t] : 0.0;
+        // no row reaches the points on the low side of a coupling whose a lies outside
+        if (ic + ax < 2 || jc + ay < 2 || kc + az < 2) d[pc] = 0.0;
+    }
+}
+
+template <bool NINE, int PARTS, int... PART>
+__device__ inline void row_parts(int part, const row_ctx &c, double *soc, int ic, int jc,
+                                 int kc, int iic, int jjc, int kkc,
+                                 std::integer_sequence<int, PART...>) {
+    ((part == PART ? row_of<NINE, PARTS, PART>(c, soc, ic, jc, kc, iic, jjc, kkc) : void()), ...);
+}
+
+// One thread per coarse point C: its row, each entry stored at the point g = C - a where the
+// plane keeps it (zero where g couples a point outside the grid).  A row is a chain of some 2000
+// loads, 100 to 140 us however few the points.  Levels of at most 256 workgroups deal the 14 entries of
+// a row to PARTS = 7 workgroups each, which read a few of its operands (25^3 145 -> 95 us, 13^3
+// 145 -> 44); at 50^3 that reads too much again (355 -> 450).
+template <bool NINE, int PARTS>
 __global__ __launch_bounds__(256) void galerkin3_k(const double *__restrict__ so,
                                                    const double *__restrict__ ci,
                                                    double *__restrict__ soc, int iif, int jjf, int kkf,
                                                    int iic, int jjc, int kkc) {
     const int ic = blockIdx.x * 64 + (threadIdx.x % 64) + 2;
     const int jc = blockIdx.y * 4 + (threadIdx.x / 64) + 2;
-    const int kc = blockIdx.z + 2;
+    const int kc = blockIdx.z / PARTS + 2;
     if (ic > iic - 1 || jc > jjc - 1) return;
     row_ctx c{so, ci, (std::size_t)iif * jjf * kkf, (std::size_t)iic * jjc * kkc};
     const int X0 = 2 * (ic - 1), Y0 = 2 * (jc - 1), Z0 = 2 * (kc - 1);
@@ -895,12 +960,14 @@ __global__ __launch_bounds__(256) void galerkin3_k(const double *__restrict__ so
         c.vy[p + 2] = Y0 + p >= 2 && Y0 + p <= jjf - 1;
         c.vz[p + 2] = Z0 + p >= 2 && Z0 + p <= kkf - 1;
     }
+    const int part = PARTS > 1 ? (int)(blockIdx.z % PARTS) : 0;
     double sum[14] = {0.0};
-    row_sums<NINE>(c, sum, std::make_integer_sequence<int, 27>{});
+    row_parts<NINE, PARTS>(part, c, sum, std::make_integer_sequence<int, PARTS>{});
     const std::size_t Pc = c.Pc, pc = ix3(ic, jc, kc, iic, jjc);
-    soc[pc] = sum[13];
+    if (13 % PARTS == part) soc[pc] = sum[13];
 #pragma unroll
     for (int t = 0; t < 13; ++t) {
+        if (t % PARTS != part) continue;
         const int ax = CP_A[t][0], ay = CP_A[t][1], az = CP_A[t][2];
         const int gx = ic - ax, gy = jc - ay, gz = kc - az;  // where the coupling is kept
         double *d = soc + (std::size_t)(CP_D[t] - 1) * Pc;
@@ -1594,10 +1661,16 @@ void setup_interp(const double *so, int nstncl, double *ci, int iif, int jjf, in
 void setup_galerkin(const double *so, int nstncl, const double *ci, double *soc, int iif, int jjf,
                     int kkf, int iic, int jjc, int kkc, hipStream_t s) {
     const dim3 g = grid3(iic - 2, jjc - 2, kkc - 2);
-    if (nstncl == 14)
-        galerkin3_k<true><<<g, 256, 0, s>>>(so, ci, soc, iif, jjf, kkf, iic, jjc, kkc);
+    const dim3 g7(g.x, g.y, g.z * 7);
+    const bool split = (std::size_t)g.x * g.y * g.z <= 256;
+    if (nstncl == 14 && split)
+        galerkin3_k<true, 7><<<g7, 256, 0, s>>>(so, ci, soc, iif, jjf, kkf, iic, jjc, kkc);
+    else if (nstncl == 14)
+        galerkin3_k<true, 1><<<g, 256, 0, s>>>(so, ci, soc, iif, jjf, kkf, iic, jjc, kkc);
+    else if (split)
+        galerkin3_k<false, 7><<<g7, 256, 0, s>>>(so, ci, soc, iif, jjf, kkf, iic, jjc, kkc);
     else
-        galerkin3_k<false><<<g, 256, 0, s>>>(so, ci, soc, iif, jjf, kkf, iic, jjc, kkc);
+        galerkin3_k<false, 1><<<g, 256, 0, s>>>(so, ci, soc, iif, jjf, kkf, iic, jjc, kkc);
 }
 
 int cg_bandwidth(int ii, int jj) { return (ii - 2) * (jj - 1) + 1; }

@@ -43,9 +43,10 @@ def test_periodic_lines(nx, ny, mask, ns):
 
 
 # coarse rows of 64 points, one less and one more; the smallest grids; even extents, whose last
-# fine points lie beyond the last coarse one
+# fine points lie beyond the last coarse one; a level of more than 256 workgroups (one point's
+# whole row per thread there, parts of it below)
 @pytest.mark.parametrize("dims", [(3, 3, 3), (4, 3, 5), (125, 5, 4), (127, 6, 5), (128, 4, 9),
-                                  (129, 9, 6), (131, 3, 3), (6, 129, 5)])
+                                  (129, 9, 6), (131, 3, 3), (6, 129, 5), (6, 260, 66)])
 @pytest.mark.parametrize("ns", [4, 14])
 def test_galerkin3(dims, ns):
     import cedar_amd as C
