@@ -880,50 +880,12 @@ __device__ inline void row_sums(const row_ctx &c, double (&sum)[14],
     (row_fine_point<NINE, PARTS, PART, F>(c, sum, std::make_integer_sequence<int, 27>{}), ...);
 }
 
-// One thread per coarse point C: its row, each entry stored at the point g = C - a where the
-// plane keeps it (zero where g couples a point outside the grid).  A row is a chain of some 2000
-// loads, 100 to 140 us however few the points.  Levels of at most 256 workgroups deal the 14 entries of
-// a row to PARTS = 7 workgroups each, which read a few of its operands (25^3 145 -> 95 us, 13^3
-// 145 -> 44); at 50^3 that reads too much again (355 -> 450).
 template <bool NINE, int PARTS, int... PART>
 __device__ inline void row_parts(int part, const row_ctx &c, double (&sum)[14],
                                  std::integer_sequence<int, PART...>) {
     ((part == PART ? row_sums<NINE, PARTS, PART>(c, sum, std::make_integer_sequence<int, 27>{})
                    : void()),
      ...);
-}
-
-// One thread per coarse point C: its row, each entry stored at the point g = C - a where the
-// plane keeps it (zero where g couples a point outside the grid).  A row is a chain of some 2000
-// loads, 100 to 140 us however few the points.  Levels of at most 256 workgroups deal the 14 entries of
-// a row to PARTS = 7 workgroups each, which read a few of its operands (25^3 145 -> 95 us, 13^3
-// 145 -> 44); at 50^3 that reads too much again (355 -> 450).
-template <bool NINE, int PARTS, int PART>
-__device__ inline void row_of(const row_ctx &c, double *soc, int ic, int jc, int kc,
-                              int iic, int jjc, int kkc) {
-    double sum[14] = {0.0};
-    row_sums<NINE, PARTS, PART>(c, sum, std::make_integer_sequence<int, 27>{});
-    const std::size_t Pc = c.Pc, pc = ix3(ic, jc, kc, iic, jjc);
-    if (row_part<PARTS, PART>(13)) soc[pc] = sum[13];
-#pragma unroll
-    for (int t = 0; t < 13; ++t) {
-        if (!row_part<PARTS, PART>(t)) continue;
-        const int ax = CP_A[t][0], ay = CP_A[t][1], az = CP_A[t][2];
-        const int gx = ic - ax, gy = jc - ay, gz = kc - az;  // where the coupling is kept
-        double *d = soc + (std::size_t)(CP_D[t] - 1) * Pc;
-        if (gx <= iic - 1 && gy <= jjc - 1 && gz <= kkc - 1)
-            d[ix3(gx, gy, gz, iic, jjc)] =
-                (gx + CP_B[t][0] >= 2 && gy + CP_B[t][1] >= 2 && gz + CP_B[t][2] >= 2) ? -sum[t] : 0.0;
-        // no row reaches the points on the low side of a coupling whose a lies outside
-        if (ic + ax < 2 || jc + ay < 2 || kc + az < 2) d[pc] = 0.0;
-    }
-}
-
-template <bool NINE, int PARTS, int... PART>
-__device__ inline void row_parts(int part, const row_ctx &c, double *soc, int ic, int jc,
-                                 int kc, int iic, int jjc, int kkc,
-                                 std::integer_sequence<int, PART...>) {
-    ((part == PART ? row_of<NINE, PARTS, PART>(c, soc, ic, jc, kc, iic, jjc, kkc) : void()), ...);
 }
 
 // One thread per coarse point C: its row, each entry stored at the point g = C - a where the
