@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void residual_k(const T *__restrict__ so, cons
     const int i = g.x * 64 + (threadIdx.x % 64) + 1;
     const int j = g.y * 4 + (threadIdx.x / 64) + 1;
     const std::size_t P = (std::size_t)ii * jj, bz = g.z;
-    so += (bz / rep) * (NINE ? 5 : 3) * P;
+    so += operator_of(bz, rep) * (NINE ? 5 : 3) * P;
     qf += bz * P;
     q += bz * P;
     res += bz * P;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void gs_colour_k(const T *__restrict__ so, con
         i = 2 * k + ((pi + j) & 1);  // (i + j) % 2 == pi
     }
     if (i < 1 || i > ii - 2 || j < 1 || j > jj - 2) return;
-    const std::size_t P = (std::size_t)ii * jj, bz = g.z, bo = bz / rep;
+    const std::size_t P = (std::size_t)ii * jj, bz = g.z, bo = operator_of(bz, rep);
     so += bo * (NINE ? 5 : 3) * P;
     qf += bz * P;
     q += bz * P;
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(256) void restrict_k(const T *__restrict__ ci, cons
     const int jc = g.y * 4 + (threadIdx.x / 64) + 1;
     if (ic > iic - 2 || jc > jjc - 2) return;
     const std::size_t Pc = (std::size_t)iic * jjc, bz = g.z;
-    ci += (bz / rep) * 8 * Pc;
+    ci += operator_of(bz, rep) * 8 * Pc;
     q += bz * iif * (std::size_t)jjf;
     qc += bz * Pc;
     qc[pidx(ic, jc, iic)] = restrict_point<T>(ci, q, iif, iic, Pc, ic, jc);
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(64 * rc_rows<T>) void restrict_cycle_k(const T *__r
     const wg_pos g = tiled_wg(rep);
     const int ic0 = g.x * 64, jc0 = g.y * 16;
     const std::size_t Pc = (std::size_t)iic * jjc, bz = g.z;
-    ci += (bz / rep) * 8 * Pc;
+    ci += operator_of(bz, rep) * 8 * Pc;
     q += bz * iif * (std::size_t)jjf;
     qc += bz * Pc;
     xc += bz * Pc;
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void interp_add_k(T *__restrict__ q, const T *
     const int m = g.x * 64 + (threadIdx.x % 64) + 1;
     const int n = g.y * 4 + (threadIdx.x / 64) + 1;
     const std::size_t Pc = (std::size_t)iic * jjc, Pf = (std::size_t)iif * jjf, bz = g.z;
-    const std::size_t bo = bz / rep;
+    const std::size_t bo = operator_of(bz, rep);
     interp_block<T>(q + bz * Pf, qc + bz * Pc, res + bz * Pf, so + bo * ns * Pf, ci + bo * 8 * Pc,
                     iic, jjc, iif, jjf, m, n);
 }
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(64) void solve_cg_k(T *__restrict__ q, const T *__r
     const int n = (ii - 2) * (jj - 2);
     q += (std::size_t)blockIdx.x * ii * jj;  // one workgroup per problem of a batch
     qf += (std::size_t)blockIdx.x * ii * jj;
-    abd += (std::size_t)(blockIdx.x / rep) * ii * n;
+    abd += operator_of(blockIdx.x, rep) * ii * n;
     x += (std::size_t)blockIdx.x * n;
     coarse_band_solve<T>(q, qf, abd, x, ii, jj, threadIdx.x, blockDim.x, sh);
 }
@@ -880,7 +880,7 @@ __global__ __launch_bounds__(256) void residual_qT_k(const T *__restrict__ so,
     const wg_pos g = tiled_wg(rep);
     const int i0 = g.x * kTI + 1, j0 = g.y * kTJ + 1;
     const std::size_t P = (std::size_t)ii * jj, bz = g.z;
-    so += (bz / rep) * (NINE ? 5 : 3) * P;
+    so += operator_of(bz, rep) * (NINE ? 5 : 3) * P;
     qf += bz * P;
     qT += bz * P;
     res += bz * P;

@@ -2,6 +2,7 @@
 #include "../../include/cedar_hip.h"
 #include "bmg2_device.hpp"
 #include "bmg2_launch.hpp"
+#include "tile_order.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(1024) void coarse_cycle_k(const coarse_level<T> *__
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ double cg_sh[CG_LDS];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    const std::size_t bz = blockIdx.x, bo = bz / rep;
+    const std::size_t bz = blockIdx.x, bo = operator_of(bz, rep);
     const int nsor = relax_planes(relax);
     auto in_memory = [&](int l) {  // the level's arrays of problem bz (operator bo)
         coarse_level<T> d = lv[l];

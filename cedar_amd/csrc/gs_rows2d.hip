@@ -34,7 +34,7 @@ __global__ __launch_bounds__(W < 256 ? 256 : W) void gs9_rows_k(const T *__restr
     __shared__ T fresh[R][W * PP + 2];  // [t + 1]: the first colour's value of pair t
     const int tx = threadIdx.x % W, r = threadIdx.x / W;
     const wg_pos g = tiled_wg(rep);
-    const std::size_t P = (std::size_t)ii * jj, bz = g.z, bo = bz / rep;
+    const std::size_t P = (std::size_t)ii * jj, bz = g.z, bo = operator_of(bz, rep);
     const int blk = rev ? (int)gridDim.x - 1 - g.x : g.x;
     const int j = first + 2 * (blk * R + r);
     const bool row = j <= jj - 2;

@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256) void relax_lines_k(const T *__restrict__ so, c
     shared_op_order((int)gridDim.x, rep, bx, prob);
     const int line = bx * (blockDim.x / WAVE) + threadIdx.x / WAVE;
     if (line >= nlines) return;  // whole wavefront leaves together; no block barrier below
-    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = bz / rep;
+    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = operator_of(bz, rep);
     so += bo * (NINE ? 5 : 3) * P;
     qf += bz * P;
     q += bz * P;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(L *W * 64) void relax_xlines_seg_k(const T *__restr
     const int line = tile * L + slot;
     const bool valid = line < nlines;  // invalid wavefronts solve a copy of the last line
     const int j = first + 2 * min(line, nlines - 1);
-    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = bz / rep;
+    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = operator_of(bz, rep);
     so += bo * (NINE ? 5 : 3) * P;
     qf += bz * P;
     q += bz * P;
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(NC *W * 64) void relax_ylines_seg_k(const T *__rest
     if (tile >= ntiles) return;  // uniform over the workgroup
     const int wl = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     const int cs = wl / W, w = wl % W;
-    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = bz / rep;
+    const std::size_t P = (std::size_t)ii * jj, bz = prob, bo = operator_of(bz, rep);
     so += bo * (NINE ? 5 : 3) * P;
     qf += bz * P;
     q += bz * P;
