@@ -836,6 +836,17 @@ constexpr bool row_reaches(int x, int y, int z) {
     return gx >= -1 && gx <= 1 && gy >= -1 && gy <= 1 && gz >= -1 && gz <= 1;
 }
 
+// whether some f + o does, for f = F from C.  Where C and C + D lie inside the grid, which holds for
+// every entry that is kept, one of these f + o does too, so f has a term of the entry in exactly these
+// cases; elsewhere w * 0 would bring an infinite or undefined weight into the sum.
+template <bool NINE, int F, int T, int... O>
+constexpr bool row_has_term(std::integer_sequence<int, O...>) {
+    constexpr int fx = F % 3 - 1, fy = F / 3 % 3 - 1, fz = F / 9 - 1;
+    return (((NINE || (O % 3 != 1) + (O / 3 % 3 != 1) + (O / 9 != 1) <= 1) &&
+             row_reaches<T>(fx + O % 3 - 1, fy + O / 3 % 3 - 1, fz + O / 9 - 1)) ||
+            ...);
+}
+
 template <bool NINE, int PARTS, int PART, int F, int O, int... T>
 __device__ inline void row_neighbour(const row_ctx &c, double (&inner)[14],
                                      std::integer_sequence<int, T...>) {
@@ -861,23 +872,30 @@ __device__ inline void row_neighbour(const row_ctx &c, double (&inner)[14],
     }
 }
 
-template <bool NINE, int PARTS, int PART, int F, int... O>
+template <bool NINE, int PARTS, int PART, int F, int... O, int... T>
 __device__ inline void row_fine_point(const row_ctx &c, double (&sum)[14],
-                                      std::integer_sequence<int, O...>) {
+                                      std::integer_sequence<int, O...>,
+                                      std::integer_sequence<int, T...> all) {
     constexpr int fx = F % 3 - 1, fy = F / 3 % 3 - 1, fz = F / 9 - 1;
     if (!(c.vx[fx + 2] && c.vy[fy + 2] && c.vz[fz + 2])) return;
     double inner[14] = {0.0};
-    (row_neighbour<NINE, PARTS, PART, F, O>(c, inner, std::make_integer_sequence<int, 14>{}), ...);
+    (row_neighbour<NINE, PARTS, PART, F, O>(c, inner, all), ...);
     const double w = row_weight<0, 0, 0, fx, fy, fz>(c);
-#pragma unroll
-    for (int t = 0; t < 14; ++t)
-        if (row_part<PARTS, PART>(t)) sum[t] += w * inner[t];  // a direction out of reach adds zero
+    (
+        [&] {
+            if constexpr (row_part<PARTS, PART>(T) &&
+                          row_has_term<NINE, F, T>(std::integer_sequence<int, O...>{}))
+                sum[T] += w * inner[T];
+        }(),
+        ...);
 }
 
 template <bool NINE, int PARTS, int PART, int... F>
 __device__ inline void row_sums(const row_ctx &c, double (&sum)[14],
                                 std::integer_sequence<int, F...>) {
-    (row_fine_point<NINE, PARTS, PART, F>(c, sum, std::make_integer_sequence<int, 27>{}), ...);
+    (row_fine_point<NINE, PARTS, PART, F>(c, sum, std::make_integer_sequence<int, 27>{},
+                                          std::make_integer_sequence<int, 14>{}),
+     ...);
 }
 
 template <bool NINE, int PARTS, int... PART>

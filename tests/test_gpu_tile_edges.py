@@ -61,6 +61,29 @@ def test_galerkin3(dims, ns):
     assert (host(soc)[:, 0] == 7.0).all() and (host(soc)[:, :, :, -1] == 7.0).all()  # ghosts untouched
 
 
+# a weight that is infinite or undefined enters exactly the sums that have a term with it: one such
+# weight per case, in each of the 26 planes in turn; the parts of a row and, at the largest, whole rows
+@pytest.mark.parametrize("dims", [(5, 4, 7), (6, 260, 66)])
+@pytest.mark.parametrize("ns", [4, 14])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_galerkin3_keeps_undefined_weights_where_they_are(dims, ns, bad):
+    import cedar_amd as C
+    print(f"\ngalerkin, weight {bad} {dims} ns={ns}", flush=True)
+    rng = np.random.default_rng(sum(dims) + ns)
+    so = rand_so3(rng, *dims, ns)
+    ci = O3.setup_interp(so)
+    nc = ci.shape[1:]
+    for p in range(26) if dims[1] < 100 else (0, 13, 25):
+        c = ci.copy()
+        at = tuple(int(rng.integers(1, n)) for n in nc)
+        c[(p,) + at] = bad
+        soc = torch.zeros((14,) + nc, dtype=torch.float64, device="cuda")
+        C.cdr3.setup_galerkin(dev(so), dev(c), soc)
+        ref = O3.setup_galerkin(so, c)
+        inner = (slice(None),) + (slice(1, -1),) * 3
+        assert np.array_equal(host(soc)[inner], ref[inner], equal_nan=True), (p, at)
+
+
 def _so2(rng, nx, ny, ns):
     """Random couplings inside the grid, diagonally dominant, zero across the boundary."""
     so = np.zeros((ns, ny + 2, nx + 2))
