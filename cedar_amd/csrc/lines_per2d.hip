@@ -70,9 +70,9 @@ __device__ inline void chain(T *v, const T *E, int n) {
 // (row-contiguous loads), the two recurrences by one lane per vector (the line's right-hand side
 // and, with sm, its Sherman-Morrison vector on another lane of the same wavefront), the divisions
 // between them and the correction by all threads again.  Bound by the recurrences, n dependent
-// products and differences per sweep; the grid is one workgroup per G lines so that every line of
-// a colour runs at once.  With one lane per line walking memory the 512 x 511
-// FP64 Poisson sweep took 765 us (x) and 420 us (y) per colour.
+// products and differences per sweep; the launcher takes G small as long as every line of a colour
+// then runs at once (lines_per_group).  With one lane per line walking memory the 512 x 511 FP64
+// Poisson sweep took 765 us (x) and 420 us (y) per colour.
 //
 // img: this launch also writes the periodic images that only it or later sweeps read.
 //   1: the lines run along the one periodic direction; each line's own images, and those of the
@@ -250,6 +250,20 @@ void launch_per(const T *so, const T *qf, T *q, const T *sor, int ii, int jj, in
                                          lds, s>>>(so, qf, q, sor, ii, jj, first, sm, img);
 }
 
+// Lines per workgroup where a colour has cnt lines (of all problems) of n points: 64, 16, or gw, one for
+// x-lines and four for y-lines.  A workgroup costs 7 us however short its lines, and the chip runs about
+// 1024 at once, so beyond that many of gw lines short ones share workgroups.  A sweep of 65536 x-lines of
+// 8 points (FP64, nine-point, wrap in x) takes 182 us by one line and 23 by 16; of 2 points 153 by one,
+// 14 by 16 and 9 by 64, of 8 points no less by 64 than by 16.  Lines of more than 32 points give every
+// thread work by themselves and share only at four times as many lines: 4096 FP32 x-lines of 48 points 15
+// us by one, 18 by 16; 32768 FP64 ones of 64 points (five-point, no wrap) 163 and 37.  (One lane per line walking memory: 70
+// us at 65536 x 8, 131 at 32768 x 64.)
+constexpr int kLongestShared = 128;
+inline int lines_per_group(int n, std::size_t cnt, int gw) {
+    if (n > kLongestShared || cnt <= (std::size_t)1024 * gw * (n <= 32 ? 1 : 4)) return gw;
+    return n <= 4 ? 64 : 16;
+}
+
 template <typename T, bool NINE, int DIR>
 void sweep_per(const T *so, const T *qf, T *q, const T *sor, T *work, int ii, int jj, int updown,
                int jpn, hipStream_t s, int nb) {
@@ -269,11 +283,16 @@ void sweep_per(const T *so, const T *qf, T *q, const T *sor, T *work, int ii, in
         const int first = (pass == 0) == (updown == 0) ? 2 : 1;
         const int cnt = first > nl ? 0 : (nl - first) / 2 + 1;
         const int img = !own ? 0 : sm ? 1 : pass == 1 ? 2 : 0;
+        const int G = lines_per_group(n, (std::size_t)cnt * nb, GW);
         if (cnt > 0) {
             if (!fits)
                 relax_lines_per_long_k<T, NINE, DIR><<<dim3((unsigned)((cnt + 63) / 64), (unsigned)nb),
                                                        64, 0, s>>>(so, qf, q, sor, work, ii, jj,
                                                                    first, sm);
+            else if (G == 64)
+                launch_per<T, NINE, DIR, 64>(so, qf, q, sor, ii, jj, first, sm, img, cnt, s, nb);
+            else if (G == 16)
+                launch_per<T, NINE, DIR, 16>(so, qf, q, sor, ii, jj, first, sm, img, cnt, s, nb);
             else if (wide)
                 launch_per<T, NINE, DIR, GW>(so, qf, q, sor, ii, jj, first, sm, img, cnt, s, nb);
             else

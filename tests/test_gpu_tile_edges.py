@@ -42,6 +42,60 @@ def test_periodic_lines(nx, ny, mask, ns):
             assert np.array_equal(host(g), O.relax_lines_periodic(so, qf, q, sor, ud, d, jpn)), (d, ud)
 
 
+# short lines of which many share a workgroup: 64 up to 4 points, 16 up to 32, and up to 128 where there
+# are four times as many; longer ones by themselves.  More of them than run at once otherwise (1024
+# x-lines or 4096 y-lines of a colour), one less, and a last workgroup that is full or has one line; odd
+# and even seams
+@pytest.mark.parametrize("n,dr,nl", [(n, dr, nl) for n in (2, 3, 4, 5, 16, 31, 32, 33)
+                                     for dr, nl in (("x", 2048), ("x", 2049), ("x", 2177), ("x", 2178),
+                                                    ("y", 8192), ("y", 8194), ("y", 8321))] +
+                         [(n, "x", nl) for n in (33, 128, 129) for nl in (8192, 8194, 8225)] +
+                         [(n, "y", nl) for n in (33, 128, 129) for nl in (32768, 32770, 32801)])
+@pytest.mark.parametrize("mask", [1, 2, 3])
+def test_many_short_periodic_lines(n, dr, nl, mask):
+    import cedar_amd as C
+    nx, ny = (n, nl) if dr == "x" else (nl, n)
+    ns = 3 + 2 * ((n + nl) % 2)
+    print(f"\nshort periodic lines {dr} {nx}x{ny} ns={ns} mask={mask}", flush=True)
+    rng = np.random.default_rng(3 * nx + ny + mask)
+    jpn = O.bc_from_mask(mask)
+    so = rand_periodic_so(rng, nx, ny, ns, mask)
+    q = rng.standard_normal((ny + 2, nx + 2))
+    qf = rng.standard_normal(q.shape)
+    sor, info = O.setup_lines_periodic(so, dr, jpn)
+    assert info == 0
+    for ud in (O.DOWN, O.UP):
+        g = C.relax_lines_periodic(dev(so), dev(qf), dev(q), dev(sor), ud, dr, jpn)
+        assert np.array_equal(host(g), O.relax_lines_periodic(so, qf, q, sor, ud, dr, jpn)), ud
+
+
+# A sweep of 2048 lines leaves the chip half empty; 32 times as many lines have 32 times the work and
+# move 30 MB.  With a workgroup for each line they took 14 to 16 times as long, shared out 1.7 to 3.
+@pytest.mark.parametrize("dr", ["x", "y"])
+def test_short_periodic_lines_scale(dr):
+    import cedar_amd as C
+    jpn = C.bc_from_mask((dr == "x", dr == "y"))
+    best = {}
+    for nl in (2048, 65536):
+        d = (8, nl) if dr == "x" else (nl, 8)
+        so = torch.full((5, d[1] + 2, d[0] + 2), 0.5, dtype=torch.float64, device="cuda")
+        so[0] = 9.0
+        sor = torch.zeros((2,) + tuple(so.shape[1:]), dtype=torch.float64, device="cuda")
+        C.setup_lines_periodic(so, sor, dr, jpn)
+        f, q = torch.rand_like(so[0]), torch.rand_like(so[0])
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            C.relax_lines_periodic(so, f, q, sor, 0, dr, jpn)
+            a.record()
+            for _ in range(20):
+                C.relax_lines_periodic(so, f, q, sor, 0, dr, jpn)
+            b.record()
+            b.synchronize()
+            best[nl] = min(best.get(nl, 1e9), a.elapsed_time(b) / 20)
+    print(f"\nshort periodic lines {dr}: {best}", flush=True)
+    assert best[65536] < 6 * best[2048], best
+
+
 # coarse rows of 64 points, one less and one more; the smallest grids; even extents, whose last
 # fine points lie beyond the last coarse one; a level of more than 256 workgroups (one point's
 # whole row per thread there, parts of it below)
