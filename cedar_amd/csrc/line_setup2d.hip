@@ -14,14 +14,13 @@ namespace {
 // (kept in DPTTRF's order, so the factors are the reference's bit for bit), which bounds the
 // kernel: about 60 ns per element whatever the number of lines.  One wavefront of the workgroup
 // runs the chains of kLines lines, a lane each, out of LDS; the other three move the tiles, with
-// unit stride in memory for either direction: the next one in, the previous one out.  A lane that
-// walked its line in memory paid a round trip per element: 320 us (x) and 245 us (y) on average
-// over the nine levels of 1500 x 1100.
-constexpr int kLines = 16, kTile = 64, kBufs = 3;
-
+// unit stride in memory for either direction: the next one in, the previous one out (kBufs = 3; a line
+// of one tile needs one buffer).  A lane that walked its line in memory paid a round trip per element:
+// 320 us (x) and 245 us (y) on average over the nine levels of 1500 x 1100.
+//
 // per: the line direction is periodic, so its wrap couplings are added to the end diagonals
 // (src/2d/ftn/BMG2_SymStd_SETUP_lines_x.f90:75-82, _y.f90:77-84) before the factorisation
-template <int DIR>
+template <int DIR, int kLines, int kTile, int kBufs>
 __global__ __launch_bounds__(256) void setup_lines_k(const double *__restrict__ so,
                                                      double *__restrict__ sor, int ii, int jj,
                                                      int ns, int *__restrict__ info, int per) {
@@ -102,11 +101,21 @@ __global__ __launch_bounds__(256) void setup_lines_k(const double *__restrict__ 
 void setup_lines(int dir, const double *so, int nstncl, double *sor, int ii, int jj, int *info,
                  hipStream_t s, int nb, int per) {
     const int nl = dir == 0 ? jj - 2 : ii - 2;
-    const dim3 g((unsigned)((nl + kLines - 1) / kLines), (unsigned)nb);
-    if (dir == 0)
-        setup_lines_k<0><<<g, 256, 0, s>>>(so, sor, ii, jj, nstncl, info, per);
+    const int n = dir == 0 ? ii - 2 : jj - 2;
+    // Three buffers of 16 lines by 64 take 50 KB, three workgroups a CU: too few where many lines are
+    // short.  Lines of one tile come without the other buffers, and those of at most 8 points 64 to a
+    // workgroup: 200000 x-lines of 4 points 81 -> 32 us (54 by a lane per line walking memory), 65536
+    // of 64 points 85 -> 60.
+    auto launch = [&](auto kernel, int lines) {
+        const dim3 g((unsigned)((nl + lines - 1) / lines), (unsigned)nb);
+        kernel<<<g, 256, 0, s>>>(so, sor, ii, jj, nstncl, info, per);
+    };
+    if (n <= 8)
+        dir == 0 ? launch(setup_lines_k<0, 64, 8, 1>, 64) : launch(setup_lines_k<1, 64, 8, 1>, 64);
+    else if (n <= 64)
+        dir == 0 ? launch(setup_lines_k<0, 16, 64, 1>, 16) : launch(setup_lines_k<1, 16, 64, 1>, 16);
     else
-        setup_lines_k<1><<<g, 256, 0, s>>>(so, sor, ii, jj, nstncl, info, per);
+        dir == 0 ? launch(setup_lines_k<0, 16, 64, 3>, 16) : launch(setup_lines_k<1, 16, 64, 3>, 16);
 }
 
 }  // namespace

@@ -227,6 +227,52 @@ def test_line_setup(nx, ny, ns):
         assert np.array_equal(host(C.setup_lines(dev(so), g, d)), sor), d
 
 
+# lines of at most 8 points, 64 to a workgroup, of at most 64, 16 to one, and longer: groups that are
+# full, one short, one over; every pivot in turn not positive
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 64, 65])
+@pytest.mark.parametrize("nl", [15, 16, 17, 63, 64, 65, 129])
+@pytest.mark.parametrize("d", ["x", "y"])
+def test_line_setup_of_short_lines(n, nl, d):
+    import cedar_amd as C
+    nx, ny = (n, nl) if d == "x" else (nl, n)
+    print(f"\nshort line setup {d} {nx}x{ny}", flush=True)
+    so = _so2(np.random.default_rng(n + nl), nx, ny, 5)
+    sor = O.setup_lines(so, d)
+    sor = sor[0] if isinstance(sor, tuple) else sor
+    g = torch.zeros(sor.shape, dtype=torch.float64, device="cuda")
+    assert np.array_equal(host(C.setup_lines(dev(so), g, d)), sor)
+    for k in range(0, n, 7):
+        bad = so.copy()
+        bad[(0,) + ((nl, k + 1) if d == "x" else (k + 1, nl))] = -1.0
+        with pytest.raises(C.CedarHipError):
+            C.setup_lines(dev(bad), g, d)
+
+
+# 200000 lines of 4 points move 20 MB, a few us beside a launch: three buffers for each group of 16 made
+# them take 3 times as long as 2048 lines, one for 64 takes 1.2
+@pytest.mark.parametrize("d", ["x", "y"])
+def test_line_setup_of_short_lines_scales(d):
+    import cedar_amd as C
+    best = {}
+    for nl in (2048, 200000):
+        nx, ny = (4, nl) if d == "x" else (nl, 4)
+        so = torch.full((5, ny + 2, nx + 2), 0.5, dtype=torch.float64, device="cuda")
+        so[0] = 9.0
+        sor = torch.zeros((2, ny + 2, nx + 2), dtype=torch.float64, device="cuda")
+        C.setup_lines(so, sor, d)
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            C.setup_lines(so, sor, d)
+            a.record()
+            for _ in range(20):
+                C.setup_lines(so, sor, d)
+            b.record()
+            b.synchronize()
+            best[nl] = min(best.get(nl, 1e9), a.elapsed_time(b) / 20)
+    print(f"\nshort line setup {d}: {best}", flush=True)
+    assert best[200000] < 2 * best[2048], best
+
+
 @pytest.mark.parametrize("k", [0, 1, 63, 64, 128])
 @pytest.mark.parametrize("d", ["x", "y"])
 def test_line_setup_reports_the_failing_pivot(k, d):
