@@ -43,6 +43,8 @@ _P = _vp
 PROTOTYPES = {
     "cdr_hip_status_string": (ctypes.c_char_p, [_i]),
     "cdr_hip_version": (ctypes.c_char_p, []),
+    "cdr_hip_memory_trim": (_sz, []),
+    "cdr_hip_memory_limit": (_sz, [_sz]),
     "cdr_hip_autotune": (_i, [_i]),
     "cdr_hip_autotune_report": (_i, [ctypes.c_char_p, _i]),
     "cdr_hip_line_shapes2d": (_i, [_i, _i, _i, _i, _i]),

@@ -188,6 +188,19 @@ def relax_lines_xy(so, qf, q, sorx, sory, updown):
     return q
 
 
+def memory_trim():
+    """Gives back the device memory kept from closed solvers (at most memory_limit); returns its
+    bytes.  For a program that wants the device's last gigabytes elsewhere."""
+    return _abi.load().cdr_hip_memory_trim()
+
+
+def memory_limit(nbytes):
+    """Sets how much device memory closed solvers may leave for the next one, in bytes for the whole
+    process (4 GiB, or CEDAR_AMD_POOL_MB of the environment; 0 keeps none); returns the previous
+    limit."""
+    return _abi.load().cdr_hip_memory_limit(int(nbytes))
+
+
 def autotune(on):
     """Turns line-kernel shape tuning on or off (process-wide); returns the previous setting."""
     return bool(_abi.load().cdr_hip_autotune(1 if on else 0))

@@ -9,6 +9,7 @@
 
 #include "bmg2_launch.hpp"
 #include "capi2d_impl.hpp"
+#include "device_pool.hpp"
 
 namespace {
 
@@ -420,6 +421,21 @@ int cdr_hip_relax_lines_xy2d_f32(const float *so, int ns, const float *qf, float
                                  const float *sorx, const float *sory, float *work, int ii, int jj,
                                  int ud, void *st) {
     return api2::relax_lines_xy<float>(so, ns, qf, q, sorx, sory, work, ii, jj, ud, S(st));
+}
+
+size_t cdr_hip_memory_trim(void) {
+    try {
+        return cedar::hip::pool_trim();
+    } catch (...) {
+        return 0;
+    }
+}
+size_t cdr_hip_memory_limit(size_t bytes) {
+    try {
+        return cedar::hip::pool_set_limit(bytes);
+    } catch (...) {
+        return 0;
+    }
 }
 
 int cdr_hip_autotune(int on) { return cdr::k2::set_autotune(on); }

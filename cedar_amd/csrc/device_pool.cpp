@@ -1,5 +1,7 @@
 #include "device_pool.hpp"
 
+#include <algorithm>
+#include <cstdlib>
 #include <list>
 #include <mutex>
 #include <unordered_map>
@@ -21,8 +23,22 @@ struct pool {
     std::mutex mu;
     std::unordered_map<void *, block> live;  // blocks handed out
     std::list<block> kept;                   // oldest first
-    std::size_t kept_bytes = 0;
+    std::size_t kept_bytes = 0, limit = kPoolBytes;
     std::vector<std::pair<int, hipStream_t>> streams;
+
+    pool() {
+        const char *v = std::getenv("CEDAR_AMD_POOL_MB");
+        char *end = nullptr;
+        const unsigned long long mb = v && *v >= '0' && *v <= '9' ? std::strtoull(v, &end, 10) : 0;
+        if (end && *end == '\0') limit = (std::size_t)std::min(mb, ~0ull >> 20) << 20;
+    }
+    // moves the blocks kept longest to out until at most `most` bytes are left (the lock is held)
+    void evict(std::size_t most, std::list<block> &out) {
+        while (kept_bytes > most) {
+            kept_bytes -= kept.front().bytes;
+            out.splice(out.end(), kept, kept.begin());
+        }
+    }
 };
 
 // never destroyed: blocks may come back while the process ends
@@ -38,9 +54,14 @@ int current_device() {
     return hipGetDevice(&d) == hipSuccess ? d : -1;
 }
 
-void release(std::vector<block> &out) {
-    for (const block &b : out) (void)hipFree(b.p);
+std::size_t release(std::list<block> &out) {
+    std::size_t bytes = 0;
+    for (const block &b : out) {
+        (void)hipFree(b.p);
+        bytes += b.bytes;
+    }
     out.clear();
+    return bytes;
 }
 
 }  // namespace
@@ -54,23 +75,21 @@ void *pool_malloc(std::size_t bytes, hipError_t *e) {
         // the block kept last is the likeliest to be of this size
         for (auto it = P.kept.rbegin(); it != P.kept.rend(); ++it) {
             if (it->bytes != bytes || it->device != dev) continue;
-            const block b = *it;
+            void *const p = it->p;
+            P.live.emplace(p, *it);  // the one that can throw, so first
+            P.kept_bytes -= it->bytes;
             P.kept.erase(std::next(it).base());
-            P.kept_bytes -= b.bytes;
-            P.live.emplace(b.p, b);
             *e = hipSuccess;
-            return b.p;
+            return p;
         }
     }
     void *p = nullptr;
     *e = hipMalloc(&p, bytes);
     if (*e == hipErrorOutOfMemory) {
-        std::vector<block> out;
+        std::list<block> out;
         {
             std::lock_guard<std::mutex> g(P.mu);
-            out.assign(P.kept.begin(), P.kept.end());
-            P.kept.clear();
-            P.kept_bytes = 0;
+            P.evict(0, out);
         }
         if (!out.empty()) {
             (void)hipGetLastError();
@@ -79,33 +98,69 @@ void *pool_malloc(std::size_t bytes, hipError_t *e) {
         }
     }
     if (*e != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> g(P.mu);
-    P.live.emplace(p, block{p, bytes, dev});
+    try {
+        std::lock_guard<std::mutex> g(P.mu);
+        P.live.emplace(p, block{p, bytes, dev});
+    } catch (...) {
+        (void)hipFree(p);
+        throw;
+    }
     return p;
 }
 
-void pool_free(void *p) {
+void pool_free(void *p) noexcept {
     if (!p) return;
     pool &P = the_pool();
-    std::vector<block> out;
-    {
+    std::list<block> out;
+    try {
+        std::list<block> mine(1);  // allocated before anything changes
         std::lock_guard<std::mutex> g(P.mu);
         const auto it = P.live.find(p);
-        const block b = it == P.live.end() ? block{p, 0, -1} : it->second;
+        mine.front() = it == P.live.end() ? block{p, 0, -1} : it->second;
         if (it != P.live.end()) P.live.erase(it);
-        if (b.device < 0 || b.device != idle_device || b.bytes > kPoolBytes) {
-            out.push_back(b);
+        const block &b = mine.front();
+        if (b.device < 0 || b.device != idle_device || b.bytes > P.limit) {
+            out.splice(out.end(), mine);
         } else {
-            P.kept.push_back(b);
             P.kept_bytes += b.bytes;
-            while (P.kept_bytes > kPoolBytes) {
-                P.kept_bytes -= P.kept.front().bytes;
-                out.push_back(P.kept.front());
-                P.kept.pop_front();
-            }
+            P.kept.splice(P.kept.end(), mine);
+            P.evict(P.limit, out);
         }
+    } catch (...) {  // no host memory for the list: the block goes back all the same
+        {
+            std::lock_guard<std::mutex> g(P.mu);
+            P.live.erase(p);
+        }
+        (void)hipFree(p);
     }
     release(out);
+}
+
+std::size_t pool_set_limit(std::size_t bytes) {
+    pool &P = the_pool();
+    std::list<block> out;
+    std::size_t prev;
+    {
+        std::lock_guard<std::mutex> g(P.mu);
+        prev = P.limit;
+        P.limit = bytes;
+        P.evict(bytes, out);
+    }
+    release(out);
+    return prev;
+}
+
+std::size_t pool_trim() {
+    pool &P = the_pool();
+    std::list<block> out;
+    std::vector<std::pair<int, hipStream_t>> streams;
+    {
+        std::lock_guard<std::mutex> g(P.mu);
+        P.evict(0, out);
+        streams.swap(P.streams);
+    }
+    for (const auto &s : streams) (void)hipStreamDestroy(s.second);
+    return release(out);
 }
 
 void pool_idle_scope::enter(hipError_t waited) {

@@ -3,8 +3,10 @@
 // A solver allocates some fifty buffers and frees them together, and every hipFree waits for the
 // device and unmaps: 10 of the 31 ms of a differentiated solve of 4 x 1025^2, which builds a solver
 // per call, went into it and 2 ms into hipMalloc.  Blocks of a destroyed solver are therefore kept
-// for the next one of the same sizes, per device and byte count, up to kPoolBytes in all; beyond
-// that the ones kept longest are freed, and when an allocation fails all of them are.
+// for the next one of the same sizes, per device and byte count, up to a limit in all; beyond
+// that the ones kept longest are freed, and when an allocation here fails all of them are.  Another
+// library's allocation cannot ask for them: pool_trim gives them back at once, and a limit of 0 keeps
+// none.
 //
 // A block may be handed to any thread and stream, so it is only kept while no queued work can still
 // use it: inside a pool_idle_scope.  Outside one pool_free is hipFree.
@@ -18,11 +20,17 @@
 namespace cedar {
 namespace hip {
 
+// Bytes kept at most, unless CEDAR_AMD_POOL_MB of the environment (MiB, read at the first use) or
+// pool_set_limit says otherwise.
 constexpr std::size_t kPoolBytes = std::size_t(4) << 30;
+// Sets the limit, frees what lies beyond it and returns the previous one.
+std::size_t pool_set_limit(std::size_t bytes);
+// Frees every kept block and stream; returns the bytes of the blocks.
+std::size_t pool_trim();
 
 // nullptr and the error in *e on failure
 void *pool_malloc(std::size_t bytes, hipError_t *e);
-void pool_free(void *p);
+void pool_free(void *p) noexcept;
 
 // While alive, blocks of the current device that this thread frees are idle: nothing queued uses
 // them.  The constructor waits for the device, or for the stream that alone used them.

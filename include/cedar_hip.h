@@ -66,6 +66,16 @@ int cdr_hip_autotune_report(char *buf, int len);
 int cdr_hip_line_shapes2d(int dir, int fp_bits, int nstncl, int ii, int jj);
 int cdr_hip_set_line_shape2d(int dir, int fp_bits, int nstncl, int ii, int jj, int nb, int shape);
 
+/* Device memory of destroyed solvers.  A solver's buffers are kept when it is destroyed, for the next
+ * solver of the same sizes on the same device, up to a limit for the whole process: 4 GiB, or
+ * CEDAR_AMD_POOL_MB (MiB, 0 keeps none) of the environment at the first use.  They are given back when
+ * an allocation of this library fails, but not when one of another library does.
+ * cdr_hip_memory_trim gives back all of them now (and the streams kept for graph captures) and returns
+ * their bytes; cdr_hip_memory_limit sets the limit, gives back what lies beyond it and returns the
+ * previous limit.  Both may be called from any thread at any time; live solvers are not affected. */
+size_t cdr_hip_memory_trim(void);
+size_t cdr_hip_memory_limit(size_t bytes);
+
 /* ---------------------------------------------------------------------------------------
  * 2D kernels (FP64 and FP32 variants where the V-cycle needs them)
  * ------------------------------------------------------------------------------------- */

@@ -78,3 +78,41 @@ def test_threads_and_streams_that_build_and_destroy_solvers():
     for t in ts:
         t.join()
     assert not bad, bad
+
+
+def test_closed_solvers_give_their_memory_back():
+    """memory_trim returns what closed solvers left, to the device and so to other libraries; with a
+    limit of 0 they leave nothing; a limit between evicts, and solutions stay the same."""
+    import cedar_amd as C
+    so, b = _problem(700, 3)
+    free = lambda: torch.cuda.mem_get_info()[0]
+
+    def solve():
+        s = C.Solver(so, **KW)
+        x, h = s.solve(b)
+        s.close()
+        return x, h
+
+    first = solve()
+    torch.cuda.synchronize()
+    C.memory_trim()
+    base = free()
+    prev = C.memory_limit(1 << 32)
+    least = 5 * 702 * 702 * 8  # the factors of both line directions and the residual of the finest level
+    try:
+        solve()
+        torch.cuda.synchronize()
+        assert base - free() > least
+        assert C.memory_trim() > least
+        assert free() >= base - (4 << 20)
+        assert C.memory_trim() == 0
+        for limit in (0, 20 << 20):
+            C.memory_limit(limit)
+            for _ in range(2):
+                x, h = solve()
+                assert torch.equal(x, first[0]) and np.array_equal(h, first[1])
+            torch.cuda.synchronize()
+            assert C.memory_limit(limit) == limit
+            assert C.memory_trim() <= limit
+    finally:
+        C.memory_limit(prev)
