@@ -47,6 +47,7 @@ PROTOTYPES = {
     "cdr_hip_memory_limit": (_sz, [_sz]),
     "cdr_hip_autotune": (_i, [_i]),
     "cdr_hip_autotune_report": (_i, [ctypes.c_char_p, _i]),
+    "cdr_hip_autotune_clear": (None, []),
     "cdr_hip_line_shapes2d": (_i, [_i, _i, _i, _i, _i]),
     "cdr_hip_set_line_shape2d": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "cdr_hip_norm_work2d": (_sz, [_i, _i]),

@@ -207,12 +207,18 @@ def autotune(on):
 
 
 def autotune_report():
-    """The recorded line-kernel shape choices (list of dicts)."""
+    """The recorded choices (list of dicts): line-kernel shapes (dir x, y, t) and first levels of the
+    fused cycle (dir f)."""
     import json
     n = _abi.load().cdr_hip_autotune_report(None, 0)
     buf = ctypes.create_string_buffer(n + 1)
     _abi.load().cdr_hip_autotune_report(buf, n + 1)
     return json.loads(buf.value.decode())
+
+
+def autotune_clear():
+    """Forgets every recorded choice, pinned line shapes included; later solvers time anew."""
+    _abi.load().cdr_hip_autotune_clear()
 
 
 def restrict(ci, q, qc, jpn=0):

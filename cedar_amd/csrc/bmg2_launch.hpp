@@ -189,8 +189,9 @@ int tune_lines_ytr(const T *so, const T *soT, int nstncl, const T *qf, T *q, con
 int line_shape_count(int dir, int wbytes, int nstncl, int ii, int jj);
 // records `shape` for (direction, word size, stencil, ii, jj, nb) (shape < 0: erases the entry)
 void set_line_shape(int dir, int wbytes, int nstncl, int ii, int jj, int nb, int shape);
-// JSON list of the recorded choices
+// JSON list of the recorded choices; tune_clear forgets all of them, pinned shapes included
 std::string tune_report();
+void tune_clear();
 
 template <typename T>
 void restrict_(const T *ci, const T *q, T *qc, int iif, int jjf, int iic, int jjc, hipStream_t s,

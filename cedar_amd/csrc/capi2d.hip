@@ -10,6 +10,7 @@
 #include "bmg2_launch.hpp"
 #include "capi2d_impl.hpp"
 #include "device_pool.hpp"
+#include "fused_start.hpp"
 
 namespace {
 
@@ -457,8 +458,15 @@ int cdr_hip_set_line_shape2d(int dir, int fp_bits, int nstncl, int ii, int jj, i
     return CDR_OK;
 }
 
+void cdr_hip_autotune_clear(void) {
+    cdr::k2::tune_clear();
+    cedar::hip::fused_start_clear();
+}
+
 int cdr_hip_autotune_report(char *buf, int len) {
-    const std::string r = cdr::k2::tune_report();
+    std::string r = cdr::k2::tune_report();
+    const std::string f = cedar::hip::fused_start_report();
+    if (!f.empty()) r.replace(r.size() - 1, 1, (r.size() > 2 ? "," : "") + f + "]");
     if (buf && len > 0) {
         const std::size_t n = std::min(r.size(), (std::size_t)len - 1);
         std::memcpy(buf, r.data(), n);

@@ -1092,6 +1092,11 @@ int tune_lines_ytr(const T *so, const T *soT, int nstncl, const T *qf, T *q, con
     return best;
 }
 
+void tune_clear() {
+    std::lock_guard<std::mutex> g(g_tune_mu);
+    g_tune.clear();
+}
+
 std::string tune_report() {
     std::lock_guard<std::mutex> g(g_tune_mu);
     std::string out = "[";

@@ -145,17 +145,47 @@ private:
 
 }  // namespace
 
+namespace {
+std::mutex g_start_mu;
+std::map<fused_start_key, int> g_start;
+}  // namespace
+
 int fused_start(const fused_start_key &key, int record) {
-    static std::mutex mu;
-    static std::map<fused_start_key, int> table;
-    std::lock_guard<std::mutex> g(mu);
+    std::lock_guard<std::mutex> g(g_start_mu);
     if (record < 0) {
-        const auto it = table.find(key);
-        return it == table.end() ? -1 : it->second;
+        const auto it = g_start.find(key);
+        return it == g_start.end() ? -1 : it->second;
     }
-    if (table.size() >= 1024) table.clear();
-    table[key] = record;
+    if (g_start.size() >= 1024) g_start.clear();
+    g_start[key] = record;
     return record;
+}
+
+void fused_start_clear() {
+    std::lock_guard<std::mutex> g(g_start_mu);
+    g_start.clear();
+}
+
+std::string fused_start_report() {
+    std::lock_guard<std::mutex> g(g_start_mu);
+    std::string out;
+    for (const auto &kv : g_start) {
+        const fused_start_key &k = kv.first;
+        int nx = k[5] - 2, ny = k[6] - 2;  // of the start level
+        for (int l = 0; l < kv.second; ++l) {
+            nx = (nx - 1) / 2 + 1;
+            ny = (ny - 1) / 2 + 1;
+        }
+        char buf[320];
+        std::snprintf(buf, sizeof(buf),
+                      "%s{\"dir\":\"f\",\"fp\":%d,\"stencil\":9,\"ii\":%d,\"jj\":%d,\"nb\":%d,"
+                      "\"shape\":%d,\"kernel\":\"fused cycle from level %d of %d x %d, relaxation %d, "
+                      "V(%d,%d), %d per operator\",\"device\":%d}",
+                      out.empty() ? "" : ",", 8 * k[1], nx + 2, ny + 2, k[8], kv.second, kv.second,
+                      k[5] - 2, k[6] - 2, k[2], k[3], k[4], k[9], k[0]);
+        out += buf;
+    }
+    return out;
 }
 
 void register_hip_kernels(kernel_manager &km, int *info) {

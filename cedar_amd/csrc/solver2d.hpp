@@ -12,7 +12,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -26,6 +25,7 @@
 #include "bmg2_launch.hpp"
 #include "capi2d_impl.hpp"
 #include "cedar_hip.hpp"
+#include "fused_start.hpp"
 #include "stop_rule.hpp"
 
 namespace cedar {
@@ -49,12 +49,6 @@ struct level_data {
     grid_func<T> x, b, res;
     relax_stencil<T> SOR[2];
 };
-
-// First level of the fused coarse cycle by word size, smoothing, extents, levels, batch and
-// right-hand sides per operator: the recorded one (record < 0; -1 if none), or records `record`.  One
-// table per process, guarded by a mutex, emptied when it holds 1024 entries.
-using fused_start_key = std::array<int, 9>;
-int fused_start(const fused_start_key &key, int record);
 
 class solver2d {
 public:
@@ -472,11 +466,13 @@ private:
         if (cand.empty()) return;
         int lt = cand[0];
         if (cand.size() > 1 && k2::autotune_enabled()) {
-            // the choice depends on sizes and settings alone, so the next solver with the same ones
-            // takes it over instead of capturing and timing five cycles again (4 of 25 ms of a 1500 x
-            // 1100 setup and solve)
+            // the choice depends on sizes, settings and the device alone, so the next solver with the
+            // same ones takes it over instead of capturing and timing five cycles again (4 of 25 ms of a
+            // 1500 x 1100 setup and solve)
             const extents &e = L[0].ext;
-            const fused_start_key key{(int)sizeof(T), set_.relaxation, set_.nrelax_pre,
+            int dev = 0;
+            check_hip(hipGetDevice(&dev), "hipGetDevice");
+            const fused_start_key key{dev, (int)sizeof(T), set_.relaxation, set_.nrelax_pre,
                                       set_.nrelax_post, e.ii, e.jj, nl, e.nb, rep_};
             const int known = fused_start(key, -1);
             if (known >= 0) {
@@ -485,6 +481,7 @@ private:
             }
             const int top = *std::min_element(cand.begin(), cand.end());
             float tbest = -1.f;
+            bool steady = true;  // no candidate's two timings more than a quarter apart
             for (int c : cand) {
                 build_fused<T>(L, c, dst);
                 k2::fill<T>(L[top].b.p, T(0), L[top].ext.total(), stream_);
@@ -493,6 +490,7 @@ private:
                 float t = -1.f;
                 for (int round = 0; round < 2; ++round) {
                     const float tr = time_graph([&] { ncycle<T>(L, top, L[top].x, L[top].b); });
+                    steady = steady && tr >= 0.f && (t < 0.f || (tr <= 1.25f * t && t <= 1.25f * tr));
                     if (tr >= 0.f && (t < 0.f || tr < t)) t = tr;
                 }
                 if (t >= 0.f && (tbest < 0.f || t < tbest)) {
@@ -500,7 +498,8 @@ private:
                     lt = c;
                 }
             }
-            if (tbest >= 0.f) fused_start(key, lt);
+            // timings beside other work on the device choose for this solver alone
+            if (tbest >= 0.f && steady) fused_start(key, lt);
         }
         build_fused<T>(L, lt, dst);
     }

@@ -52,10 +52,16 @@ const char *cdr_hip_version(void);
  * direction and records the fastest in a process-wide table used by every later launch of the
  * same precision, stencil, direction, extents and batch size.  cdr_hip_autotune(0) turns it off
  * (shape 0 runs where nothing is recorded); returns the previous setting.
+ * Setup also times from which level down the 2D cycle runs fused in one launch, and records that per
+ * device, sizes and smoothing for later solvers, unless the timings were disturbed (two of one
+ * candidate more than a quarter apart); that choice never changes a result either.
  * cdr_hip_autotune_report writes the recorded choices as a JSON list into buf (len bytes,
- * NUL-terminated, truncated if short) and returns the full length. */
+ * NUL-terminated, truncated if short) and returns the full length: dir x, y, t (see below) for line
+ * shapes, f for the fused cycle, with the extents and index (shape) of its first level.
+ * cdr_hip_autotune_clear forgets all of them, pinned shapes included: later solvers time anew. */
 int cdr_hip_autotune(int on);
 int cdr_hip_autotune_report(char *buf, int len);
+void cdr_hip_autotune_clear(void);
 /* Number of candidate shapes for lines of direction dir (0: x, 1: y) at fp_bits (32 or 64)
  * precision, stencil nstncl and extents ii x jj; cdr_hip_set_line_shape2d pins one of them for
  * those extents and batch size nb (shape -1 removes the entry; returns a cdr_status).

@@ -43,3 +43,12 @@ def test_argument_errors_without_gpu():
     assert lib.cdr_hip_residual2d_f64(None, 5, None, None, None, 10, 10, None) == 1
     assert lib.cdr_hip_solver2d_create(None, 5, 10, 10, None, None, None) == 1
     assert lib.cdr_hip_norm_work2d(2, 2) == 0
+
+
+def test_forgotten_choices_without_gpu():
+    lib = _abi.load()
+    assert lib.cdr_hip_set_line_shape2d(0, 64, 5, 1026, 1026, 1, 0) == 0
+    buf = ctypes.create_string_buffer(4096)
+    assert lib.cdr_hip_autotune_report(buf, 4096) > 2 and buf.value.startswith(b'[{"dir":"x"')
+    lib.cdr_hip_autotune_clear()
+    assert lib.cdr_hip_autotune_report(buf, 4096) == 2 and buf.value == b"[]"

@@ -116,3 +116,38 @@ def test_closed_solvers_give_their_memory_back():
             assert C.memory_trim() <= limit
     finally:
         C.memory_limit(prev)
+
+
+def test_recorded_fused_starts_are_listed_and_forgotten():
+    """The first level of the fused cycle that a solver's setup chose is listed with its device, taken
+    over by the next solver, and forgotten with the line shapes; none of it changes a solution."""
+    import cedar_amd as C
+    so, b = _problem(300, 5)
+    prev = C.autotune(True)
+    mine = lambda: [r for r in C.autotune_report() if r["dir"] == "f" and "300 x 300" in r["kernel"]]
+    try:
+        C.autotune_clear()
+        assert C.autotune_report() == []
+        ref = None
+        for _ in range(6):  # disturbed timings are not recorded
+            s = C.Solver(so, **KW)
+            x, h = s.solve(b)
+            s.close()
+            ref = ref or (x, h)
+            assert torch.equal(x, ref[0]) and np.array_equal(h, ref[1])
+            if mine():
+                break
+        r, = mine()
+        assert r["device"] == torch.cuda.current_device() and r["fp"] == 64 and r["nb"] == 1
+        n = 300
+        for _ in range(r["shape"]):
+            n = (n - 1) // 2 + 1
+        assert n <= 128 and (r["ii"], r["jj"]) == (n + 2, n + 2)
+        s = C.Solver(so, **KW)
+        x, h = s.solve(b)
+        s.close()
+        assert mine() == [r] and torch.equal(x, ref[0]) and np.array_equal(h, ref[1])
+        C.autotune_clear()
+        assert C.autotune_report() == []
+    finally:
+        C.autotune(prev)
