@@ -33,6 +33,10 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=
          "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument"]
 
 
+def _command(src, obj):
+    return [HIPCC] + FLAGS + ["-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj]
+
+
 def _headers_mtime():
     hdrs = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hpp", ".h"))]
     inc = os.path.join(os.path.dirname(HERE), "include")
@@ -42,15 +46,20 @@ def _headers_mtime():
 
 def _compile(src, incremental=False):
     obj = os.path.join(OBJDIR, os.path.basename(src) + ".o")
-    if incremental and os.path.exists(obj):
+    cmd = _command(src, obj)
+    made_by = obj + ".cmd"  # the command the object was built with
+    if incremental and os.path.exists(obj) and os.path.exists(made_by):
         newest = max(os.path.getmtime(os.path.join(CSRC, src)), _headers_mtime())
-        if os.path.getmtime(obj) > newest:
-            return obj
-    lang = ["-x", "hip"] if src.endswith(".hip") else ["-x", "hip"]
-    cmd = [HIPCC] + FLAGS + lang + ["-c", os.path.join(CSRC, src), "-o", obj]
+        with open(made_by) as f:
+            if os.path.getmtime(obj) > newest and f.read() == "\n".join(cmd):
+                return obj
+    if os.path.exists(made_by):
+        os.remove(made_by)  # until the new object is there
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
+    with open(made_by, "w") as f:
+        f.write("\n".join(cmd))
     # the host pass does not know the packed-fp32 target feature; that warning is expected
     noise = [ln for ln in r.stderr.splitlines() if ln.strip() and "packed-fp32-ops" not in ln]
     if noise:
@@ -60,7 +69,7 @@ def _compile(src, incremental=False):
 
 def build(verbose=True, incremental=False):
     """Compiles every source (incremental=True skips objects newer than their source and every
-    header) and links the library."""
+    header that were built with the same command) and links the library."""
     os.makedirs(OBJDIR, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(len(SOURCES), 4)) as ex:
