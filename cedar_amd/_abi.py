@@ -120,6 +120,9 @@ PROTOTYPES = {
     "cdr_hip_solve_cg3d_f32": (_i, [_P, _P, _P, _i, _P, _i, _i, _i, _vp]),
     # 3D solver
     "cdr_hip_default_settings3": (None, [ctypes.POINTER(Settings3)]),
+    "cdr_hip_relax_gs7_to3d_f64": (_i, [_P, _P, _P, _P, _P, _P, _i, _i, _i, _i, _i, _i, _vp]),
+    "cdr_hip_relax_gs7_to3d_f32": (_i, [_P, _P, _P, _P, _P, _P, _i, _i, _i, _i, _i, _i, _vp]),
+    "cdr_hip_relax_gs7_to_pays3d": (_i, [_i, _i, _i]),
     "cdr_hip_relax_gs3d_per_f64": (_i, [_P, _i, _P, _P, _P, _i, _i, _i, _i, _i, _vp]),
     "cdr_hip_relax_gs3d_per_f32": (_i, [_P, _i, _P, _P, _P, _i, _i, _i, _i, _i, _vp]),
     "cdr_hip_restrict3d_per_f64": (_i, [_P, _P, _P, _i, _i, _i, _i, _i, _i, _i, _vp]),

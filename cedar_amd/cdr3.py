@@ -60,6 +60,19 @@ def relax_gs(so, qf, q, sor, updown):
     return q
 
 
+def relax_gs7_to(so, qf, q, out, sor, updown, ghosts=None, rows=0, planes=0):
+    """A 7-point sweep from q to out in one launch (the ghosts read are those of ghosts, else of q)."""
+    _abi.call(f"cdr_hip_relax_gs7_to3d_{_sfx(q)}", _p(so), _p(qf), _p(q), _p(out),
+              _p(q if ghosts is None else ghosts), _p(sor), *_dims(q), int(updown), int(rows),
+              int(planes), _stream())
+    return out
+
+
+def relax_gs7_to_pays(nx, ny, nz):
+    """Whether the solver takes the out-of-place sweep at these interior extents."""
+    return bool(_abi.load().cdr_hip_relax_gs7_to_pays3d(nx + 2, ny + 2, nz + 2))
+
+
 def restrict(ci, q, qc):
     _abi.call(f"cdr_hip_restrict3d_{_sfx(q)}", _p(ci), _p(q), _p(qc), *_dims(q), *_dims(qc),
               _stream())

@@ -46,11 +46,14 @@ bool relax_gs27_rows(const T *so, const T *qf, T *q, const T *sor, int ii, int j
 
 // A 7-point sweep in one launch, from q to out (another array).  The ghosts read are those of g and
 // no ghost is written, so a sweep to a scratch array and one back leave what two sweeps in place do.
-// gs7_sweep_pays: whether it is expected to take less time than relax_gs.
+// gs7_sweep_pays: whether it is expected to take less time than relax_gs.  rows (at most 14) and planes:
+// those of a workgroup, 0: chosen; gs7_shape_ok: whether such a launch is possible.  The result does not
+// depend on them.
 bool gs7_sweep_pays(int ii, int jj, int kk);
+bool gs7_shape_ok(int ii, int jj, int kk, int rows, int planes);
 template <typename T>
 void relax_gs7_sweep(const T *so, const T *qf, const T *q, T *out, const T *g, const T *sor, int ii,
-                     int jj, int kk, int updown, hipStream_t s);
+                     int jj, int kk, int updown, hipStream_t s, int rows = 0, int planes = 0);
 
 template <typename T>
 void restrict_(const T *ci, const T *q, T *qc, int iif, int jjf, int kkf, int iic, int jjc,

@@ -107,6 +107,16 @@ int interp3_per_t(T *q, const T *qc, const T *res, const T *so, int ns, const T 
 }
 
 template <typename T>
+int gs7_to3_t(const T *so, const T *qf, const T *q, T *out, const T *ghosts, const T *sor, int ii, int jj,
+              int kk, int ud, int rows, int planes, void *st) {
+    if (!so || !qf || !q || !out || !ghosts || !sor || q == out || !ext3_ok(ii, jj, kk) ||
+        (ud != CDR_DOWN && ud != CDR_UP) || !k3::gs7_shape_ok(ii, jj, kk, rows, planes))
+        return CDR_ERR_ARG;
+    k3::relax_gs7_sweep<T>(so, qf, q, out, ghosts, sor, ii, jj, kk, ud, S(st), rows, planes);
+    return launched();
+}
+
+template <typename T>
 int solve_cg3_per_t(T *q, const T *qf, const double *abd, double *bbd, int ii, int jj, int kk,
                     int jpn, void *st) {
     if (!q || !qf || !abd || !bbd || !ext3_ok(ii, jj, kk) || !jpn3_ok(jpn) ||
@@ -156,6 +166,20 @@ int cdr_hip_relax_gs3d_f64(const double *so, int ns, const double *qf, double *q
 int cdr_hip_relax_gs3d_f32(const float *so, int ns, const float *qf, float *q, const float *sor,
                            int ii, int jj, int kk, int ud, void *st) {
     return gs3_t<float>(so, ns, qf, q, sor, ii, jj, kk, ud, st);
+}
+
+int cdr_hip_relax_gs7_to3d_f64(const double *so, const double *qf, const double *q, double *out,
+                               const double *ghosts, const double *sor, int ii, int jj, int kk, int ud,
+                               int rows, int planes, void *st) {
+    return gs7_to3_t<double>(so, qf, q, out, ghosts, sor, ii, jj, kk, ud, rows, planes, st);
+}
+int cdr_hip_relax_gs7_to3d_f32(const float *so, const float *qf, const float *q, float *out,
+                               const float *ghosts, const float *sor, int ii, int jj, int kk, int ud,
+                               int rows, int planes, void *st) {
+    return gs7_to3_t<float>(so, qf, q, out, ghosts, sor, ii, jj, kk, ud, rows, planes, st);
+}
+int cdr_hip_relax_gs7_to_pays3d(int ii, int jj, int kk) {
+    return ext3_ok(ii, jj, kk) && k3::gs7_sweep_pays(ii, jj, kk) ? 1 : 0;
 }
 
 int cdr_hip_restrict3d_f64(const double *ci, const double *q, double *qc, int iif, int jjf,

@@ -181,20 +181,26 @@ struct sweep_shape {
 };
 
 // Slabs of planes such that the workgroups, one per CU, fill the chip's 256 a whole number of times
-// as far as the two extra planes of a slab (and the latency of its start) allow.
-sweep_shape shape_of(int ii, int jj, int kk) {
+// as far as the two extra planes of a slab (and the latency of its start) allow.  rows, planes: J and K
+// as given, where positive.
+sweep_shape shape_of(int ii, int jj, int kk, int rows = 0, int planes = 0) {
     sweep_shape r{};
     r.nchunk = std::max(1, ((ii - 1) / 2 - 2) / (LANES - 2) + 1);
     r.ntile = (jj - 2 + ROWS - 3) / (ROWS - 2);
     r.J = (jj - 2 + r.ntile - 1) / r.ntile;
+    if (rows > 0) {
+        r.J = rows;
+        r.ntile = (jj - 2 + rows - 1) / rows;
+    }
     const long columns = (long)r.nchunk * r.ntile;
     for (int n = 1; n <= std::min(kk - 2, 64); ++n) {
-        const int k = (kk - 2 + n - 1) / n;
+        const int k = planes > 0 ? planes : (kk - 2 + n - 1) / n;
         const long tiles = columns * ((kk - 2 + k - 1) / k), steps = (tiles + 255) / 256 * (k + 4);
         if (n == 1 || steps < r.steps) r.steps = steps, r.K = k, r.tiles = tiles;
     }
     return r;
 }
+constexpr long kMaxTiles = 1L << 30;
 
 }  // namespace
 
@@ -203,13 +209,18 @@ sweep_shape shape_of(int ii, int jj, int kk) {
 // (128^3: 65 pairs on two) and small levels stay with the two launches.
 bool gs7_sweep_pays(int ii, int jj, int kk) {
     const sweep_shape f = shape_of(ii, jj, kk);
-    return (double)f.steps * 4.9 < (double)ii * jj * kk * 26e-6 && f.tiles < (1L << 30);
+    return (double)f.steps * 4.9 < (double)ii * jj * kk * 26e-6 && f.tiles < kMaxTiles;
+}
+
+bool gs7_shape_ok(int ii, int jj, int kk, int rows, int planes) {
+    return rows >= 0 && rows <= ROWS - 2 && planes >= 0 && planes <= kk - 2 &&
+           shape_of(ii, jj, kk, rows, planes).tiles < kMaxTiles;
 }
 
 template <typename T>
 void relax_gs7_sweep(const T *so, const T *qf, const T *q, T *out, const T *g, const T *sor, int ii,
-                     int jj, int kk, int updown, hipStream_t s) {
-    const sweep_shape f = shape_of(ii, jj, kk);
+                     int jj, int kk, int updown, hipStream_t s, int rows, int planes) {
+    const sweep_shape f = shape_of(ii, jj, kk, rows, planes);
     gs7_sweep_k<T><<<(unsigned)((f.tiles + 7) / 8 * 8), LANES * ROWS, 0, s>>>(
         so, qf, q, out, g, sor, ii, jj, kk, updown == 0 ? 1 : 0, f.nchunk, f.ntile, (int)f.tiles, f.J,
         f.K);
@@ -217,9 +228,10 @@ void relax_gs7_sweep(const T *so, const T *qf, const T *q, T *out, const T *g, c
 
 template void relax_gs7_sweep<double>(const double *, const double *, const double *, double *,
                                       const double *, const double *, int, int, int, int,
-                                      hipStream_t);
+                                      hipStream_t, int, int);
 template void relax_gs7_sweep<float>(const float *, const float *, const float *, float *,
-                                     const float *, const float *, int, int, int, int, hipStream_t);
+                                     const float *, const float *, int, int, int, int, hipStream_t,
+                                     int, int);
 
 }  // namespace k3
 }  // namespace cdr

@@ -438,6 +438,18 @@ int cdr_hip_relax_gs3d_f64(const double *so, int nstncl, const double *qf, doubl
                            const double *sor, int ii, int jj, int kk, int updown, void *stream);
 int cdr_hip_relax_gs3d_f32(const float *so, int nstncl, const float *qf, float *q,
                            const float *sor, int ii, int jj, int kk, int updown, void *stream);
+/* The 7-point sweep in one launch instead of one per colour, out of place: from q to out (another
+ * array), bitwise the interior that cdr_hip_relax_gs3d leaves in q.  The ghosts read are those of
+ * `ghosts` (q itself, where q has them); none is written.  rows (1 to 14) and planes (1 to kk-2) of a
+ * workgroup, 0: chosen; the result does not depend on them.  The 3D solver takes this form in pairs of
+ * sweeps where cdr_hip_relax_gs7_to_pays3d is 1 (0 too for invalid extents). */
+int cdr_hip_relax_gs7_to3d_f64(const double *so, const double *qf, const double *q, double *out,
+                               const double *ghosts, const double *sor, int ii, int jj, int kk,
+                               int updown, int rows, int planes, void *stream);
+int cdr_hip_relax_gs7_to3d_f32(const float *so, const float *qf, const float *q, float *out,
+                               const float *ghosts, const float *sor, int ii, int jj, int kk,
+                               int updown, int rows, int planes, void *stream);
+int cdr_hip_relax_gs7_to_pays3d(int ii, int jj, int kk);
 /* BMG3_SymStd_restrict (src/3d/restrict.cc:7-10) */
 int cdr_hip_restrict3d_f64(const double *ci, const double *q, double *qc, int iif, int jjf,
                            int kkf, int iic, int jjc, int kkc, void *stream);

@@ -347,12 +347,127 @@ def _cycle3(C, lv, abd, l, x, b, pre, post):
         C.cdr3.relax_gs(so, b, x, sor, 1)
 
 
+def _op7(rand, shape):
+    so = torch.zeros((4,) + shape, device="cuda", dtype=torch.float64)
+    so[0, 1:-1, 1:-1, 1:-1] = 7.0
+    so[1, 1:-1, 1:-1, 1:] = 0.1 + 0.9 * rand(shape[0] - 2, shape[1] - 2, shape[2] - 1)
+    so[2, 1:-1, 1:, 1:-1] = 0.1 + 0.9 * rand(shape[0] - 2, shape[1] - 1, shape[2] - 2)
+    so[3, 1:, 1:-1, 1:-1] = 0.1 + 0.9 * rand(shape[0] - 1, shape[1] - 2, shape[2] - 2)
+    return so
+
+
+# One 7-point sweep out of place against the one in place, every shape of the launch by itself: 1 to 4
+# points a side; rows of one group of 62 pairs that is nearly full, full, one over, and of three; tiles
+# of 1, 3, 13 and 14 rows with and without a remainder; slabs of one plane, of all, and of lengths that
+# divide the planes and do not; a march of 25 and of 60 planes; 1, 255 to 257 and 1000 workgroups.
+# Ghosts are those of a third array (those of q and out are NaN), the rest of out stays.
+@pytest.mark.parametrize("dims,rows,planes", [
+    ((1, 1, 1), 0, 0), ((2, 1, 1), 0, 0), ((1, 2, 3), 1, 1), ((3, 3, 3), 0, 0), ((4, 4, 4), 3, 2),
+    ((4, 2, 3), 14, 3), ((3, 4, 1), 1, 1), ((121, 5, 4), 0, 0), ((122, 13, 9), 13, 3), ((123, 14, 9), 14, 4),
+    ((124, 15, 9), 14, 1), ((125, 28, 7), 14, 7), ((126, 29, 10), 14, 5), ((127, 9, 6), 3, 6),
+    ((247, 15, 4), 0, 0), ((371, 17, 5), 7, 2), ((200, 16, 50), 14, 25), ((130, 30, 60), 0, 60),
+    ((30, 60, 52), 14, 20), ((20, 51, 15), 3, 1), ((20, 16, 128), 14, 1), ((20, 3, 257), 3, 1),
+    ((140, 70, 100), 14, 1), ((200, 200, 200), 0, 0)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_gs7_sweep_shapes(dims, rows, planes, dtype):
+    import cedar_amd as C
+    print(f"\n7-point sweep {dims} rows {rows} planes {planes} {dtype}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(sum(dims) + rows + planes)
+    shape = tuple(n + 2 for n in dims[::-1])
+    rand = lambda *s: torch.rand(*s, generator=gen, device="cuda", dtype=torch.float64)
+    so = _op7(rand, shape)
+    sor = torch.zeros((2,) + shape, device="cuda", dtype=torch.float64)
+    C.cdr3.setup_recip(so, sor)
+    so, sor, f, x = (t.to(dtype) for t in (so, sor, rand(*shape) - 0.5, rand(*shape) - 0.5))
+    inner = (slice(1, -1),) * 3
+    q = torch.full_like(x, float("nan"))
+    q[inner] = x[inner]
+    ghosts = torch.full_like(x, float("nan"))
+    edge = torch.ones_like(x, dtype=torch.bool)
+    edge[inner] = False
+    ghosts[edge] = x[edge]
+    for ud in (0, 1):
+        want = C.cdr3.relax_gs(so, f, x.clone(), sor, ud)
+        out = torch.full_like(x, 7.0)
+        C.cdr3.relax_gs7_to(so, f, q, out, sor, ud, ghosts=ghosts, rows=rows, planes=planes)
+        assert torch.equal(out[inner], want[inner]), ud
+        assert bool((out[edge] == 7.0).all())
+
+
+def test_gs7_sweep_refuses_what_it_cannot_launch():
+    import cedar_amd as C
+    x, so, sor = (torch.zeros(n + (5, 5, 5), dtype=torch.float64, device="cuda") for n in ((), (4,), (2,)))
+    out = torch.zeros_like(x)
+    for rows, planes in ((15, 1), (-1, 1), (1, 4), (1, -1)):
+        with pytest.raises(C.CedarHipError):
+            C.cdr3.relax_gs7_to(so, x, x, out, sor, 0, rows=rows, planes=planes)
+    with pytest.raises(C.CedarHipError):
+        C.cdr3.relax_gs7_to(so, x, x, x, sor, 0)
+
+
+# the cycles of test_gs7_sweeps take the out-of-place form at their sizes, small levels do not
+@pytest.mark.parametrize("dims,taken", [((125, 97, 104), True), ((126, 167, 59), True),
+                                        ((126, 65, 152), True), ((117, 70, 152), True),
+                                        ((249, 70, 71), True), ((248, 97, 53), True),
+                                        ((373, 53, 62), True), ((200, 200, 200), True),
+                                        ((63, 63, 63), False), ((3, 3, 3), False)])
+def test_gs7_sweep_sizes(dims, taken):
+    import cedar_amd as C
+    assert C.cdr3.relax_gs7_to_pays(*dims) == taken
+
+
+def _fmg3(C, lv, abd, l, x, b, pre, post):
+    """The F-cycle from the finest level down, every sweep in place."""
+    so, ci, sor = lv[l]
+    if l == len(lv) - 1:
+        C.cdr3.solve_cg(x, b, abd)
+        return
+    ci = lv[l + 1][1]
+    bc, xc = torch.zeros_like(lv[l + 1][0][0]), torch.zeros_like(lv[l + 1][0][0])
+    C.cdr3.restrict(ci, b, bc)
+    _fmg3(C, lv, abd, l + 1, xc, bc, pre, post)
+    x.zero_()
+    C.cdr3.interp_add(x, xc, torch.zeros_like(x), so, ci)
+    _cycle3(C, lv, abd, l, x, b, pre, post)
+
+
+# an F-cycle enters the V-cycle with the residual's array written; the sweeps borrow that array
+@pytest.mark.parametrize("dims", [(125, 97, 104), (126, 167, 59)])
+@pytest.mark.parametrize("pre,post", [(2, 1), (1, 2)])
+def test_gs7_sweeps_in_f_cycles(dims, pre, post):
+    import cedar_amd as C
+    print(f"\nF-cycle, 7-point sweeps {dims} {pre},{post}", flush=True)
+    assert C.cdr3.relax_gs7_to_pays(*dims)
+    gen = torch.Generator(device="cuda").manual_seed(sum(dims) + pre)
+    shape = tuple(n + 2 for n in dims[::-1])
+    rand = lambda *s: torch.rand(*s, generator=gen, device="cuda", dtype=torch.float64)
+    so = _op7(rand, shape)
+    b = torch.zeros(shape, device="cuda", dtype=torch.float64)
+    b[1:-1, 1:-1, 1:-1] = rand(*dims[::-1]) - 0.5
+    s = C.Solver3(so, nrelax_pre=pre, nrelax_post=post, maxiter=1, tol=1e-30, cycle="f")
+    lv = []
+    for l in range(s.nlevels):
+        a, ci = s.level_arrays(l)
+        a = dev(a)
+        sor = torch.zeros((2,) + tuple(a.shape[1:]), device="cuda", dtype=torch.float64)
+        C.cdr3.setup_recip(a, sor)
+        lv.append((a, None if ci is None else dev(ci), sor))
+    abd = C.cdr3.setup_cg(lv[-1][0])
+    want, got = torch.zeros_like(b), torch.zeros_like(b)
+    for _ in range(2):  # the second one finds the arrays as the first one left them
+        s.vcycle(got, b)
+        _fmg3(C, lv, abd, 0, want, b, pre, post)
+        assert torch.equal(got, want)
+
+
 # 7-point sweeps that take both colours in one launch: one to three groups of 62 pairs along a row,
 # the last one full, nearly full or short, odd and even; tiles of 14 rows with and without a
-# remainder, slabs likewise; couplings to the ghosts of a nonzero boundary; odd and even numbers of
-# sweeps.  The sizes are about the smallest that take this path.
+# remainder, slabs of three planes with one of two; couplings to the ghosts of a nonzero boundary; odd
+# and even numbers of sweeps.  The sizes are about the smallest that take this path (asserted in
+# test_gs7_sweep_sizes); test_gs7_sweep_shapes has the other slabs.
 @pytest.mark.parametrize("dims", [(125, 96, 104), (126, 167, 59), (126, 65, 152), (117, 70, 152),
-                                  (249, 70, 71), (248, 94, 53), (373, 53, 62)])
+                                  (249, 70, 71), (248, 94, 53), (373, 53, 62), (125, 97, 104),
+                                  (248, 97, 53)])
 @pytest.mark.parametrize("pre,post", [(2, 1), (1, 2), (3, 0)])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_gs7_sweeps(dims, pre, post, dtype):
