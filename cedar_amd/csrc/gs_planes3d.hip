@@ -204,12 +204,19 @@ constexpr long kMaxTiles = 1L << 30;
 
 }  // namespace
 
-// The march takes 4.9 us per plane and CU in FP64 (200^3: 142 us), two launches of one colour 26 ps
-// per point (200^3: 218 us); FP32 about 0.6 of either.  Rows that leave most of a wavefront idle
-// (128^3: 65 pairs on two) and small levels stay with the two launches.
+// The march takes 4.9 us per plane and CU in FP64 (200^3: 142 us) and less where its arrays stay in the
+// last cache (120^3: 30 us for 9 planes), two launches of one colour 23 to 30 ps per point (200^3: 216
+// us); FP32 about 0.6 of either.  Over 132 sizes of up to 25 million points, most of them about the line,
+// what is taken is 0.99 to 2.4 times as fast, 1.6 in the middle.  Rows that leave most of a wavefront idle (128^3: 65 pairs on two)
+// and small levels stay with the two launches; so do planes whose workgroups are a multiple of 8 up to
+// 1.6 million points: each XCD then finds its rows of the plane before in its own cache, and the two
+// launches take 17 ps per point (125 x 96 x 104: 22 us, the march 26; 122 x 157 x 77: 26 and 28).
 bool gs7_sweep_pays(int ii, int jj, int kk) {
     const sweep_shape f = shape_of(ii, jj, kk);
-    return (double)f.steps * 4.9 < (double)ii * jj * kk * 26e-6 && f.tiles < kMaxTiles;
+    const double points = (double)ii * jj * kk;
+    const int plane_groups = ((ii - 1) / 2 + 63) / 64 * ((jj - 2 + 3) / 4);  // of relax_gs
+    if (plane_groups % 8 == 0 && points <= 1.6e6) return false;
+    return (double)f.steps * 4.9 < points * 26e-6 && f.tiles < kMaxTiles;
 }
 
 bool gs7_shape_ok(int ii, int jj, int kk, int rows, int planes) {
