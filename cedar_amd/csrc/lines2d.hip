@@ -129,8 +129,31 @@ struct seg_map {
 // chunk u's right-hand sides; afun(u) returns its multipliers a_k (reloaded when needed, so that
 // only b stays in registers) and dval(u) its pivots.  On exit b[u] = y_k / d_k.  xch: this
 // line's LDS slots, one per chunk of the line.
-template <typename T, int CPW, int W, typename AF, typename DF>
+// AHEAD > 1 (W == 1): the multipliers and pivots of AHEAD chunks are loaded at a time.
+template <typename T, int CPW, int W, int AHEAD = 1, typename AF, typename DF>
 __device__ inline void seg_forward(T (&b)[CPW], AF afun, DF dval, seg_map<T> *xch, int w) {
+    if constexpr (AHEAD > 1) {
+        static_assert(W == 1 && CPW % AHEAD == 0, "whole groups of a line's one segment");
+        T carry = T(0);
+#pragma unroll
+        for (int g = 0; g < CPW; g += AHEAD) {
+            T a[AHEAD], d[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                a[u] = afun(g + u);
+                d[u] = dval(g + u);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                scan_affine_dpp(a[u], b[g + u]);
+                const T y = affine(a[u], carry, b[g + u]);
+                carry = last_lane(y);
+                b[g + u] = div_pivot(y, d[u]);
+            }
+        }
+        return;
+    }
     if (W > 1) {
 #pragma unroll
         for (int u = 0; u < CPW; ++u) {
@@ -162,8 +185,27 @@ __device__ inline void seg_forward(T (&b)[CPW], AF afun, DF dval, seg_map<T> *xc
 // c holds element 64c + 63 - l); the carry runs from the line's last chunk to its first.
 // coef(u, a, b[u]) turns b[u] (the forward results) into the chunk's coefficients and returns
 // the multipliers in a; afun(u) returns the multipliers alone.  On exit b[u] = x.
-template <typename T, int CPW, int W, typename CF, typename AF>
+template <typename T, int CPW, int W, int AHEAD = 1, typename CF, typename AF>
 __device__ inline void seg_backward(T (&b)[CPW], CF coef, AF afun, seg_map<T> *xch, int w) {
+    if constexpr (AHEAD > 1) {
+        static_assert(W == 1 && CPW % AHEAD == 0, "whole groups of a line's one segment");
+        T carry = T(0);
+#pragma unroll
+        for (int g = CPW - AHEAD; g >= 0; g -= AHEAD) {
+            T a[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) coef(g + u, a[u], b[g + u]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = AHEAD - 1; u >= 0; --u) {
+                scan_affine_dpp(a[u], b[g + u]);
+                const T x = affine(a[u], carry, b[g + u]);
+                carry = last_lane(x);
+                b[g + u] = x;
+            }
+        }
+        return;
+    }
     if (W > 1) {
 #pragma unroll
         for (int u = 0; u < CPW; ++u) {
@@ -430,6 +472,10 @@ __global__ __launch_bounds__(NC *W * 64) void relax_ylines_seg_k(const T *__rest
     // not when the scans reach them: per colour, 10.2 -> 8.5 us at 511^2 in FP32, 9.9 -> 8.2 at
     // 750 x 550 in FP64
     constexpr bool PRE = CPW * sizeof(T) <= 64;
+    // The longest FP32 segments have no registers for that; left to itself the compiler loaded their
+    // factors one at a time (five-point, per sweep: 4090^2 295 us, in groups of 8 149, of 4 159; 3000^2
+    // 177 and 107).
+    constexpr int AHEAD = W == 1 && CPW == 64 && sizeof(T) == 4 ? 8 : 1;
     T pe[PRE ? CPW : 1], pd[PRE ? CPW : 1], pb[PRE ? CPW : 1];
     auto fwd_a = [&](int u) {  // forward coefficient of chunk u
         const int k = (w * CPW + u) * WAVE + lane;
@@ -508,8 +554,8 @@ __global__ __launch_bounds__(NC *W * 64) void relax_ylines_seg_k(const T *__rest
         for (int u = 0; u < CPW; ++u) bwd_coef(u, a[u], b[u]);
         seg_backward_ab<T, CPW, W>(a, b, xch[1][cs], w);
     } else {
-        seg_forward<T, CPW, W>(b, fwd_a, pivot, xch[0][cs], w);
-        seg_backward<T, CPW, W>(b, bwd_coef, bwd_a, xch[1][cs], w);
+        seg_forward<T, CPW, W, AHEAD>(b, fwd_a, pivot, xch[0][cs], w);
+        seg_backward<T, CPW, W, AHEAD>(b, bwd_coef, bwd_a, xch[1][cs], w);
     }
 #pragma unroll
     for (int g = 0; g < CPW; g += G) {

@@ -356,6 +356,30 @@ def _op7(rand, shape):
     return so
 
 
+# A five-point sweep moves 8 values a point where a nine-point one moves 12: it takes 0.57 of its time
+# when it waits for memory alone, and took 1.07 of it when its factors were loaded one at a time.
+def test_long_fp32_y_lines_load_their_factors_in_groups():
+    import cedar_amd as C
+    n, best = 4090, {}
+    for ns in (3, 5):
+        so = torch.full((ns, n + 2, n + 2), 0.5, device="cuda")
+        so[0] = 9.0
+        sor = torch.full((2, n + 2, n + 2), 0.1, device="cuda")
+        sor[0] = 9.0
+        f, q = torch.rand_like(so[0]), torch.rand_like(so[0])
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            C.relax_lines(so, f, q, sor, 0, "y")
+            a.record()
+            for _ in range(10):
+                C.relax_lines(so, f, q, sor, 0, "y")
+            b.record()
+            b.synchronize()
+            best[ns] = min(best.get(ns, 1e9), a.elapsed_time(b) / 10)
+    print(f"\nFP32 y-lines of {n} points: {best}", flush=True)
+    assert best[3] < 0.85 * best[5], best
+
+
 # One 7-point sweep out of place against the one in place, every shape of the launch by itself: 1 to 4
 # points a side; rows of one group of 62 pairs that is nearly full, full, one over, and of three; tiles
 # of 1, 3, 13 and 14 rows with and without a remainder; slabs of one plane, of all, and of lengths that
