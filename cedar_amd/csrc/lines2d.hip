@@ -331,6 +331,10 @@ __global__ __launch_bounds__(L *W * 64) void relax_xlines_seg_k(const T *__restr
     // arrive during the forward scans and the exchange.  FP32, per colour: 77.5 -> 74.4 us at 4095^2,
     // 21.8 -> 19.1 at 2048^2, about 5 % on the levels below.
     constexpr bool PRE = CPW * sizeof(T) <= 16, MID = !PRE && W > 1 && CPW * sizeof(T) <= 64;
+    // FP32 lines of one wavefront and 8 to 17 chunks load a chunk ahead of the one they scan: left to the
+    // compiler the loads came late, 24.3 us per nine-point sweep at 1080^2 (20.9 before its registers
+    // were dealt anew for PRE and MID), 26.6 at 1000 x 2048; 16.0 and 19.8.
+    constexpr bool PIPE = W == 1 && !PRE && sizeof(T) == 4 && CPW >= 8 && CPW <= 17;
     line_raw<T> raw[PRE ? CPW : 1];
     T pe[PRE ? CPW : 1], pd[PRE || MID ? CPW : 1], pb[PRE || MID ? CPW : 1];
     if constexpr (PRE) {
@@ -381,14 +385,37 @@ __global__ __launch_bounds__(L *W * 64) void relax_xlines_seg_k(const T *__restr
     if constexpr (W == 1) {
         // one wavefront per line: scan and carry chunk by chunk, only the results kept
         T carry = T(0);
+        if constexpr (PIPE) {
+            line_raw<T> r[2];
+            T e[2], d[2];
+            auto load = [&](int u) {
+                const int kc = min(u * WAVE + lane, n - 1);
+                line_load<T, NINE, 0>(r[u % 2], so, qf, q, P, ii, row + kc + 1, ZQ);
+                e[u % 2] = E[max(kc - 1, 0)];
+                d[u % 2] = D[kc];
+            };
+            load(0);
 #pragma unroll
-        for (int u = 0; u < CPW; ++u) {
-            T au, bu;
-            fwd_coef(u, au, bu);
-            scan_affine_dpp(au, bu);
-            const T y = affine(au, carry, bu);
-            carry = last_lane(y);
-            b[u] = div_pivot(y, pivot(u));
+            for (int u = 0; u < CPW; ++u) {
+                if (u + 1 < CPW) load(u + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                T bu = line_rhs<T, NINE, TR>(r[u % 2]);
+                T au = u * WAVE + lane > 0 ? -e[u % 2] : T(0);
+                scan_affine_dpp(au, bu);
+                const T y = affine(au, carry, bu);
+                carry = last_lane(y);
+                b[u] = div_pivot(y, d[u % 2]);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < CPW; ++u) {
+                T au, bu;
+                fwd_coef(u, au, bu);
+                scan_affine_dpp(au, bu);
+                const T y = affine(au, carry, bu);
+                carry = last_lane(y);
+                b[u] = div_pivot(y, pivot(u));
+            }
         }
         carry = T(0);
 #pragma unroll
