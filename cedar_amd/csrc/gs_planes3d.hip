@@ -41,7 +41,7 @@ __device__ inline T pick(int c, T a, T b) {
 // registers; the operands of plane k + 2 are on their way meanwhile.  Ghosts are read from g and
 // never written.  Bound by HBM: a sweep reads the operator, its reciprocal diagonal, the right-hand
 // side and the iterate once instead of once per colour, the halos (a quarter more) mostly from L2.
-// 200^3 in FP64: 142 us against 2 x 109.
+// 200^3 in FP64: 142 us against 2 x 109 (gs7_sweep_pays has the other sizes).
 template <typename T>
 __global__ __launch_bounds__(LANES *ROWS) void gs7_sweep_k(
     const T *__restrict__ so, const T *__restrict__ qf, const T *__restrict__ q,
@@ -206,11 +206,12 @@ constexpr long kMaxTiles = 1L << 30;
 
 // The march takes 4.9 us per plane and CU in FP64 (200^3: 142 us) and less where its arrays stay in the
 // last cache (120^3: 30 us for 9 planes), two launches of one colour 23 to 30 ps per point (200^3: 216
-// us); FP32 about 0.6 of either.  Over 132 sizes of up to 25 million points, most of them about the line,
-// what is taken is 0.99 to 2.4 times as fast, 1.6 in the middle.  Rows that leave most of a wavefront idle (128^3: 65 pairs on two)
-// and small levels stay with the two launches; so do planes whose workgroups are a multiple of 8 up to
-// 1.6 million points: each XCD then finds its rows of the plane before in its own cache, and the two
-// launches take 17 ps per point (125 x 96 x 104: 22 us, the march 26; 122 x 157 x 77: 26 and 28).
+// us); FP32 about 0.6 of either.  Over 132 sizes of up to 25 million points, most of them about the
+// line, what is taken is 0.99 to 2.4 times as fast, 1.6 in the middle.  Rows that leave most of a
+// wavefront idle (128^3: 65 pairs on two) and small levels stay with the two launches; so do planes
+// whose workgroups are a multiple of 8 up to 1.6 million points: each XCD then finds its rows of the
+// plane before in its own cache, and the two launches take 17 ps per point (125 x 96 x 104: 22 us, the
+// march 26; 122 x 157 x 77: 26 and 28).
 bool gs7_sweep_pays(int ii, int jj, int kk) {
     const sweep_shape f = shape_of(ii, jj, kk);
     const double points = (double)ii * jj * kk;

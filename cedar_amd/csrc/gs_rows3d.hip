@@ -25,11 +25,9 @@ constexpr int row_threads = W < 64 ? 64 : 256;
 // while the compiler waited for a few loads at a time).
 template <typename T, int W, bool ODD>
 __global__ __launch_bounds__(row_threads<W>, 1) __attribute__((amdgpu_waves_per_eu(1, 2)))
-void gs27_rows_k(const T *__restrict__ so,
-                                                   const T *__restrict__ qf, T *__restrict__ q,
-                                                   const T *__restrict__ sor, int ii, int jj,
-                                                   int kk, int j0, int k0, int nj, int rows,
-                                                   int rev) {
+void gs27_rows_k(const T *__restrict__ so, const T *__restrict__ qf, T *__restrict__ q,
+                 const T *__restrict__ sor, int ii, int jj, int kk, int j0, int k0, int nj, int rows,
+                 int rev) {
     constexpr int R = row_threads<W> / W;
     __shared__ T fresh[R][W + 2];  // [t + 1]: the first colour's value of pair t
     const int t = threadIdx.x % W, r = threadIdx.x / W;
