@@ -163,16 +163,13 @@ std::size_t pool_trim() {
     return release(out);
 }
 
-void pool_idle_scope::enter(hipError_t waited) {
-    prev_ = idle_device;
-    if (waited == hipSuccess)
+pool_idle_scope::pool_idle_scope(hipStream_t s) : prev_(idle_device) {
+    idle_device = -1;
+    if (hipStreamSynchronize(s) == hipSuccess)
         idle_device = current_device();
     else
         (void)hipGetLastError();  // blocks then go back through hipFree, which waits itself
 }
-
-pool_idle_scope::pool_idle_scope() { enter(hipDeviceSynchronize()); }
-pool_idle_scope::pool_idle_scope(hipStream_t s) { enter(hipStreamSynchronize(s)); }
 pool_idle_scope::~pool_idle_scope() { idle_device = prev_; }
 
 hipStream_t pool_capture_stream(hipError_t *e) {

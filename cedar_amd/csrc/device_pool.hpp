@@ -33,28 +33,34 @@ void *pool_malloc(std::size_t bytes, hipError_t *e);
 void pool_free(void *p) noexcept;
 
 // While alive, blocks of the current device that this thread frees are idle: nothing queued uses
-// them.  The constructor waits for the device, or for the stream that alone used them.
+// them.  The constructor waits for the stream that alone used them, and not for the device: that
+// breaks every capture in the process, whichever thread captures and in whatever mode, where hipFree
+// leaves those of other threads alone.
 class pool_idle_scope {
 public:
-    pool_idle_scope();
     explicit pool_idle_scope(hipStream_t s);
     ~pool_idle_scope();
     pool_idle_scope(const pool_idle_scope &) = delete;
     pool_idle_scope &operator=(const pool_idle_scope &) = delete;
 
 private:
-    void enter(hipError_t waited);
     int prev_;
 };
 
-// First member of a class that owns buffers: its destructor calls enter(), and as the first member
-// is destroyed last, the members after it give their blocks back idle.
+// First member of a class that owns buffers used on stream s: its destructor calls enter(s), and as the
+// first member is destroyed last, the members after it give their blocks back idle.  Where the caller
+// has been given pointers to the buffers (lend), work of its own on other streams may use them, so
+// they go back through hipFree, which waits for the device.
 class pool_guard {
 public:
-    void enter() { scope_.emplace(); }
+    void lend() { lent_ = true; }
+    void enter(hipStream_t s) {
+        if (!lent_) scope_.emplace(s);
+    }
 
 private:
     std::optional<pool_idle_scope> scope_;
+    bool lent_ = false;
 };
 
 // A non-blocking stream of the current device for captures alone (no work runs on it, so the next

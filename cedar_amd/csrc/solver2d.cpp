@@ -330,6 +330,7 @@ int cdr_hip_solver2d_level(const cdr_hip_solver2d *slv, int lvl, int *nx, int *n
                            const double **sor1) {
     if (!slv || lvl < 0 || lvl >= slv->impl->nlevels()) return CDR_ERR_ARG;
     const auto &L = slv->impl->level(lvl);
+    if (so || ci || sor0 || sor1) slv->impl->lend();
     if (nx) *nx = L.ext.nx();
     if (ny) *ny = L.ext.ny();
     if (so) *so = L.A.p;

@@ -70,7 +70,7 @@ public:
     }
 
     ~solver2d() {
-        guard_.enter();
+        guard_.enter(stream_);
         for (auto *g : {&g64_, &g32_})
             if (g->exec) (void)hipGraphExecDestroy(g->exec);
         pool_return_capture_stream(cap_stream_);
@@ -84,6 +84,8 @@ public:
     int nbatch() const { return L64_[0].ext.nb; }  // problems (operators x right-hand sides)
     int nrep() const { return rep_; }
     const level_data<double> &level(int l) const { return L64_[l]; }
+    // the caller keeps pointers to the levels' arrays
+    void lend() { guard_.lend(); }
     double setup_seconds() const { return setup_s_; }
     double solve_seconds() const { return solve_s_; }
     kernel_manager &kernels() { return km_; }

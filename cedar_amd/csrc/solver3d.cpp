@@ -381,7 +381,7 @@ public:
         build(so_dev, ns, nx, ny, nz);
     }
     ~solver3d() {
-        guard_.enter();
+        guard_.enter(stream_);
         (void)hipEventDestroy(ev0_);
         (void)hipEventDestroy(ev1_);
         if (host_norm_) (void)hipHostFree(host_norm_);
@@ -389,6 +389,8 @@ public:
 
     int nlevels() const { return (int)L_.size(); }
     const level3 &level(int l) const { return L_[l]; }
+    // the caller keeps pointers to the levels' arrays
+    void lend() { guard_.lend(); }
     double setup_seconds() const { return setup_s_; }
     double solve_seconds() const { return solve_s_; }
     bool mixed() const { return set_.precision == CDR_PREC_MIXED; }
@@ -865,6 +867,7 @@ int cdr_hip_solver3d_level(const cdr_hip_solver3d *slv, int lvl, int *nx, int *n
                            const double **so, const double **ci) {
     if (!slv || lvl < 0 || lvl >= slv->impl->nlevels()) return CDR_ERR_ARG;
     const auto &L = slv->impl->level(lvl);
+    if (so || ci) slv->impl->lend();
     if (nx) *nx = L.e.ii - 2;
     if (ny) *ny = L.e.jj - 2;
     if (nz) *nz = L.e.kk - 2;

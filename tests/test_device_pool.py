@@ -47,8 +47,7 @@ inline hipError_t hipFree(void *p) {
     std::free(p);
     return hipSuccess;
 }
-inline hipError_t hipDeviceSynchronize() { return fake::busy ? hipErrorUnknown : hipSuccess; }
-inline hipError_t hipStreamSynchronize(hipStream_t) { return hipDeviceSynchronize(); }
+inline hipError_t hipStreamSynchronize(hipStream_t) { return fake::busy ? hipErrorUnknown : hipSuccess; }
 inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, int) {
     *s = new fake_stream{fake::device};
     ++fake::streams;
@@ -70,7 +69,7 @@ PROGRAM = r"""
 using namespace cedar::hip;
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
 static void *get(std::size_t n) { hipError_t e; return pool_malloc(n, &e); }
-static void give(void *p) { pool_idle_scope s; pool_free(p); }
+static void give(void *p) { pool_idle_scope s(nullptr); pool_free(p); }
 int main() {
     const std::size_t K = 1024, first = pool_set_limit(8 * K);
     std::printf("%zu\n", first);
@@ -85,15 +84,35 @@ int main() {
     fake::device = 0;
     void *c = get(K);
     CHECK(c != a && get(2 * K) == a);
-    // not idle: outside a scope, of another device, and where the device cannot be waited for
+    // not idle: outside a scope, of another device, where the stream cannot be waited for (inside a
+    // scope of another stream too), and where the caller has been given pointers
     pool_free(c);
     CHECK(fake::used == 2 * K);
-    { pool_idle_scope s; fake::device = 1; void *o = get(K); pool_free(o); fake::device = 0; }
+    { pool_idle_scope s(nullptr); fake::device = 1; void *o = get(K); pool_free(o); fake::device = 0; }
     CHECK(fake::used == 2 * K);
     fake::busy = true;
     give(a);
     fake::busy = false;
     CHECK(fake::used == 0);
+    a = get(K);
+    {
+        pool_idle_scope s(nullptr);
+        fake::busy = true;
+        give(a);
+        fake::busy = false;
+        CHECK(fake::used == 0);
+        pool_free(get(K));  // the outer scope holds again
+        CHECK(fake::used == K && pool_trim() == K);
+    }
+    for (bool lent : {true, false}) {
+        void *p = get(K);
+        pool_guard guard;
+        if (lent) guard.lend();
+        guard.enter(nullptr);
+        pool_free(p);
+        CHECK(fake::used == (lent ? 0 : K));
+    }
+    CHECK(pool_trim() == K);
     // the ones kept longest go beyond the limit; one larger than it is never kept
     std::vector<void *> v;
     for (int i = 0; i < 5; ++i) v.push_back(get(2 * K));

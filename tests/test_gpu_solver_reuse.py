@@ -151,3 +151,104 @@ def test_recorded_fused_starts_are_listed_and_forgotten():
         assert C.autotune_report() == []
     finally:
         C.autotune(prev)
+
+
+# Solvers built, used and closed beside a capture of the caller's, in the modes that allow it: another
+# thread's work beside a thread-local or relaxed capture, and a close inside a relaxed one
+@pytest.mark.parametrize("mode,thread,what", [("thread_local", True, "close"), ("thread_local", True, "new"),
+                                              ("relaxed", True, "close"), ("relaxed", True, "new"),
+                                              ("relaxed", False, "close")])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_solvers_beside_a_capture(mode, thread, what, dim):
+    import cedar_amd as C
+    print(f"\n{dim}D solver, {what} beside a {mode} capture, other thread: {thread}", flush=True)
+    if dim == 2:
+        so, b = _problem(96, 1)
+        build = lambda: C.Solver(so, **KW)
+    else:
+        so, b, _ = G.poisson3_sine(17)
+        so, b = torch.as_tensor(so).cuda(), torch.as_tensor(b).cuda()
+        build = lambda: C.Solver3(so, relaxation="plane-xy", maxiter=3)
+    held = build()
+    ref = held.solve(b)
+    x, y = torch.ones(1000, device="cuda"), torch.zeros(1000, device="cuda")
+    torch.cuda.synchronize()
+    g, got = torch.cuda.CUDAGraph(), []
+
+    def act():
+        try:
+            if what == "close":
+                held.close()
+            else:
+                s = build()
+                got.append(s.solve(b))
+                s.close()
+        except Exception as exc:  # reported below
+            got.append(exc)
+
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode=mode):
+        y.add_(x)
+        if thread:
+            t = threading.Thread(target=act)
+            t.start()
+            t.join()
+        else:
+            act()
+        y.add_(x)
+    for _ in range(3):
+        g.replay()
+    torch.cuda.synchronize()
+    assert bool((y == 6).all())
+    if what == "close":
+        assert got == []
+    else:
+        assert torch.equal(got[0][0], ref[0]) and np.array_equal(got[0][1], ref[1])
+
+
+def test_threads_that_capture_while_others_close():
+    """Every solver times and captures its cycles anew while three other threads close theirs."""
+    import cedar_amd as C
+    sizes = (65, 66, 96, 97)
+    probs = {n: _problem(n, n) for n in sizes}
+    ref = {n: C.Solver(probs[n][0], **KW).solve(probs[n][1]) for n in sizes}
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for r in range(4):
+                    n = sizes[(k + r) % len(sizes)]
+                    s = C.Solver(probs[n][0], **KW)
+                    x, h = s.solve(probs[n][1])
+                    s.close()
+                    if not (torch.equal(x, ref[n][0]) and np.array_equal(h, ref[n][1])):
+                        bad.append((k, r, n))
+                torch.cuda.current_stream().synchronize()
+        except BaseException as exc:  # reported by the main thread
+            bad.append(exc)
+
+    for _ in range(20):
+        C.autotune_clear()
+        ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert not bad, bad
+
+
+def test_a_solver_whose_level_pointers_were_given_out_leaves_nothing():
+    """Work of the caller's own on another stream may still use such a pointer after the solver is
+    destroyed, so its blocks go back to the device and not to the next solver."""
+    import cedar_amd as C
+    so, b = _problem(200, 2)
+    for give in (True, False):
+        s = C.Solver(so, **KW)
+        s.solve(b)
+        if give:
+            assert s.level(1)[2]
+        C.memory_trim()  # what setup itself gave back
+        s.close()
+        left = C.memory_trim()
+        assert left == 0 if give else left > 5 * 202 * 202 * 8
