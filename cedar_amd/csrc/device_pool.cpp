@@ -48,6 +48,7 @@ pool &the_pool() {
 }
 
 thread_local int idle_device = -1;  // the device whose freed blocks are idle, or -1
+thread_local int busy_scopes = 0;   // open pool_busy_scopes
 
 int current_device() {
     int d = 0;
@@ -119,7 +120,7 @@ void pool_free(void *p) noexcept {
         mine.front() = it == P.live.end() ? block{p, 0, -1} : it->second;
         if (it != P.live.end()) P.live.erase(it);
         const block &b = mine.front();
-        if (b.device < 0 || b.device != idle_device || b.bytes > P.limit) {
+        if (b.device < 0 || b.device != idle_device || busy_scopes > 0 || b.bytes > P.limit) {
             out.splice(out.end(), mine);
         } else {
             P.kept_bytes += b.bytes;
@@ -165,12 +166,16 @@ std::size_t pool_trim() {
 
 pool_idle_scope::pool_idle_scope(hipStream_t s) : prev_(idle_device) {
     idle_device = -1;
+    if (busy_scopes > 0) return;
     if (hipStreamSynchronize(s) == hipSuccess)
         idle_device = current_device();
     else
         (void)hipGetLastError();  // blocks then go back through hipFree, which waits itself
 }
 pool_idle_scope::~pool_idle_scope() { idle_device = prev_; }
+
+pool_busy_scope::pool_busy_scope() { ++busy_scopes; }
+pool_busy_scope::~pool_busy_scope() { --busy_scopes; }
 
 hipStream_t pool_capture_stream(hipError_t *e) {
     pool &P = the_pool();

@@ -47,19 +47,39 @@ private:
     int prev_;
 };
 
+// While alive, no block that this thread frees is idle, whatever scope is opened inside.
+class pool_busy_scope {
+public:
+    pool_busy_scope();
+    ~pool_busy_scope();
+    pool_busy_scope(const pool_busy_scope &) = delete;
+    pool_busy_scope &operator=(const pool_busy_scope &) = delete;
+};
+
 // First member of a class that owns buffers used on stream s: its destructor calls enter(s), and as the
-// first member is destroyed last, the members after it give their blocks back idle.  Where the caller
-// has been given pointers to the buffers (lend), work of its own on other streams may use them, so
-// they go back through hipFree, which waits for the device.
+// first member is destroyed last, the members after it give their blocks back idle.  Where work of the
+// caller's own on other streams may use the buffers (lend: it has pointers to them; lend_if_captured:
+// it records what is enqueued on s into a graph), they go back through hipFree, which waits for the
+// device.
 class pool_guard {
 public:
     void lend() { lent_ = true; }
+    void lend_if_captured(hipStream_t s) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        const hipError_t e = hipStreamIsCapturing(s, &st);
+        if (e != hipSuccess) (void)hipGetLastError();
+        if (e != hipSuccess || st != hipStreamCaptureStatusNone) lent_ = true;
+    }
     void enter(hipStream_t s) {
-        if (!lent_) scope_.emplace(s);
+        if (lent_)
+            busy_.emplace();
+        else
+            idle_.emplace(s);
     }
 
 private:
-    std::optional<pool_idle_scope> scope_;
+    std::optional<pool_idle_scope> idle_;
+    std::optional<pool_busy_scope> busy_;
     bool lent_ = false;
 };
 

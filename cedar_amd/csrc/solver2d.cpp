@@ -312,6 +312,7 @@ int cdr_hip_solver2d_solve(cdr_hip_solver2d *slv, const double *b_dev, double *x
 int cdr_hip_solver2d_vcycle(cdr_hip_solver2d *slv, const double *b_dev, double *x_dev) {
     if (!slv || !b_dev || !x_dev) return CDR_ERR_ARG;
     return guarded([&] {
+        slv->impl->lend_if_captured();
         slv->impl->vcycle<double>(b_dev, x_dev);
         return (int)CDR_OK;
     });

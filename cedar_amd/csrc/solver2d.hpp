@@ -86,6 +86,8 @@ public:
     const level_data<double> &level(int l) const { return L64_[l]; }
     // the caller keeps pointers to the levels' arrays
     void lend() { guard_.lend(); }
+    // work is about to be enqueued on the solver's stream that the caller may be capturing
+    void lend_if_captured() { guard_.lend_if_captured(stream_); }
     double setup_seconds() const { return setup_s_; }
     double solve_seconds() const { return solve_s_; }
     kernel_manager &kernels() { return km_; }

@@ -391,6 +391,8 @@ public:
     const level3 &level(int l) const { return L_[l]; }
     // the caller keeps pointers to the levels' arrays
     void lend() { guard_.lend(); }
+    // work is about to be enqueued on the solver's stream that the caller may be capturing
+    void lend_if_captured() { guard_.lend_if_captured(stream_); }
     double setup_seconds() const { return setup_s_; }
     double solve_seconds() const { return solve_s_; }
     bool mixed() const { return set_.precision == CDR_PREC_MIXED; }
@@ -844,6 +846,7 @@ int cdr_hip_solver3d_solve(cdr_hip_solver3d *slv, const double *b_dev, double *x
 int cdr_hip_solver3d_vcycle(cdr_hip_solver3d *slv, const double *b_dev, double *x_dev) {
     if (!slv || !b_dev || !x_dev) return CDR_ERR_ARG;
     return guarded3([&] {
+        slv->impl->lend_if_captured();
         slv->impl->vcycle(b_dev, x_dev);
         return (int)CDR_OK;
     });
@@ -853,6 +856,7 @@ int cdr_hip_solver3d_relax_planes(cdr_hip_solver3d *slv, int lvl, int family, do
                                   const double *b_dev, int updown) {
     if (!slv || !b_dev || !x_dev || (updown != CDR_DOWN && updown != CDR_UP)) return CDR_ERR_ARG;
     return guarded3([&] {
+        slv->impl->lend_if_captured();
         slv->impl->relax_planes(lvl, family, x_dev, b_dev,
                                 updown == CDR_UP ? cedar::hip::Dir::UP : cedar::hip::Dir::DOWN);
         return (int)CDR_OK;

@@ -25,7 +25,7 @@ inline std::mutex mu;
 inline std::map<void *, std::size_t> blocks;
 inline std::size_t used = 0, room = ~std::size_t(0);
 inline int streams = 0;
-inline bool busy = false;  // waiting fails, as while the caller captures
+inline bool busy = false, capturing = false;  // busy: waiting fails
 inline thread_local int device = 0;
 }
 inline hipError_t hipGetDevice(int *d) { *d = fake::device; return hipSuccess; }
@@ -56,7 +56,7 @@ inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, int) {
 inline hipError_t hipStreamDestroy(hipStream_t s) { delete s; --fake::streams; return hipSuccess; }
 inline hipError_t hipStreamGetDevice(hipStream_t s, int *d) { *d = s->device; return hipSuccess; }
 inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *st) {
-    *st = hipStreamCaptureStatusNone;
+    *st = fake::capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
 """
@@ -112,6 +112,25 @@ int main() {
         pool_free(p);
         CHECK(fake::used == (lent ? 0 : K));
     }
+    CHECK(pool_trim() == K);
+    // captured: nothing is kept, nor by a guard that is destroyed inside
+    for (bool captured : {true, false}) {
+        void *outer = get(K), *inner = get(2 * K);
+        pool_guard guard;
+        fake::capturing = captured;
+        guard.lend_if_captured(nullptr);
+        fake::capturing = false;
+        guard.enter(nullptr);
+        {
+            pool_guard g2;
+            g2.enter(nullptr);
+            pool_free(inner);
+        }
+        pool_free(outer);
+        CHECK(fake::used == (captured ? 0 : 3 * K));
+    }
+    CHECK(pool_trim() == 3 * K);
+    give(get(K));
     CHECK(pool_trim() == K);
     // the ones kept longest go beyond the limit; one larger than it is never kept
     std::vector<void *> v;

@@ -252,3 +252,39 @@ def test_a_solver_whose_level_pointers_were_given_out_leaves_nothing():
         s.close()
         left = C.memory_trim()
         assert left == 0 if give else left > 5 * 202 * 202 * 8
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("captured", [True, False])
+def test_a_solver_recorded_into_a_graph_leaves_nothing(dim, captured):
+    """A graph of the caller's may still run on another stream when its solver is destroyed: the
+    solver's blocks, and those of its plane solvers, then go back to the device."""
+    import cedar_amd as C
+    side = torch.cuda.Stream()
+    if dim == 2:
+        so, b = _problem(200, 2)
+        build = lambda: C.Solver(so, **KW)
+    else:
+        so, b, _ = G.poisson3_sine(33)
+        so, b = torch.as_tensor(so).cuda(), torch.as_tensor(b).cuda()
+        build = lambda: C.Solver3(so, relaxation="plane-xyz", maxiter=3)
+    with torch.cuda.stream(side):
+        s = build()
+        want = torch.zeros_like(b)
+        s.vcycle(want, b)
+    torch.cuda.synchronize()
+    x = torch.zeros_like(b)
+    g = torch.cuda.CUDAGraph()
+    if captured:
+        with torch.cuda.graph(g, stream=side):
+            s.vcycle(x, b)
+        g.replay()  # on the current stream
+    else:
+        with torch.cuda.stream(side):
+            s.vcycle(x, b)
+    C.memory_trim()
+    s.close()
+    left = C.memory_trim()
+    torch.cuda.synchronize()
+    assert torch.equal(x, want)
+    assert left == 0 if captured else left > 0
